@@ -57,7 +57,12 @@ constexpr int block_keys(int nw) { return nw == 16 ? 128 : (resident(nw) ? kResi
 constexpr int QPW = 32;  // query rows per wavefront
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
-constexpr float kRescaleSlack = 8.0f;  // log2 units a step may exceed the running max by
+// log2 units a checked step may exceed the running max by: of the folded kernels, whose scan
+// checks one block in kAnchorBlocks (the less the max may lag, the more room a key in the blocks
+// between has below the f16 range), and of the VALU kernels, which check every step
+constexpr float kFoldSlack = 4.0f, kRescaleSlack = 8.0f;
+// Blocks from one checked block of a folded scan to the next (see the block loop).
+constexpr int kAnchorBlocks = 8;
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
@@ -716,7 +721,7 @@ icl_attention_kernel(const Args a) {
         bool moves = false;
         if (check) {
             if constexpr (FOLD) bm = max16f(x);
-            moves = first || __any(bm > kRescaleSlack);
+            moves = first || __any(bm > (FOLD ? kFoldSlack : kRescaleSlack));
         }
         if (moves) {
             {
@@ -786,13 +791,22 @@ icl_attention_kernel(const Args a) {
     //   * two buffers (wide heads): block i+1 is staged before the second-to-last step of
     //     block i, fenced by a barrier on each side, so the K operands of its first step can
     //     be read during the last step of block i.
-    // The folded kernels scan optimistically: every block after the first skips the per-step
-    // rescale test and keeps the running max the first block anchored. Probabilities then stay
-    // finite in f16 while no logit exceeds that max by 16 (log2 units); one that does turns into
-    // inf, and the denominator the PV MFMA sums in its last row becomes inf or NaN (no rescale
-    // runs in such a scan, so nothing multiplies it back). Each wavefront tests its denominators
-    // after the scan; if any is not finite, the workgroup scans its context range again with the
-    // test on every step (pass 1, the lazy-rescale scan). The two scans do the same arithmetic
+    // The folded kernels scan optimistically: of every kAnchorBlocks blocks the first runs the
+    // per-step rescale test, which moves the running max up where a key exceeds it by kFoldSlack,
+    // and the others skip it. Probabilities stay finite in f16 while no logit of theirs exceeds
+    // the max by 16 (log2 units); one that does turns into inf, and the denominator the PV MFMA
+    // sums in its last row becomes inf or NaN (a later rescale leaves it so: inf times a factor
+    // above 0 is inf, times 0 is NaN). Each wavefront tests its denominators after every
+    // kAnchorBlocks blocks; if any is not finite, the workgroup drops the scan there and scans its
+    // context range again with the test on every step (pass 1, the lazy-rescale scan). New maxima
+    // come ever more rarely as a scan goes on, so a scan that fails mostly does so early.
+    // Anchored on the first block alone, and tested only at the end, a cache with a few wide
+    // channels (2 % of them eight times the rest: logits of 6 log2 units' spread) sent most
+    // workgroups through both scans: 6.46 -> 3.53 ms at d 44, 33 x 8 x 1024 queries x 65536 keys,
+    // 1.50 -> 0.92 ms at 16384 keys. Unit-normal caches, which never rescan, pay for the added
+    // tests: 3.52 -> 3.59 ms. (16 blocks apart, the same cache rescans again: 4.2 ms; a slack of
+    // 8: 4.3 ms; a test in one step of every block: 3.59-3.63 ms.) The two scans do the same
+    // arithmetic
     // otherwise. (The VALU-mode kernels scan once with the test on: at DP 64 the second pass's
     // live state spills inside their loop and costs more than the test.)
     if constexpr (resident(NW)) {
@@ -891,7 +905,10 @@ icl_attention_kernel(const Args a) {
     f32x16 s_cur = logits(kfr);
     read_k(KsL + k_lane + 32 * G::KPITCH, kfr);  // the K operands of step 1
 
-    for (int blk = 0; blk < nblk; ++blk) {
+    bool restart = false;
+    for (int c0 = 0; c0 < nblk;) {
+    const int c1 = checked_scan ? nblk : min(nblk, c0 + kAnchorBlocks);
+    for (int blk = c0; blk < c1; ++blk) {
         const int64_t kb = k_begin + (int64_t)blk * KB;
         const int cur = blk % G::NBUF, nxt = (blk + 1) % G::NBUF;
         // this lane's operand addresses in the current and next buffers; every step of the
@@ -912,7 +929,7 @@ icl_attention_kernel(const Args a) {
                     __syncthreads();
                 }
             }
-            step(checked_scan || blk == 0, s_cur, kfr, st + 1 < G::SPB ? Kc + 32 * (st + 1) * G::KPITCH : Kn,
+            step(checked_scan || blk == c0, s_cur, kfr, st + 1 < G::SPB ? Kc + 32 * (st + 1) * G::KPITCH : Kn,
                  kf + ((FOLD || KVT != NORI_I8) ? 0 : 32 * st), Vc + st * G::VSTEP, blk * KB + 32 * st,
                  blk == 0 && st == 0);
             // K operands of the step after next: this block's rows, or the next block's (a
@@ -928,14 +945,17 @@ icl_attention_kernel(const Args a) {
         }
         if constexpr (AHEAD == 2) __syncthreads();
     }
-    if (checked_scan) break;
-    {
+    if (!checked_scan) {
         // the denominators sit in O^T row DP-1: tile VT-1, element 3 of lanes 48-63
         const bool bad = lane >= 48 && !(__builtin_isfinite(o[G::VT - 1][0][3]) && __builtin_isfinite(o[G::VT - 1][1][3]));
         if (__any(bad) && lane == 0) rescan = 1;
+        __syncthreads();  // every flag written; every read of the ring done before pass 1 restages it
+        restart = __builtin_amdgcn_readfirstlane(rescan);
+        if (restart) break;
     }
-    __syncthreads();  // every flag written; every read of the ring done before pass 1 restages it
-    if (!rescan) break;
+    c0 = c1;
+    }
+    if (!restart) break;
     }
     }  // ring scan
 

@@ -278,6 +278,33 @@ def test_late_key_above_the_anchored_max(cuda, d, lift):
     assert ((lse.double().cpu() - exp_lse).abs().numpy() <= lse_bound(q, values, 1)).all()
 
 
+@pytest.mark.parametrize("d,nq", [(44, 512), (44, 300), (56, 512), (100, 200)])
+@pytest.mark.parametrize("late", [(511,), (512, 1023), (1024, 1025), (2099,), (140, 700, 1500, 2050)])
+def test_late_keys_around_the_checked_blocks(cuda, d, nq, late):
+    # A folded scan checks its running max in one block of eight (1024 keys with 128-key blocks,
+    # 512 with 64-key ones) and drops the scan for a checked one where a denominator overflowed.
+    # Keys at the first and last rows of checked and unchecked blocks, of the ragged last block,
+    # and several of them rising by 20 log2 units each, so one run overflows more than once; at
+    # 16-wave, 5-wave and two-buffer (d = 100) launches.
+    bg, h, nk = 2, 2, 2100
+    scale = 1.0 / math.sqrt(d)
+    g = torch.Generator().manual_seed(67)
+    q0 = torch.randn(bg, 1, h, d, generator=g)
+    q = q0 + 0.02 * torch.randn(bg, nq, h, d, generator=g)
+    kv = 0.1 * torch.randn(bg, nk, 2, h, d, generator=g)
+    for i, row in enumerate(late):
+        lift = 20.0 * (i + 1)
+        kv[:, row, 0] = q0[:, 0] * (lift * math.log(2.0) / scale) / (q0[:, 0] ** 2).sum(-1, keepdim=True)
+    codes, scales = nori_amd.quantize_int8(kv.to(torch.float16).to(cuda))
+    q = q.to(torch.float16).to(cuda)
+    lse = torch.empty(bg, h, nq, device=cuda)
+    got = nori_amd.icl_attention(q, codes, scales, lse=lse)
+    values = codes.double() * scales.double()
+    exp, exp_lse = reference(q, values)
+    check(got, exp)
+    assert ((lse.double().cpu() - exp_lse).abs().numpy() <= lse_bound(q, values, 1)).all()
+
+
 def test_merge_of_two_halves_equals_one_call(cuda):
     bg, h, nq, nk, d = 2, 4, 50, 300, 56
     kv = make_cache(bg, nk, 1, d, cuda, seed=31)
