@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "nori_hip.h"
+#include "nori_ops.h"
 
 namespace nori {
 

@@ -165,6 +165,33 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
     }
 }
 
+// The base scale: one output per thread. Every workgroup forms the 64 hidden units anew (one erf a
+// lane) rather than pass them through memory. As torch ops this vector of a few hundred values
+// took eleven launches a layer (fill, two GEMMs with their bias copies, GELU, tanh, add, multiply,
+// weight casts), 37 us of device time and three times that on the host; as one kernel about 3 us.
+__global__ void __launch_bounds__(64)
+qass_base_kernel(float log_n, const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, int n_out,
+                 uint16_t* out) {
+    __shared__ float hid[kHid];
+    const int tid = threadIdx.x;
+    const float l = r16(log_n);
+    hid[tid] = gelu16(r16(f16_to_f32(w1[tid]) * l + f16_to_f32(b1[tid])));
+    __syncthreads();
+    const int o = blockIdx.x * 64 + tid;
+    if (o >= n_out) return;
+    const u32x4_t* wr = reinterpret_cast<const u32x4_t*>(w2 + (int64_t)o * kHid);
+    u32x4_t w[kHid / 8];
+#pragma unroll
+    for (int c = 0; c < kHid / 8; ++c) w[c] = wr[c];
+    float acc = 0.0f;
+#pragma unroll
+    for (int c = 0; c < kHid / 8; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = fmaf(f16_to_f32((uint16_t)(w[c][i >> 1] >> (16 * (i & 1)))), hid[8 * c + i], acc);
+    const float delta = r16(acc + f16_to_f32(b2[o]));
+    out[o] = f32_to_f16(l * r16(1.0f + r16(tanhf(delta))));
+}
+
 template <int KS1, int NT2>
 void launch(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, const uint16_t* w1, const uint16_t* b1,
             const uint16_t* w2, const uint16_t* b2, const uint16_t* bs, uint16_t* out, int64_t os, hipStream_t stream) {
@@ -210,4 +237,18 @@ extern "C" int nori_qass_gate(const void* q, int dtype, int64_t rows, int32_t he
         default: launch<4, 2>(qh, rows, heads, d, q_row_stride, w1h, b1h, w2h, b2h, bsh, oh, out_row_stride, stream); break;
     }
     return launch_status("qass_gate");
+}
+
+extern "C" int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2,
+                              int32_t hidden, int32_t n_out, void* out, void* stream_v) {
+    clear_error();
+    if (hidden != kHid) return fail(NORI_ERR_UNSUPPORTED, "qass_base: hidden width %d (64 only)", hidden);
+    if (n_out <= 0) return fail(NORI_ERR_INVALID, "qass_base: %d outputs", n_out);
+    if (!w1 || !b1 || !w2 || !b2 || !out) return fail(NORI_ERR_INVALID, "qass_base: null pointer");
+    if ((uintptr_t)w2 % 16) return fail(NORI_ERR_INVALID, "qass_base: w2 must be 16-byte aligned");
+    hipLaunchKernelGGL(qass_base_kernel, dim3((unsigned)((n_out + 63) / 64)), dim3(64), 0, (hipStream_t)stream_v, log_n,
+                       reinterpret_cast<const uint16_t*>(w1), reinterpret_cast<const uint16_t*>(b1),
+                       reinterpret_cast<const uint16_t*>(w2), reinterpret_cast<const uint16_t*>(b2), n_out,
+                       reinterpret_cast<uint16_t*>(out));
+    return launch_status("qass_base");
 }

@@ -114,6 +114,11 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "nori_quant_f16_scale_probe": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp]),
 }
 
+# The package's own entry points beyond the C ABI (csrc/nori_ops.h).
+OPS: dict[str, tuple[object, list]] = {
+    "nori_qass_base": (ctypes.c_int, [_f32, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp]),
+}
+
 _lib: ctypes.CDLL | None = None
 
 
@@ -135,7 +140,7 @@ def lib() -> ctypes.CDLL:
         found = handle.nori_abi_version()
         if found != ABI_VERSION:
             raise RuntimeError(f"{LIBRARY} has ABI version {found}, this package binds version {ABI_VERSION}; rebuild it")
-        for name, (restype, argtypes) in SIGNATURES.items():
+        for name, (restype, argtypes) in (SIGNATURES | OPS).items():
             fn = getattr(handle, name)
             fn.restype = restype
             fn.argtypes = argtypes

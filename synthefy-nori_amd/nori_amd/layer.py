@@ -39,8 +39,8 @@ from .attention import attend_dense, compute_attention_blockwise, icl_attention,
 from . import kv_project
 from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
-from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, operand_dtype, projection_operand, qass_gate,
-                   residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp)
+from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, operand_dtype, projection_operand,
+                   qass_base, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp)
 
 ACTIVATION_FN = {"gelu": nn.GELU(), "relu": nn.ReLU(), "silu": nn.SiLU()}
 _SDPA_BACKENDS_WITHOUT_CUDNN = [SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION, SDPBackend.MATH]
@@ -89,6 +89,12 @@ class QASSMaxScaling(nn.Module):
     def forward(self, q: torch.Tensor, key_len: int) -> torch.Tensor:
         if key_len <= 1:
             return q
+        if self.qass_mode == "full" and self._fused_base_applies(q):
+            base_scale = qass_base(math.log(float(max(key_len, 2))), *self._half_weights("_base16", self.base_mlp))
+            base_scale = base_scale.view(1, 1, self.num_heads, self.head_dim)
+            if self._fused_gate_applies(q, base_scale):
+                return qass_gate(q, *self._gate_weights(), base_scale)
+            return q * base_scale * (1.0 + torch.tanh(self.gate_mlp(q)))
         # log n in double, cast once: an fp16 key count overflows at 65520 rows (a fill on the
         # device, not a host copy, so the pass can be captured into a graph)
         log_n = torch.full((), math.log(float(max(key_len, 2))), device=q.device, dtype=q.dtype)
@@ -107,6 +113,23 @@ class QASSMaxScaling(nn.Module):
     # separate torch ops
     fused = True
 
+    def _fused_base_applies(self, q: torch.Tensor) -> bool:
+        """The base scale as one HIP launch: where its linears compute in fp16 and no gradient is
+        asked for, the 64-wide hidden layer."""
+        first, last = self.base_mlp[0], self.base_mlp[-1]
+        if not (self.fused and q.is_cuda and q.dtype == torch.float16 and first.weight.is_cuda):
+            return False
+        if first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None:
+            return False
+        return self._computes_in_fp16(q, first)
+
+    @staticmethod
+    def _computes_in_fp16(q: torch.Tensor, first: nn.Linear) -> bool:
+        autocast16 = torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.float16
+        if not (autocast16 or first.weight.dtype == torch.float16):
+            return False
+        return not (torch.is_grad_enabled() and (q.requires_grad or first.weight.requires_grad))
+
     def _fused_gate_applies(self, q: torch.Tensor, base_scale: torch.Tensor) -> bool:
         """The gate MLP as one HIP pass: inference on fp16 queries whose gate linears compute in
         fp16 (autocast, or fp16 weights), the 64-wide hidden layer, heads up to 64 wide."""
@@ -116,22 +139,23 @@ class QASSMaxScaling(nn.Module):
         if first.out_features != QASS_GATE_HIDDEN or self.head_dim > 64 or self.head_dim % 4 or first.bias is None \
                 or last.bias is None:
             return False
-        autocast16 = torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.float16
-        if not (autocast16 or first.weight.dtype == torch.float16):
-            return False
-        return not (torch.is_grad_enabled() and (q.requires_grad or first.weight.requires_grad))
+        return self._computes_in_fp16(q, first)
 
-    def _gate_weights(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-        """(w1, b1, w2, b2) of the gate MLP in fp16 (the casts autocast makes), cached until a
-        parameter changes."""
-        first, last = self.gate_mlp[0], self.gate_mlp[-1]
+    def _half_weights(self, slot: str, mlp: nn.Sequential) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+        """(w1, b1, w2, b2) of a two-layer MLP in fp16 (the casts autocast makes), kept in ``slot``
+        until a parameter changes."""
+        first, last = mlp[0], mlp[-1]
         params = (first.weight, first.bias, last.weight, last.bias)
         key = tuple((p.data_ptr(), p._version, p.device) for p in params)
-        cached = getattr(self, "_gate16", None)
+        cached = getattr(self, slot, None)
         if cached is None or cached[0] != key:
             with torch.no_grad():
-                cached = self._gate16 = (key, tuple(p.detach().to(torch.float16).contiguous() for p in params))
+                cached = (key, tuple(p.detach().to(torch.float16).contiguous() for p in params))
+            setattr(self, slot, cached)
         return cached[1]
+
+    def _gate_weights(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+        return self._half_weights("_gate16", self.gate_mlp)
 
 
 class SwiGLUMLP(nn.Module):

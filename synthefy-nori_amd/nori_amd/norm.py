@@ -433,6 +433,22 @@ def qass_gate(q: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Ten
             q3.data_ptr(), nat.dtype_code(q.dtype), q3.shape[0], h, d, q3.stride(0), w1.data_ptr(), b1.data_ptr(),
             w2.data_ptr(), b2.data_ptr(), QASS_GATE_HIDDEN, bs.data_ptr(), out.data_ptr(), h * d, nat.stream_of(device),
         ),
+def qass_base(log_n: float, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Tensor, b2: torch.Tensor) -> torch.Tensor:
+    """The QASS base scale ``T(log n) * (1 + tanh(base_mlp(T(log n))))`` as fp16 [n_out] in one launch
+    (``nori_qass_base``), T the rounding to fp16, rounded where the separate fp16 ops round: w1
+    [64, 1], b1 [64], w2 [n_out, 64], b2 [n_out], fp16 and contiguous."""
+    device = nat.require_device(w1, b1, w2, b2)
+    out = torch.empty(w2.shape[0], dtype=torch.float16, device=device)
+    nat.check(
+        nat.lib().nori_qass_base(
+            float(log_n), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), w2.shape[1], w2.shape[0],
+            out.data_ptr(), nat.stream_of(device),
+        ),
+        "qass_base",
+    )
+    return out
+
+
         "qass_gate",
     )
     return out.view(q.shape)

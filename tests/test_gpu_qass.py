@@ -118,3 +118,22 @@ def test_single_key_and_fp32_queries_keep_the_torch_path(monkeypatch):
         assert torch.equal(m(q.half(), 1), q.half())  # one key: q unscaled
         out = m(q, 100)  # fp32 queries without autocast: the separate ops
     assert out.dtype == torch.float32
+
+
+@pytest.mark.parametrize("heads,d", [(10, 56), (1, 64), (8, 44), (2, 8), (1, 4), (3, 128)])
+@pytest.mark.parametrize("n_keys", [2, 300, 65536, 200000])
+def test_base_scale_against_the_separate_ops(heads, d, n_keys):
+    # nori_qass_base against the module's torch ops under fp16 autocast: the hidden layer rounds at
+    # the same points, and its 64-term sum, in another order, can move the rounded delta by one fp16
+    # ulp, which moves 1 + tanh by at most two (2^-10 in [1, 2)) and its product with T(log n) by a
+    # last rounding: 3 * 2^-10 * T(log n) in all. Head counts fill a last workgroup only in part
+    # (4, 352, 384 outputs).
+    m = _module(heads, d, seed=heads + 7 * d).to(DEV)
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        log_n = torch.full((), math.log(float(n_keys)), device=DEV, dtype=torch.float16)
+        want = log_n * (1.0 + torch.tanh(m.base_mlp(log_n.view(1, 1))))
+        got = layer_mod.qass_base(math.log(float(n_keys)), *m._half_weights("_base16", m.base_mlp))
+        assert got.dtype == torch.float16 and got.shape == (heads * d,)
+        assert float((got.double() - want.view(-1).double()).abs().max()) <= 3 * 2.0**-10 * float(log_n)
+        m.base_mlp[-1].bias.add_(1.0)  # in place: the fp16 copies follow
+        assert not torch.equal(layer_mod.qass_base(math.log(float(n_keys)), *m._half_weights("_base16", m.base_mlp)), got)
