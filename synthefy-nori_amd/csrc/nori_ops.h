@@ -17,6 +17,13 @@ extern "C" {
 int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int32_t hidden,
                    int32_t n_out, void* out, void* stream);
 
+// nori_rms_norm_to (no weight) of fp32 rows at three strides, written as contiguous fp16 or bf16
+// rows: row r = (i0 * d1 + i1) * d2 + i2 of x starts at element i0 * s0 + i1 * s1 + i2 * s2. Bit for
+// bit nori_rms_norm_to of the gathered rows. Rows of more than 1024 elements, cols not a multiple
+// of 4, 2^31 rows or more and unaligned operands return NORI_ERR_UNSUPPORTED.
+int nori_rms_norm_rows(const float* x, int64_t rows, int32_t cols, int64_t d1, int64_t d2, int64_t s0, int64_t s1,
+                       int64_t s2, float eps, void* y, int y_dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

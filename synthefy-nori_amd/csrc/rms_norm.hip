@@ -125,6 +125,48 @@ rms_norm_chunked_kernel(const uint8_t* x, int64_t rows, int cols, int64_t x_row_
     }
 }
 
+// rms_norm_chunked_kernel of fp32 rows at three strides, written contiguously (rows, d1 * d2 and d2
+// below 2^31: 32-bit divisions). A layer's context rows [table, row, group] are normalized
+// straight into the [table, group, row] order its sequence projections flatten; written in the
+// stream's order, every projection of several tables first copied its operand.
+template <int OT, int G>
+__global__ void __launch_bounds__(kThreads)
+rms_norm_rows_kernel(const float* x, uint32_t rows, int cols, uint32_t d1, uint32_t d2, int64_t s0, int64_t s1,
+                     int64_t s2, float eps, uint8_t* y) {
+    constexpr int EPC = 4;
+    const int lane_in_row = threadIdx.x % G;
+    const uint32_t row = blockIdx.x * (kThreads / G) + threadIdx.x / G;
+    const int nchunks = cols / EPC;
+    const bool active = row < rows;
+    const uint32_t t = row / d2;
+    const float* xr = x + (int64_t)(t / d1) * s0 + (int64_t)(t % d1) * s1 + (int64_t)(row - t * d2) * s2;
+    float v[kMaxChunksPerLane][EPC];
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kMaxChunksPerLane; ++k) {
+        const int ch = lane_in_row + k * G;
+        if (active && ch < nchunks) {
+            const uint4 c = *reinterpret_cast<const uint4*>(xr + ch * EPC);
+            unpack_chunk<NORI_F32>(c, v[k]);
+#pragma unroll
+            for (int e = 0; e < EPC; ++e) acc = fmaf(v[k][e], v[k][e], acc);
+        }
+    }
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, G);
+    const float inv = rsqrtf(acc / (float)cols + eps);
+#pragma unroll
+    for (int k = 0; k < kMaxChunksPerLane; ++k) {
+        const int ch = lane_in_row + k * G;
+        if (active && ch < nchunks) {
+            float o[EPC];
+#pragma unroll
+            for (int e = 0; e < EPC; ++e) o[e] = v[k][e] * inv;
+            store_chunk<NORI_F32, OT, EPC>(y + ((int64_t)row * cols + ch * EPC) * 2, o);
+        }
+    }
+}
+
 // One wavefront per row, element-wise loads: any width and alignment. Each element is read
 // and then written by the same lane, so y may be x.
 template <int DT, int WDT, int OT>
@@ -370,4 +412,49 @@ extern "C" int nori_residual_add_rms_norm(const float* x, const void* u, int u_d
     if (y_dtype == NORI_F16) return launch_residual<NORI_F32, NORI_F16>(x, u, ur, alpha, rows, cols, eps, x_out, y, y_group, gb, rb, stream);
     if (y_dtype == NORI_BF16) return launch_residual<NORI_F32, NORI_BF16>(x, u, ur, alpha, rows, cols, eps, x_out, y, y_group, gb, rb, stream);
     return launch_residual<NORI_F32, NORI_F32>(x, u, ur, alpha, rows, cols, eps, x_out, y, y_group, gb, rb, stream);
+}
+
+namespace {
+
+template <int OT>
+int launch_rows(const float* x, uint32_t rows, int cols, uint32_t d1, uint32_t d2, int64_t s0, int64_t s1, int64_t s2,
+                float eps, void* y, hipStream_t stream) {
+    const int nchunks = cols / 4;
+    int g = 1;
+    while (g < nchunks && g < 64) g <<= 1;
+    const int rows_per_block = kThreads / g;
+    const unsigned grid = (rows + rows_per_block - 1) / rows_per_block;
+#define NORI_ROWS_CASE(GV)                                                                                          \
+    case GV:                                                                                                         \
+        hipLaunchKernelGGL((rms_norm_rows_kernel<OT, GV>), dim3(grid), dim3(kThreads), 0, stream, x, rows, cols, d1, \
+                           d2, s0, s1, s2, eps, (uint8_t*)y);                                                        \
+        break;
+    switch (g) {
+        NORI_ROWS_CASE(1) NORI_ROWS_CASE(2) NORI_ROWS_CASE(4) NORI_ROWS_CASE(8)
+        NORI_ROWS_CASE(16) NORI_ROWS_CASE(32) NORI_ROWS_CASE(64)
+    }
+#undef NORI_ROWS_CASE
+    return launch_status("rms_norm_rows");
+}
+
+}  // namespace
+
+extern "C" int nori_rms_norm_rows(const float* x, int64_t rows, int32_t cols, int64_t d1, int64_t d2, int64_t s0,
+                                  int64_t s1, int64_t s2, float eps, void* y, int y_dtype, void* stream_v) {
+    clear_error();
+    if (rows < 0 || cols <= 0 || d1 <= 0 || d2 <= 0)
+        return fail(NORI_ERR_INVALID, "rms_norm_rows: bad shape rows=%lld cols=%d (%lld x %lld)", (long long)rows, cols,
+                    (long long)d1, (long long)d2);
+    if (y_dtype != NORI_F16 && y_dtype != NORI_BF16)
+        return fail(NORI_ERR_UNSUPPORTED, "rms_norm_rows: unsupported output dtype %s", dtype_name(y_dtype));
+    constexpr int64_t kMax = 0x7fffffffLL;
+    if (rows > kMax || d1 > kMax || d2 > kMax || cols % 4 || cols / 4 > 64 * kMaxChunksPerLane || (uintptr_t)x % 16 ||
+        (uintptr_t)y % 8 || s0 % 4 || s1 % 4 || s2 % 4)
+        return fail(NORI_ERR_UNSUPPORTED, "rms_norm_rows: %lld rows of %d elements at these strides", (long long)rows, cols);
+    if (rows == 0) return NORI_OK;
+    if (!x || !y) return fail(NORI_ERR_INVALID, "rms_norm_rows: null pointer");
+    hipStream_t stream = (hipStream_t)stream_v;
+    if (y_dtype == NORI_F16)
+        return launch_rows<NORI_F16>(x, (uint32_t)rows, cols, (uint32_t)d1, (uint32_t)d2, s0, s1, s2, eps, y, stream);
+    return launch_rows<NORI_BF16>(x, (uint32_t)rows, cols, (uint32_t)d1, (uint32_t)d2, s0, s1, s2, eps, y, stream);
 }

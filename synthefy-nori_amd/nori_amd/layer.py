@@ -39,7 +39,7 @@ from .attention import attend_dense, compute_attention_blockwise, icl_attention,
 from . import kv_project
 from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
-from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, operand_dtype, projection_operand,
+from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, group_major_operand, operand_dtype, projection_operand,
                    qass_base, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp)
 
 ACTIVATION_FN = {"gelu": nn.GELU(), "relu": nn.ReLU(), "silu": nn.SiLU()}
@@ -433,11 +433,12 @@ class MultiheadAttention(nn.Module):
         mult = float(torch.tensor(math.log(float(max(n_keys, 2))), dtype=dtype)) if n_keys > 1 else 1.0
         return mult / math.sqrt(float(self.head_dim))
 
-    def _linear_weights(self, device: torch.device):
-        """(q weight [H*D, E], k|v weight [2*H*D, E], output weight [E, H*D]) as F.linear takes
-        them, in the dtype the projections compute in (the autocast dtype under GPU autocast),
-        cached until a weight changes. Autocast does not keep casts of these reshaped views, so
-        without the cache every call would cast them again; the values are the same casts."""
+    def _cast_weights(self, device: torch.device):
+        """(key, q weight [H*D, E], k|v weight [2*H*D, E], output weight [E, H*D], q|k|v weight
+        [3*H*D, E]) as F.linear takes them, in the dtype the projections compute in (the autocast
+        dtype under GPU autocast), cached until a weight changes. Autocast does not keep casts of
+        these reshaped views, so without the cache every call would cast them again; the values
+        are the same casts."""
         dtype = self.qkv_proj_weight.dtype
         if device.type == "cuda" and torch.is_autocast_enabled("cuda"):
             dtype = torch.get_autocast_dtype("cuda")
@@ -449,8 +450,17 @@ class MultiheadAttention(nn.Module):
             with torch.no_grad():
                 w = self.qkv_proj_weight.to(device=device, dtype=dtype)
                 out_w = self.out_proj_weight.reshape(hd, self.embed_dim).t().to(device=device, dtype=dtype).contiguous()
-                cached = self._cast = (key, w[0].reshape(hd, self.embed_dim), w[1:].reshape(2 * hd, self.embed_dim), out_w)
-        return cached[1:]
+                cached = self._cast = (key, w[0].reshape(hd, self.embed_dim), w[1:].reshape(2 * hd, self.embed_dim), out_w,
+                                       w.reshape(3 * hd, self.embed_dim))
+        return cached
+
+    def _linear_weights(self, device: torch.device):
+        """(q weight, k|v weight, output weight) of ``_cast_weights``."""
+        return self._cast_weights(device)[1:4]
+
+    def _projects_with_cast_weights(self, x: torch.Tensor) -> bool:
+        """Whether a projection of x may take the cached casts (which carry no gradient)."""
+        return x.is_cuda and not torch.is_grad_enabled()
 
     def _apply_extra_attn_scale(self, q: torch.Tensor, n_keys: int) -> torch.Tensor:
         """q * temperature * log(n)/log(n_ref) (reference layer.py:555-583)."""
@@ -522,6 +532,10 @@ class MultiheadAttention(nn.Module):
         kv_proj_weight = self.qkv_proj_weight[1:]
         if copy_first_head_kv:
             kv = torch.einsum("... s, j h d s -> ... j h d", x_kv_flat, kv_proj_weight[:, :1])
+        elif self._projects_with_cast_weights(x_kv_flat):
+            # the same library GEMM on the same casts of the weight, not cast again on each call
+            kv = torch.nn.functional.linear(x_kv_flat, self._cast_weights(x_kv_flat.device)[2])
+            kv = kv.view(*x_kv_flat.shape[:-1], 2, self.num_heads, self.head_dim)
         else:
             kv = torch.nn.functional.linear(
                 x_kv_flat, kv_proj_weight.reshape(2 * self.num_heads * self.head_dim, self.embed_dim)
@@ -593,7 +607,11 @@ class MultiheadAttention(nn.Module):
         BS = B * S
         if self.qkv_combined:
             x = x.reshape(-1, *x.shape[-2:])
-            qkv = torch.einsum("... s, j h d s -> ... j h d", x, self.qkv_proj_weight)
+            if self._projects_with_cast_weights(x):
+                qkv = proj_linear(x, self._cast_weights(x.device)[4])
+                qkv = qkv.view(*x.shape[:-1], 3, self.num_heads, self.head_dim)
+            else:
+                qkv = torch.einsum("... s, j h d s -> ... j h d", x, self.qkv_proj_weight)
             if self.qk_norm:
                 qkv = torch.stack((self.q_norm(qkv[:, :, 0]), self.k_norm(qkv[:, :, 1]), qkv[:, :, 2]), dim=2)
             if self.use_qassmax:
@@ -620,7 +638,7 @@ class MultiheadAttention(nn.Module):
         B, S, F, _ = x.shape
         BS = B * S
         n_kv = int(x_kv.shape[-2])
-        use_linear = self._is_linear_projection_used(x.device)
+        use_linear = self._is_linear_projection_used(x.device) or self._projects_with_cast_weights(x)
         # the projections read x and x_kv as they lie: a strided view such as the column
         # attention's [table, group, row] transpose of the cells goes through the projection
         # kernel without the copy its flattening would make (the result is contiguous)
@@ -1166,7 +1184,8 @@ class EncoderBaseLayer(nn.Module):
             return x, x
         if not pre_steps:
             # src feeds only projections: under autocast the norm writes their fp16 operand directly
-            return x, projection_operand(seq_norm, x)
+            # (in the [batch, groups, rows] order the sequence attention's projections flatten)
+            return x, group_major_operand(seq_norm, x)
         first = self._step_output(pre_steps[0], projection_operand(self.layer_norms[pre_steps[0]], x), feature_atten_mask,
                                   eval_pos)
         return self._add_then_steps(x, first, pre_steps[1:], feature_atten_mask, eval_pos, then_norm=seq_norm)

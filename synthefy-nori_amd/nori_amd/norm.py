@@ -153,6 +153,28 @@ def projection_operand(norm: "RMSNorm", x: torch.Tensor) -> torch.Tensor:
     return norm(x)
 
 
+def group_major_operand(norm: "RMSNorm", x: torch.Tensor) -> torch.Tensor:
+    """``projection_operand(norm, x)`` of a stream x [batch, rows, groups, width] for projections
+    of its [batch, groups, rows] transpose: the same values, laid out so that
+    ``.transpose(1, 2)`` is contiguous where one kernel can write them so (fp32 streams of several
+    groups, a norm without weight, fp16 or bf16 autocast)."""
+    dt = operand_dtype(x)
+    if (isinstance(norm, RMSNorm) and norm.weight is None and x.dim() == 4 and x.is_cuda and x.dtype == torch.float32
+            and dt != torch.float32 and x.stride(-1) == 1 and tuple(norm.normalized_shape) == (int(x.shape[-1]),)
+            and x.shape[2] > 1 and x.numel()):
+        b, r, g, width = x.shape
+        y = torch.empty((b, g, r, width), dtype=dt, device=x.device)
+        rc = nat.lib().nori_rms_norm_rows(
+            x.data_ptr(), b * g * r, width, g, r, x.stride(0), x.stride(2), x.stride(1), float(norm.eps), y.data_ptr(),
+            nat.dtype_code(dt), nat.stream_of(x.device),
+        )
+        if rc == nat.NORI_OK:
+            return y.transpose(1, 2)
+        if rc != nat.NORI_ERR_UNSUPPORTED:
+            nat.check(rc, "rms_norm_rows")
+    return projection_operand(norm, x)
+
+
 class RMSNorm(nn.Module):
     """RMSNorm with the reference constructor and state dict (layer.py:233-258), computed by HIP."""
 
@@ -411,6 +433,22 @@ def swiglu_mlp_residual_norm(x: torch.Tensor, gate_up: torch.Tensor, down: torch
 QASS_GATE_HIDDEN = 64
 
 
+def qass_base(log_n: float, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Tensor, b2: torch.Tensor) -> torch.Tensor:
+    """The QASS base scale ``T(log n) * (1 + tanh(base_mlp(T(log n))))`` as fp16 [n_out] in one launch
+    (``nori_qass_base``), T the rounding to fp16, rounded where the separate fp16 ops round: w1
+    [64, 1], b1 [64], w2 [n_out, 64], b2 [n_out], fp16 and contiguous."""
+    device = nat.require_device(w1, b1, w2, b2)
+    out = torch.empty(w2.shape[0], dtype=torch.float16, device=device)
+    nat.check(
+        nat.lib().nori_qass_base(
+            float(log_n), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), w2.shape[1], w2.shape[0],
+            out.data_ptr(), nat.stream_of(device),
+        ),
+        "qass_base",
+    )
+    return out
+
+
 def qass_gate(q: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Tensor, b2: torch.Tensor,
               base_scale: torch.Tensor) -> torch.Tensor:
     """QASS "full" scaling ``q * base_scale * (1 + tanh(gate_mlp(q)))`` in one HIP pass
@@ -433,22 +471,6 @@ def qass_gate(q: torch.Tensor, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Ten
             q3.data_ptr(), nat.dtype_code(q.dtype), q3.shape[0], h, d, q3.stride(0), w1.data_ptr(), b1.data_ptr(),
             w2.data_ptr(), b2.data_ptr(), QASS_GATE_HIDDEN, bs.data_ptr(), out.data_ptr(), h * d, nat.stream_of(device),
         ),
-def qass_base(log_n: float, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Tensor, b2: torch.Tensor) -> torch.Tensor:
-    """The QASS base scale ``T(log n) * (1 + tanh(base_mlp(T(log n))))`` as fp16 [n_out] in one launch
-    (``nori_qass_base``), T the rounding to fp16, rounded where the separate fp16 ops round: w1
-    [64, 1], b1 [64], w2 [n_out, 64], b2 [n_out], fp16 and contiguous."""
-    device = nat.require_device(w1, b1, w2, b2)
-    out = torch.empty(w2.shape[0], dtype=torch.float16, device=device)
-    nat.check(
-        nat.lib().nori_qass_base(
-            float(log_n), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), w2.shape[1], w2.shape[0],
-            out.data_ptr(), nat.stream_of(device),
-        ),
-        "qass_base",
-    )
-    return out
-
-
         "qass_gate",
     )
     return out.view(q.shape)

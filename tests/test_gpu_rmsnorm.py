@@ -157,3 +157,24 @@ def test_residual_add_norm_equals_the_two_calls(cuda, udtype, out_dtype, cols):
     ref = rms_norm(residual_add(xw, uw, alpha), 2 * cols + 1024, None, 1e-5)
     xg = xw.clone()
     assert torch.equal(residual_add_norm(xg, uw, alpha, wide), ref)
+
+
+@pytest.mark.parametrize("shape", [(1, 300, 9, 128), (3, 41, 5, 352), (2, 7, 33, 560), (1, 1, 2, 4), (2, 3, 2, 1024), (2, 5, 3, 1028), (2, 6, 1, 128)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("view", ["whole", "rows", "groups"])
+def test_group_major_operand_is_the_operand_transposed(cuda, shape, dt, view):
+    # nori_rms_norm_rows (one to 256 chunks a row; 1028 columns and single groups take the other
+    # path): bit for bit projection_operand, in memory order [batch, groups, rows], from contiguous
+    # streams and from slices of a larger one
+    from nori_amd.norm import RMSNorm, group_major_operand, projection_operand
+
+    b, r, g, e = shape
+    x = torch.randn(b, r + 2, g + 1, e, generator=torch.Generator().manual_seed(r * e)).to(cuda)
+    x = {"whole": x[:, :r, :g].contiguous(), "rows": x.contiguous()[:, 1 : r + 1], "groups": x[:, :, :g]}[view]
+    norm = RMSNorm(e, eps=1e-5)
+    with torch.inference_mode(), torch.autocast("cuda", dtype=dt):
+        want = projection_operand(norm, x.contiguous())
+        got = group_major_operand(norm, x)
+    assert got.dtype == dt and torch.equal(got, want)
+    if x.shape[2] > 1 and e <= 1024:
+        assert got.transpose(1, 2).is_contiguous()
