@@ -228,6 +228,181 @@ __global__ void __launch_bounds__(kThreads) icl_attention_short_kernel(const Arg
     if (a.lse && sub == 0) a.lse[row] = lse_out;
 }
 
+// The same attention for fp16 queries over an fp16 cache (heads of up to 64, a multiple of 8 wide),
+// several queries to a group: 8 lanes hold 8 head elements each and QB queries of one (b, h), so
+// that each K/V row is loaded, and its norm formed, once for QB queries instead of once for each.
+// Normed q and k are fp16 values either way (the separate passes round them so) and stay packed:
+// a logit is four v_dot2_f32_f16 and three DPP adds a lane, fp32 throughout; the probabilities and
+// the output sums are fp32 as in the kernel above. What bounded that one is its issue: per query
+// and key it unpacked and normed the key row again.
+template <int QB>
+__global__ void __launch_bounds__(kThreads) icl_attention_rows_kernel(const Args a, uint32_t groups, uint32_t nqb,
+                                                                      const Prologue pro) {
+    constexpr int G = 8, KC = 4;
+    uint32_t gi = blockIdx.x * (kThreads / G) + threadIdx.x / G;  // (b, h, query block), the block fastest
+    const bool valid = gi < groups;
+    if (!valid) gi = groups - 1;  // keep every lane of the group active through the reductions
+    const int sub = (int)(threadIdx.x % G);
+    const uint32_t bh = gi / nqb, q0 = (gi - bh * nqb) * QB;
+    const int b32 = (int)(bh / (uint32_t)a.heads), h = (int)(bh - (uint32_t)b32 * a.heads);
+    const int64_t b = b32;
+    const int c0 = 8 * sub, d = a.d, nq = (int)a.nq, nk = (int)a.nk;
+    const bool live = c0 < d;  // d % 8 == 0: a lane's 8 elements are all in or all out
+    const int cl = live ? c0 : 0;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+
+    const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + b * a.q_bg + (int64_t)h * a.q_head + cl;
+    u32x4 qw[QB];  // this lane's packed elements of the block's queries (past nq: the last query again)
+#pragma unroll
+    for (int i = 0; i < QB; ++i) {
+        qw[i] = *reinterpret_cast<const u32x4*>(qp + (int64_t)min((int)q0 + i, nq - 1) * a.q_row);
+        if (!live) qw[i] = zero;
+    }
+    // T(T(v * rsqrt(mean(v^2) + eps)) * w) over the group's row, T rounding to fp16
+    auto norm8 = [&](u32x4 v, const float (&w)[8]) {
+        float x[8], ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            x[e] = f16_to_f32((uint16_t)(v[e >> 1] >> (16 * (e & 1))));
+            ss += x[e] * x[e];
+        }
+        const float inv = rsqrtf(group_sum<G>(ss) / (float)d + pro.eps);
+        u32x4 r;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t lo = f32_to_f16(round_to<NORI_F16>(x[2 * k] * inv) * w[2 * k]);
+            r[k] = lo | ((uint32_t)f32_to_f16(round_to<NORI_F16>(x[2 * k + 1] * inv) * w[2 * k + 1]) << 16);
+        }
+        return r;
+    };
+    auto gains = [&](const void* p, float (&w)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = live ? load_as_f32(p, pro.wdt, cl + e) : 0.f;
+    };
+    if (pro.qw) {
+        float w[8];
+        gains(pro.qw, w);
+#pragma unroll
+        for (int i = 0; i < QB; ++i) qw[i] = norm8(qw[i], w);
+    }
+    if (pro.qmult != 1.f) {
+#pragma unroll
+        for (int i = 0; i < QB; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                qw[i][k] = (uint32_t)f32_to_f16(f16_to_f32((uint16_t)qw[i][k]) * pro.qmult) |
+                           ((uint32_t)f32_to_f16(f16_to_f32((uint16_t)(qw[i][k] >> 16)) * pro.qmult) << 16);
+    }
+    const bool knorm = pro.kw != nullptr;
+    float kw[8];
+    if (knorm) gains(pro.kw, kw);
+
+    const uint16_t* kp = reinterpret_cast<const uint16_t*>(a.kv) + b * a.kv_bg + (int64_t)(h / a.hgroup) * d + cl;
+    float m[QB], l[QB], o[QB][8];
+#pragma unroll
+    for (int i = 0; i < QB; ++i) {
+        m[i] = -INFINITY;
+        l[i] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[i][e] = 0.f;
+    }
+    // keys in chunks of KC, every K/V row of a chunk loaded before the first is used (past nk: the
+    // last row again, left out of the sums); the chunk length is uniform over the launch
+    for (int j0 = 0; j0 < nk; j0 += KC) {
+        u32x4 rk[KC], rv[KC];
+#pragma unroll
+        for (int u = 0; u < KC; ++u) {
+            const uint16_t* kr = kp + (int64_t)min(j0 + u, nk - 1) * a.kv_row;
+            rk[u] = *reinterpret_cast<const u32x4*>(kr);
+            rv[u] = *reinterpret_cast<const u32x4*>(kr + a.kv_half);
+        }
+        float s[QB][KC], m_new[QB];
+#pragma unroll
+        for (int i = 0; i < QB; ++i) m_new[i] = m[i];
+#pragma unroll
+        for (int u = 0; u < KC; ++u) {
+#pragma unroll
+            for (int i = 0; i < QB; ++i) s[i][u] = -INFINITY;
+            if (j0 + u < nk) {
+                if (!live) rk[u] = zero;
+                if (knorm) rk[u] = norm8(rk[u], kw);
+#pragma unroll
+                for (int i = 0; i < QB; ++i) {
+                    float dot = 0.f;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t x = qw[i][k], y = rk[u][k];  // (a bit cast of a vector's element takes element 0)
+                        dot = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, x), __builtin_bit_cast(f16x2, y), dot, false);
+                    }
+                    s[i][u] = group_sum<G>(dot) * a.scale_log2;
+                    m_new[i] = fmaxf(m_new[i], s[i][u]);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < QB; ++i) {
+            const float alpha = __builtin_amdgcn_exp2f(m[i] - m_new[i]);
+            m[i] = m_new[i];
+            l[i] *= alpha;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[i][e] *= alpha;
+        }
+#pragma unroll
+        for (int u = 0; u < KC; ++u) {
+            if (j0 + u < nk) {
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = f16_to_f32((uint16_t)(rv[u][e >> 1] >> (16 * (e & 1))));
+#pragma unroll
+                for (int i = 0; i < QB; ++i) {
+                    const float p = __builtin_amdgcn_exp2f(s[i][u] - m[i]);
+                    l[i] += p;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[i][e] = fmaf(p, v[e], o[i][e]);
+                }
+            }
+        }
+    }
+    if (!valid) return;
+    const bool bf = a.out_dtype == NORI_BF16;
+#pragma unroll
+    for (int i = 0; i < QB; ++i) {
+        const int qi = (int)q0 + i;
+        if (qi >= nq) break;
+        const float inv = 1.0f / l[i];
+        if (live) {
+            uint16_t* op = reinterpret_cast<uint16_t*>(a.out) + b * a.o_bg + (int64_t)qi * a.o_row + (int64_t)h * a.o_head + c0;
+            uint32_t w[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float v0 = o[i][2 * k] * inv, v1 = o[i][2 * k + 1] * inv;
+                w[k] = (uint32_t)(bf ? f32_to_bf16(v0) : f32_to_f16(v0)) | ((uint32_t)(bf ? f32_to_bf16(v1) : f32_to_f16(v1)) << 16);
+            }
+            *reinterpret_cast<u32x2*>(op) = u32x2{w[0], w[1]};  // (8-byte aligned)
+            *reinterpret_cast<u32x2*>(op + 4) = u32x2{w[2], w[3]};
+        }
+        if (a.lse && sub == 0) a.lse[(int64_t)bh * nq + qi] = (m[i] + __log2f(l[i])) * kLn2;
+    }
+}
+
+// Whether the kernel above takes a call: 16-byte loads of q, K and V, 8-byte stores.
+bool takes_rows(const Args& a, int64_t groups) {
+    return a.q_dtype == NORI_F16 && (a.flags & kQVec8) && (a.flags & kOutVec4) && a.d % 8 == 0 && a.d <= 64 &&
+           (uintptr_t)a.kv % 16 == 0 && a.kv_bg % 8 == 0 && a.kv_row % 8 == 0 && a.kv_half % 8 == 0 && groups < 0x7fffffffLL;
+}
+
+int launch_rows(const Args& a, uint32_t groups, uint32_t nqb, int qb, const Prologue& pro, hipStream_t stream) {
+    const dim3 grid((groups + kThreads / 8 - 1) / (kThreads / 8)), block(kThreads);
+    switch (qb) {
+        case 1: hipLaunchKernelGGL((icl_attention_rows_kernel<1>), grid, block, 0, stream, a, groups, nqb, pro); break;
+        case 2: hipLaunchKernelGGL((icl_attention_rows_kernel<2>), grid, block, 0, stream, a, groups, nqb, pro); break;
+        case 3: hipLaunchKernelGGL((icl_attention_rows_kernel<3>), grid, block, 0, stream, a, groups, nqb, pro); break;
+        case 4: hipLaunchKernelGGL((icl_attention_rows_kernel<4>), grid, block, 0, stream, a, groups, nqb, pro); break;
+        default: hipLaunchKernelGGL((icl_attention_rows_kernel<5>), grid, block, 0, stream, a, groups, nqb, pro); break;
+    }
+    return NORI_OK;
+}
+
 template <int KVT, int KC>
 int launch_chunked(const Args& a, const Prologue& pro, hipStream_t stream) {
     const int quads = (a.d + 3) / 4;
@@ -262,7 +437,12 @@ namespace attn {
 int launch_short(int kv_dtype, const Args& a, const Prologue& pro, hipStream_t stream) {
     switch (kv_dtype) {
         case NORI_I8: return launch_group<NORI_I8>(a, pro, stream);
-        case NORI_F16: return launch_group<NORI_F16>(a, pro, stream);
+        case NORI_F16: {
+            // blocks of up to 5 queries, as even as they come
+            const int64_t nqb = (a.nq + 4) / 5, qb = (a.nq + nqb - 1) / nqb, groups = a.bg * a.heads * nqb;
+            if (takes_rows(a, groups)) return launch_rows(a, (uint32_t)groups, (uint32_t)nqb, (int)qb, pro, stream);
+            return launch_group<NORI_F16>(a, pro, stream);
+        }
         case NORI_BF16: return launch_group<NORI_BF16>(a, pro, stream);
         default: return launch_group<NORI_F32>(a, pro, stream);
     }

@@ -686,3 +686,44 @@ def test_few_token_shape_with_a_query_view_off_the_4_element_grid(cuda, offset):
     assert ((lse.double().cpu() - exp_lse).abs().numpy() <= lse_bound(q, kv.double(), heads // kv_heads)).all()
     # the same values in an aligned view give the same answer to the bar
     check(nori_amd.icl_attention(q.contiguous(), kv), exp)
+
+
+@pytest.mark.parametrize("d,h,hk", [(8, 1, 1), (24, 2, 1), (64, 4, 2), (64, 3, 3)])
+@pytest.mark.parametrize("nq,nk", [(1, 1), (1, 16), (2, 5), (3, 4), (4, 6), (5, 9), (6, 8), (11, 18), (7, 128)])
+@pytest.mark.parametrize("prologue", [False, True])
+def test_grouped_queries_against_the_row_kernel(cuda, d, h, hk, nq, nk, prologue):
+    # The short-context kernel of fp16 calls with 16-byte rows holds up to five queries a group;
+    # rows on 8-byte boundaries take the one of a query a group. Both against float64 over the same
+    # fp16 values: the sums are fp32, so an output is its fp16 rounding (2^-11 of itself) and
+    # about 2^-20 of the largest value for each of a few roundings of logit and sum away; with the
+    # prologue a normed value one fp16 ulp off (its mean of squares summed in another order) moves a
+    # logit of sum |q k| <= |q| |k| by 2^-11 of a term, so 4 ulps of the largest value.
+    bg = 5
+    if not prologue and nq >= 8 and nk <= 64:
+        pytest.skip("without a prologue these run on the few-token MFMA kernel")
+    g = torch.Generator().manual_seed(100 * nq + nk + d)
+    wide_q = torch.randn(bg, nq, h, d + 8, generator=g).half().to(cuda)
+    kv = torch.randn(bg, nk, 2, hk, d, generator=g).half().to(cuda)
+    pro = None
+    q = wide_q[..., :d]
+    x, k = q.double().cpu(), kv[:, :, 0].double().cpu()
+    if prologue:
+        gq, gk = (torch.rand(d, generator=g) + 0.5 for _ in range(2))
+        pro = {"q_weight": gq.to(cuda), "k_weight": gk.to(cuda), "eps": 1e-6, "q_mult": 1.5}
+
+        def norm(t, w):
+            t = (t.float() * torch.rsqrt(t.float().square().mean(-1, keepdim=True) + 1e-6)).half()
+            return (t.float() * w).half()
+
+        x, k = (norm(x, gq).float() * 1.5).half().double(), norm(k, gk).double()
+    k, v = (t.repeat_interleave(h // hk, 2) for t in (k, kv[:, :, 1].double().cpu()))
+    p = (torch.einsum("bqhd,bkhd->bhqk", x, k) / math.sqrt(d)).softmax(-1)
+    exp = torch.einsum("bhqk,bkhd->bqhd", p, v)
+    tol = 2.0**-11 * exp.abs() + (4 * 2.0**-11 if prologue else 8 * 2.0**-20) * v.abs().max()
+    shifted = torch.empty(bg, nq, h, d + 8, dtype=torch.float16, device=cuda)
+    shifted[..., 4 : d + 4] = q
+    for queries in (q, shifted[..., 4 : d + 4]):
+        lse = torch.empty(bg, h, nq, device=cuda)
+        got = nori_amd.icl_attention(queries, kv, lse=lse, qk_prologue=pro)
+        assert bool(((got.double().cpu() - exp).abs() <= tol).all())
+        assert torch.isfinite(lse).all()
