@@ -8,10 +8,9 @@
 // Shapes. These GEMMs are HBM-bound (K = 128 or 256: every output element costs 2 bytes of
 // write against 2K FLOP), so the kernel is built for bandwidth: each x row is read from HBM
 // once and each output row written once.
-//   * A workgroup of 8 wavefronts owns a block of 256 rows and a chunk of NC output columns
-//     (128 for K = 128, 64 for K = 256); the chunk's weight rows are staged in LDS as f16
-//     (zero rows past n).
-//   * Each wavefront holds its 32 rows of x as v_mfma_f32_16x16x32_f16 B operands (lane
+//   * A workgroup of 8 wavefronts keeps a chunk of 128 output columns of W in LDS as f16 (zero
+//     rows past n) and walks blocks of 256 rows (128 while 256 leave CUs idle).
+//   * Each wavefront holds its 32 (16) rows of x as v_mfma_f32_16x16x32_f16 B operands (lane
 //     n + 16*(k/8) holds row n, elements 8*(k/8)..+8 of every 32-wide step) and computes the
 //     transposed product W x^T tile by tile: each lane ends with four consecutive output
 //     columns of one row. 64 columns at a time are staged in the wavefront's LDS slice and
@@ -22,9 +21,16 @@
 //     x_outer, x_mid, x_row and y_outer, y_mid, y_row), so strided views (a token subset of
 //     each row, a slice of a stacked output, the [table, group, row] transpose of a
 //     [table, row, group] cell buffer) are read and written in place.
-//   * Workgroups are numbered so that the column chunks of one row block are consecutive on
-//     one XCD (the hardware deals workgroup i to XCD i % 8): the x block is read from HBM once
-//     and served to the other chunks by that XCD's L2.
+//   * Each XCD takes a contiguous range of the row blocks (the hardware deals workgroup i to XCD
+//     i % 8), and its workgroups come in teams of one per column chunk over the same row blocks:
+//     an x block is read from HBM once and served to the other chunks by that XCD's L2.
+//   * Measured against workgroups of one row block each, which staged W again for every 256 rows
+//     and waited out each x load: 655,360 rows 128 -> 640 286 -> 262 us (1.0 GB, 3.8 TB/s).
+//   * The head-norm variant also RMS-norms heads of 64 as their rows leave LDS: 8 lanes hold a head
+//     row there, so the mean of squares is three DPP adds. As passes of their own the q/k norms of
+//     one cell layer (128 x 512 x 10 cells of 128) read and wrote 280 us' worth of projections, and
+//     an attention kernel that normed its rows as it loaded them (2,048 columns x 2 heads, 320 x 256)
+//     ran 352 us against 282 us on normed operands.
 //
 // nori_linear_f16_residual_rms_norm fuses the output projection of an attention sublayer with
 // the deep-norm residual update of an fp32 stream and the next sublayer's RMSNorm (no weight)
@@ -54,127 +60,16 @@ using namespace nori;
 
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
-constexpr int kNR = 2;                    // 16-row tiles per wavefront
-constexpr int kRows = kWaves * kNR * 16;  // rows per workgroup
 
 struct LinArgs {
     const _Float16* x; int64_t rows, n_mid, n_inner, x_outer, x_mid, x_row;
     const _Float16* w; int64_t w_row;
     int n;
     _Float16* y; int64_t y_outer, y_mid, y_row;
-    int nchunks;
-    int64_t grid;
-};
-
-// element offsets of row r in x and y on the three-level row grid
-__device__ __forceinline__ void row_offsets(const LinArgs& a, int64_t r, int64_t& xo, int64_t& yo) {
-    const int64_t oj = r / a.n_inner, i = r - oj * a.n_inner;
-    const int64_t o = oj / a.n_mid, j = oj - o * a.n_mid;
-    xo = o * a.x_outer + j * a.x_mid + i * a.x_row;
-    yo = o * a.y_outer + j * a.y_mid + i * a.y_row;
-}
-
-__device__ __forceinline__ uint32_t pack_f16_rn(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi});
-}
-
-template <int KS, int NC>
-__global__ void __launch_bounds__(kThreads) linear_f16_kernel(const LinArgs a) {
-    constexpr int PITCH = 32 * KS + 8;  // f16 per staged W row: +16 bytes spreads the 16-row reads over the banks
-    constexpr int GC = 64;              // output columns staged per wavefront between stores
-    constexpr int SP = GC + 8;          // f16 per staged output row
-    __shared__ __attribute__((aligned(16))) _Float16 wt[NC * PITCH];
-    __shared__ __attribute__((aligned(16))) _Float16 ot[kWaves * kNR * 16 * SP];
-
-    const int64_t wg = blockIdx.x;
-    const int64_t xcd = wg % 8, local = wg / 8, per = a.grid / 8, extra = a.grid % 8;
-    const int64_t t = xcd * per + (xcd < extra ? xcd : extra) + local;
-    const int chunk = (int)(t % a.nchunks);
-    const int64_t rb = t / a.nchunks;
-    const int c0 = chunk * NC;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4;
-
-    f16x8 xf[kNR][KS];
-#pragma unroll
-    for (int nt = 0; nt < kNR; ++nt) {
-        const int64_t row = rb * kRows + wave * (kNR * 16) + nt * 16 + (lane & 15);
-        int64_t xo, yo;
-        row_offsets(a, row < a.rows ? row : a.rows - 1, xo, yo);
-        const _Float16* xrow = a.x + xo + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) xf[nt][ks] = *reinterpret_cast<const f16x8*>(xrow + 32 * ks);
-    }
-    // rows this lane stores from the staged tile: 8 rows per pass, 8 lanes per row
-    int64_t soff[4];
-    bool svalid[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const int64_t row = rb * kRows + wave * (kNR * 16) + 8 * p + (lane >> 3);
-        svalid[p] = row < a.rows;
-        int64_t xo;
-        row_offsets(a, svalid[p] ? row : a.rows - 1, xo, soff[p]);
-    }
-
-    for (int e = tid; e < NC * KS * 4; e += kThreads) {
-        const int r = e / (KS * 4), q = e % (KS * 4);
-        uint4 v = {0u, 0u, 0u, 0u};
-        if (c0 + r < a.n) v = *reinterpret_cast<const uint4*>(a.w + (int64_t)(c0 + r) * a.w_row + 8 * q);
-        *reinterpret_cast<uint4*>(wt + r * PITCH + 8 * q) = v;
-    }
-    __syncthreads();
-
-    const _Float16* wa = wt + (lane & 15) * PITCH + 8 * g;
-    _Float16* my = ot + wave * (kNR * 16) * SP;
-    const int ncols = min(NC, a.n - c0);
-    for (int gc = 0; gc < ncols; gc += GC) {
-#pragma unroll
-        for (int mm = 0; mm < GC / 16; ++mm) {
-            const int m = gc / 16 + mm;
-            f32x4 acc[kNR];
-#pragma unroll
-            for (int nt = 0; nt < kNR; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const f16x8 av = *reinterpret_cast<const f16x8*>(wa + 16 * m * PITCH + 32 * ks);
-#pragma unroll
-                for (int nt = 0; nt < kNR; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, xf[nt][ks], acc[nt], 0, 0, 0);
-            }
-#pragma unroll
-            for (int nt = 0; nt < kNR; ++nt)
-                *reinterpret_cast<uint2*>(my + (nt * 16 + (lane & 15)) * SP + 16 * mm + 4 * g) =
-                    uint2{pack_f16_rn(acc[nt][0], acc[nt][1]), pack_f16_rn(acc[nt][2], acc[nt][3])};
-        }
-        // the wavefront's 32 rows x 64 columns, row by row: 16 bytes per lane, 128 per row
-        const int col = c0 + gc + 8 * (lane & 7);
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            const uint4 v = *reinterpret_cast<const uint4*>(my + (8 * p + (lane >> 3)) * SP + 8 * (lane & 7));
-            if (svalid[p]) {
-                if (col + 8 <= a.n) *reinterpret_cast<uint4*>(a.y + soff[p] + col) = v;
-                else if (col + 4 <= a.n) *reinterpret_cast<uint2*>(a.y + soff[p] + col) = uint2{v.x, v.y};
-            }
-        }
-    }
-}
-
-template <int KS, int NC>
-int launch(LinArgs a, hipStream_t stream) {
-    a.nchunks = (a.n + NC - 1) / NC;
-    a.grid = (a.rows + kRows - 1) / kRows * a.nchunks;
-    if (a.grid > 0x7fffffffLL) return fail(NORI_ERR_UNSUPPORTED, "linear_f16: %lld rows exceed one launch", (long long)a.rows);
-    hipLaunchKernelGGL((linear_f16_kernel<KS, NC>), dim3((unsigned)a.grid), dim3(kThreads), 0, stream, a);
-    return launch_status("linear_f16");
-}
-
-// ---------------------------------------------------------------- projection + residual + norm
-
-struct ResArgs {
-    const _Float16* a; int64_t rows, n_mid, n_inner, a_outer, a_mid, a_row;
-    const _Float16* w; int64_t w_row;
-    float* x; int64_t x_outer, x_mid, x_row;
-    _Float16* y; int64_t y_outer, y_mid, y_row;
-    float alpha, eps;
-    int64_t nblocks;
+    int nchunks, teams;  // column chunks; workgroups per XCD and chunk
+    int64_t nblocks;     // row blocks
+    // head norm (NORM kernels): columns below norm_cols are heads of 64 with gains [64]
+    const void* gain; int gain_dtype; float eps; int norm_cols;
 };
 
 struct RowIndex { int64_t o, j, i; };
@@ -191,6 +86,184 @@ __device__ __forceinline__ RowIndex split_row(int64_t r, int64_t n_mid, int64_t 
     const int64_t o = oj / n_mid, j = oj - o * n_mid;
     return {o, j, i};
 }
+
+__device__ __forceinline__ uint32_t pack_f16_rn(float lo, float hi) {
+    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi});
+}
+
+// sum over the 8 lanes of a store row (DPP: lane ^ 1, lane ^ 2, the other quad of 8)
+__device__ __forceinline__ float sum8(float v) {
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4e, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, false));
+    return v;
+}
+
+// 8 fp16 values of a 64-wide head row whose other values the neighbouring 7 lanes hold:
+// T(T(v * rsqrt(mean(v^2) + eps)) * w), T rounding to fp16 (the per-head RMSNorm pass)
+__device__ __forceinline__ uint4 head_norm8(uint4 v, const float (&w)[8], float eps) {
+    const uint32_t h[4] = {v.x, v.y, v.z, v.w};
+    float x[8], ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        x[e] = f16_to_f32((uint16_t)(h[e >> 1] >> (16 * (e & 1))));
+        ss = fmaf(x[e], x[e], ss);
+    }
+    const float inv = rsqrtf(sum8(ss) / 64.0f + eps);
+    uint32_t r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t lo = f32_to_f16(round_to<NORI_F16>(x[2 * k] * inv) * w[2 * k]);
+        r[k] = lo | ((uint32_t)f32_to_f16(round_to<NORI_F16>(x[2 * k + 1] * inv) * w[2 * k + 1]) << 16);
+    }
+    return uint4{r[0], r[1], r[2], r[3]};
+}
+
+// NR 16-row tiles per wavefront. A workgroup keeps its column chunk of W in LDS and walks row
+// blocks, loading the next block's x rows before it computes the current one's; the workgroups
+// of a chunk's row blocks and those of the other chunks over the same rows share an XCD.
+template <int KS, int NC, int NR, bool NORM>
+__global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(const LinArgs a) {
+    constexpr int PITCH = 32 * KS + 8;  // f16 per staged W row: +16 bytes spreads the 16-row reads over the banks
+    constexpr int GC = 64;              // output columns staged per wavefront between stores
+    constexpr int SP = GC + 8;          // f16 per staged output row
+    constexpr int WROWS = NR * 16, BROWS = kWaves * WROWS;
+    extern __shared__ __attribute__((aligned(16))) _Float16 lds[];
+    _Float16* wt = lds;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4;
+
+    const int xcd = blockIdx.x % 8, local = blockIdx.x / 8;
+    const int chunk = local % a.nchunks, team = local / a.nchunks;
+    const int64_t per = a.nblocks / 8, extra = a.nblocks % 8;
+    const int64_t first = xcd * per + (xcd < extra ? xcd : extra), last = first + per + (xcd < extra ? 1 : 0);
+    int64_t blk = first + team;
+    if (blk >= last) return;  // uniform over the workgroup, before its barrier
+    const int c0 = chunk * NC;
+    const bool narrow = a.rows <= 0x7fffffffLL;
+
+    auto load_x = [&](int64_t rb, f16x8 (&xf)[NR][KS]) {
+#pragma unroll
+        for (int nt = 0; nt < NR; ++nt) {
+            const int64_t row = rb * BROWS + wave * WROWS + nt * 16 + (lane & 15);
+            const RowIndex ri = split_row(row < a.rows ? row : a.rows - 1, a.n_mid, a.n_inner, narrow);
+            const _Float16* xrow = a.x + ri.o * a.x_outer + ri.j * a.x_mid + ri.i * a.x_row + 8 * g;
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) xf[nt][ks] = *reinterpret_cast<const f16x8*>(xrow + 32 * ks);
+        }
+    };
+    f16x8 xf[NR][KS];
+    load_x(blk, xf);
+
+    for (int e = tid; e < NC * KS * 4; e += kThreads) {
+        const int r = e / (KS * 4), q = e % (KS * 4);
+        uint4 v = {0u, 0u, 0u, 0u};
+        if (c0 + r < a.n) v = *reinterpret_cast<const uint4*>(a.w + (int64_t)(c0 + r) * a.w_row + 8 * q);
+        *reinterpret_cast<uint4*>(wt + r * PITCH + 8 * q) = v;
+    }
+    float gain[8];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int c = 8 * (lane & 7) + e;
+            gain[e] = a.gain_dtype == NORI_F32   ? load_elem<NORI_F32>(a.gain, c)
+                      : a.gain_dtype == NORI_F16 ? load_elem<NORI_F16>(a.gain, c)
+                                                 : load_elem<NORI_BF16>(a.gain, c);
+        }
+    }
+    __syncthreads();
+
+    const _Float16* wa = wt + (lane & 15) * PITCH + 8 * g;
+    _Float16* my = lds + NC * PITCH + wave * WROWS * SP;
+    const int ncols = min(NC, a.n - c0);
+    for (; blk < last; blk += a.teams) {
+        // the next block's rows (the last block loads its own again, unused)
+        f16x8 xn[NR][KS];
+        load_x(blk + a.teams < last ? blk + a.teams : blk, xn);
+        // lane r < WROWS has row r's place in y; the store passes (8 rows each, 8 lanes a row)
+        // take it from there
+        const int64_t row0 = blk * BROWS + wave * WROWS;
+        const int64_t yrow = row0 + (lane & (WROWS - 1));
+        const RowIndex ri = split_row(yrow < a.rows ? yrow : a.rows - 1, a.n_mid, a.n_inner, narrow);
+        const int64_t yo = ri.o * a.y_outer + ri.j * a.y_mid + ri.i * a.y_row;
+        for (int gc = 0; gc < ncols; gc += GC) {
+#pragma unroll
+            for (int mm = 0; mm < GC / 16; ++mm) {
+                const int m = gc / 16 + mm;
+                f32x4 acc[NR];
+#pragma unroll
+                for (int nt = 0; nt < NR; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const f16x8 av = *reinterpret_cast<const f16x8*>(wa + 16 * m * PITCH + 32 * ks);
+#pragma unroll
+                    for (int nt = 0; nt < NR; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, xf[nt][ks], acc[nt], 0, 0, 0);
+                }
+#pragma unroll
+                for (int nt = 0; nt < NR; ++nt)
+                    *reinterpret_cast<uint2*>(my + (nt * 16 + (lane & 15)) * SP + 16 * mm + 4 * g) =
+                        uint2{pack_f16_rn(acc[nt][0], acc[nt][1]), pack_f16_rn(acc[nt][2], acc[nt][3])};
+            }
+            // the wavefront's rows x 64 columns, row by row: 16 bytes per lane, 128 per row
+            const int col = c0 + gc + 8 * (lane & 7);
+#pragma unroll
+            for (int p = 0; p < 2 * NR; ++p) {
+                const int rr = 8 * p + (lane >> 3);
+                uint4 v = *reinterpret_cast<const uint4*>(my + rr * SP + 8 * (lane & 7));
+                if constexpr (NORM) {
+                    if (c0 + gc < a.norm_cols) v = head_norm8(v, gain, a.eps);
+                }
+                const int64_t at = __shfl(yo, rr) + col;
+                if (row0 + rr < a.rows) {
+                    if (col + 8 <= a.n) *reinterpret_cast<uint4*>(a.y + at) = v;
+                    else if (col + 4 <= a.n) *reinterpret_cast<uint2*>(a.y + at) = uint2{v.x, v.y};
+                }
+            }
+        }
+#pragma unroll
+        for (int nt = 0; nt < NR; ++nt)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) xf[nt][ks] = xn[nt][ks];
+    }
+}
+
+template <int KS, int NC, int NR, bool NORM>
+int launch_tiles(LinArgs a, int cus, hipStream_t stream) {
+    constexpr int BROWS = kWaves * NR * 16;
+    constexpr size_t lds = ((size_t)NC * (32 * KS + 8) + (size_t)BROWS * 72) * sizeof(_Float16);
+    static_assert(lds <= 160 * 1024, "a chunk of W and the staged rows fit one workgroup's LDS");
+    if (hipFuncSetAttribute((const void*)linear_f16_kernel<KS, NC, NR, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess)
+        return fail(NORI_ERR_RUNTIME, "linear_f16: cannot reserve %zu bytes of LDS", lds);
+    a.nblocks = (a.rows + BROWS - 1) / BROWS;
+    // resident workgroups (LDS-bound, 16 wavefronts per CU at most), dealt to the XCDs in whole
+    // teams: one workgroup per column chunk over the same row blocks
+    const int64_t slots = (int64_t)cus * std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / lds, 2)) / 8;
+    a.teams = (int)std::max<int64_t>(1, std::min<int64_t>(slots / a.nchunks, (a.nblocks + 7) / 8));
+    const int64_t grid = 8 * (int64_t)a.teams * a.nchunks;
+    if (grid > 0x7fffffffLL) return fail(NORI_ERR_UNSUPPORTED, "linear_f16: %d columns exceed one launch", a.n);
+    hipLaunchKernelGGL((linear_f16_kernel<KS, NC, NR, NORM>), dim3((unsigned)grid), dim3(kThreads), lds, stream, a);
+    return launch_status("linear_f16");
+}
+
+template <int KS, int NC, bool NORM>
+int launch(LinArgs a, hipStream_t stream) {
+    a.nchunks = (a.n + NC - 1) / NC;
+    const int cus = device_cus();
+    // 256-row blocks; 128-row ones while those leave CUs without a workgroup
+    if ((a.rows + 255) / 256 * a.nchunks < cus) return launch_tiles<KS, NC, 1, NORM>(a, cus, stream);
+    return launch_tiles<KS, NC, 2, NORM>(a, cus, stream);
+}
+
+// ---------------------------------------------------------------- projection + residual + norm
+
+struct ResArgs {
+    const _Float16* a; int64_t rows, n_mid, n_inner, a_outer, a_mid, a_row;
+    const _Float16* w; int64_t w_row;
+    float* x; int64_t x_outer, x_mid, x_row;
+    _Float16* y; int64_t y_outer, y_mid, y_row;
+    float alpha, eps;
+    int64_t nblocks;
+};
 
 // K = N = 32 KS; one 16-row tile per wavefront and block; W in dynamic LDS (K rows of K + 8
 // f16), then each wavefront's 16 x 72 f16 slice for u. Per block a wavefront issues its
@@ -343,10 +416,12 @@ int launch_residual(ResArgs a, hipStream_t stream) {
 
 }  // namespace
 
-extern "C" int nori_linear_f16(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
-                               int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, const void* weight,
-                               int64_t w_row_stride, int32_t n, void* y, int64_t y_outer_stride, int64_t y_mid_stride,
-                               int64_t y_row_stride, void* stream) {
+namespace {
+
+int run_linear(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k, int64_t x_outer_stride,
+               int64_t x_mid_stride, int64_t x_row_stride, const void* weight, int64_t w_row_stride, int32_t n, void* y,
+               int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, const void* gain, int gain_dtype,
+               float eps, int32_t norm_cols, void* stream) {
     clear_error();
     if (n_outer < 0 || n_mid < 0 || n_inner < 0 || k <= 0 || n <= 0)
         return fail(NORI_ERR_INVALID, "linear_f16: bad shape n_outer=%lld n_mid=%lld n_inner=%lld k=%d n=%d",
@@ -379,9 +454,42 @@ extern "C" int nori_linear_f16(const void* x, int64_t n_outer, int64_t n_mid, in
     a.y_outer = y_outer_stride;
     a.y_mid = y_mid_stride;
     a.y_row = y_row_stride;
+    a.gain = gain;
+    a.gain_dtype = gain_dtype;
+    a.eps = eps;
+    a.norm_cols = norm_cols;
     hipStream_t s = (hipStream_t)stream;
-    return k == 128 ? launch<4, 128>(a, s) : launch<8, 64>(a, s);
+    if (norm_cols > 0) return k == 128 ? launch<4, 128, true>(a, s) : launch<8, 128, true>(a, s);
+    return k == 128 ? launch<4, 128, false>(a, s) : launch<8, 128, false>(a, s);
 }
+
+}  // namespace
+
+extern "C" int nori_linear_f16(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
+                               int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, const void* weight,
+                               int64_t w_row_stride, int32_t n, void* y, int64_t y_outer_stride, int64_t y_mid_stride,
+                               int64_t y_row_stride, void* stream) {
+    return run_linear(x, n_outer, n_mid, n_inner, k, x_outer_stride, x_mid_stride, x_row_stride, weight, w_row_stride, n,
+                      y, y_outer_stride, y_mid_stride, y_row_stride, nullptr, NORI_F32, 0.f, 0, stream);
+}
+
+extern "C" int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
+                                         int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride,
+                                         const void* weight, int64_t w_row_stride, int32_t n, void* y,
+                                         int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride,
+                                         const void* gain, int gain_dtype, float eps, int32_t norm_cols, void* stream) {
+    if (norm_cols <= 0 || norm_cols > n || norm_cols % 64) {
+        clear_error();
+        return fail(NORI_ERR_INVALID, "linear_f16_head_norm: %d columns of %d are not whole heads of 64", norm_cols, n);
+    }
+    if (!gain || (gain_dtype != NORI_F32 && gain_dtype != NORI_F16 && gain_dtype != NORI_BF16)) {
+        clear_error();
+        return fail(NORI_ERR_INVALID, "linear_f16_head_norm: gains must be float32, float16 or bfloat16");
+    }
+    return run_linear(x, n_outer, n_mid, n_inner, k, x_outer_stride, x_mid_stride, x_row_stride, weight, w_row_stride, n,
+                      y, y_outer_stride, y_mid_stride, y_row_stride, gain, gain_dtype, eps, norm_cols, stream);
+}
+
 
 extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner,
                                                  int32_t k, int64_t a_outer_stride, int64_t a_mid_stride,

@@ -24,6 +24,16 @@ int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, 
 int nori_rms_norm_rows(const float* x, int64_t rows, int32_t cols, int64_t d1, int64_t d2, int64_t s0, int64_t s1,
                        int64_t s2, float eps, void* y, int y_dtype, void* stream);
 
+// nori_linear_f16 followed by the per-head RMSNorm of its first norm_cols columns, taken as heads
+// of 64 (a multiple of 64): each head row v becomes T(T(v * rsqrt(mean(v^2) + eps)) * gain) with T
+// the rounding to fp16 and gain [64] of gain_dtype -- the projection and the q/k norm pass over it
+// (MultiheadAttention with qk_norm, layer.py:497-500, 1122-1134), up to the order of the sums.
+int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
+                              int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, const void* weight,
+                              int64_t w_row_stride, int32_t n, void* y, int64_t y_outer_stride, int64_t y_mid_stride,
+                              int64_t y_row_stride, const void* gain, int gain_dtype, float eps, int32_t norm_cols,
+                              void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -117,6 +117,10 @@ SIGNATURES: dict[str, tuple[object, list]] = {
 # The package's own entry points beyond the C ABI (csrc/nori_ops.h).
 OPS: dict[str, tuple[object, list]] = {
     "nori_qass_base": (ctypes.c_int, [_f32, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp]),
+    "nori_linear_f16_head_norm": (
+        ctypes.c_int,
+        [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _i32, _vp, _i64, _i64, _i64, _vp, _i32, _f32, _i32, _vp],
+    ),
     "nori_rms_norm_rows": (ctypes.c_int, [_vp, _i64, _i32, _i64, _i64, _i64, _i64, _i64, _f32, _vp, _i32, _vp]),
 }
 

@@ -39,6 +39,7 @@ from .attention import attend_dense, compute_attention_blockwise, icl_attention,
 from . import kv_project
 from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
+from .projection import linear_head_norm
 from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, group_major_operand, operand_dtype, projection_operand,
                    qass_base, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp)
 
@@ -642,6 +643,12 @@ class MultiheadAttention(nn.Module):
         # the projections read x and x_kv as they lie: a strided view such as the column
         # attention's [table, group, row] transpose of the cells goes through the projection
         # kernel without the copy its flattening would make (the result is contiguous)
+        if use_linear and not copy_first_head_kv:
+            normed = self._project_normed(x, x_kv)
+            if normed is not None:
+                return self.attend_projected(normed[0].view(BS, F, self.num_heads, self.head_dim),
+                                             normed[1].view(BS, n_kv, 2, self.num_heads, self.head_dim), attn_mask,
+                                             normed=True)
         if use_linear:
             w_q, w_kv, _ = self._linear_weights(x.device)
             q = proj_linear(x, w_q).view(BS, F, self.num_heads, self.head_dim)
@@ -656,19 +663,35 @@ class MultiheadAttention(nn.Module):
             kv = torch.einsum("... s, j h d s -> ... j h d", x_kv.reshape(BS, n_kv, -1), kv_w)
         return self.attend_projected(q, kv, attn_mask)
 
-    def attend_projected(self, q: torch.Tensor, kv: torch.Tensor, attn_mask: torch.Tensor | None = None) -> torch.Tensor:
+    def _project_normed(self, x: torch.Tensor, x_kv: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor] | None:
+        """The q and k|v projections with their q/k norms formed in the same kernels, or None where
+        those do not take them (heads other than 64 wide, other dtypes or widths, gradients)."""
+        if not (self.qk_norm and self.head_dim == 64 and self._projects_with_cast_weights(x)):
+            return None
+        if self.q_norm.weight is None or self.k_norm.weight is None:
+            return None
+        w_q, w_kv, _ = self._linear_weights(x.device)
+        width = self.num_heads * self.head_dim
+        q = linear_head_norm(x, w_q, self.q_norm.weight, self.q_norm.eps, width)
+        if q is None:
+            return None
+        kv = linear_head_norm(x_kv, w_kv, self.k_norm.weight, self.k_norm.eps, width)
+        return None if kv is None else (q, kv)
+
+    def attend_projected(self, q: torch.Tensor, kv: torch.Tensor, attn_mask: torch.Tensor | None = None, *,
+                         normed: bool = False) -> torch.Tensor:
         """The separate-Q/KV attention after its projections (layer.py:1114-1162 less the
         projections): ``q`` [BS, F, H, D] and ``kv`` [BS, N, 2, Hkv, D] (any strides with a
         contiguous head axis, e.g. views into one stacked projection) through the q/k norms,
         QASS and the HIP kernel; returns the attention output [BS, F, H, D] before the output
-        projection."""
-        prologue = self._fused_prologue(q, kv) if attn_mask is None else None
+        projection. ``normed``: the q/k norms are in already."""
+        prologue = self._fused_prologue(q, kv) if attn_mask is None and not normed else None
         if prologue is not None:
             # q/k norms and the log-n multiply fused into the attention kernel's loads
             if self._attention_dropout_p() != 0.0:
                 raise RuntimeError("the HIP attention path is inference-only (dropout must be zero)")
             return icl_attention(q, kv, qk_prologue=prologue)
-        if self.qk_norm:
+        if self.qk_norm and not normed:
             q = self._norm_q(q)
             kv = self._norm_kv(kv if kv.is_contiguous() else kv.contiguous())
         n_keys = int(kv.shape[1])

@@ -20,7 +20,7 @@ import torch
 
 from . import _native as nat
 
-__all__ = ["linear", "linear_residual_norm", "takes_kernel"]
+__all__ = ["linear", "linear_head_norm", "linear_residual_norm", "takes_kernel"]
 
 _WIDTHS = (128,)  # inner widths routed to the kernel (it also takes 256, where the library GEMM was faster)
 _MAX_N = 256      # output widths up to this (past it the library GEMM was as fast or faster)
@@ -82,7 +82,7 @@ def _common_grid(*tensors: torch.Tensor) -> tuple | None:
     return (grid,) + tuple(tuple([0] * pad + st[::-1]) for st in strides)
 
 
-def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = False) -> bool:
+def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = False, min_rows: int = _MIN_ROWS) -> bool:
     """Whether ``linear(x, weight)`` runs on the HIP kernel (``any_width``: whether the kernel
     can take the operands at all, whatever the routing rule says)."""
     if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == torch.float16 and weight.dim() == 2):
@@ -97,7 +97,7 @@ def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = Fal
         return False
     if weight.stride(-1) != 1 or weight.stride(0) % 8 or weight.data_ptr() % 16 or x.data_ptr() % 16:
         return False
-    if x.numel() // k < _MIN_ROWS:
+    if x.numel() // k < min_rows:
         return False
     levels = _row_levels(x)
     return levels is not None and all(st % 8 == 0 for _, st in levels)
@@ -131,6 +131,33 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None = Non
             ctypes.c_void_p(out.data_ptr()), yo, ym, yr, nat.stream_of(x.device),
         ),
         "linear_f16",
+    )
+    return out
+
+
+def linear_head_norm(x: torch.Tensor, weight: torch.Tensor, gain: torch.Tensor, eps: float,
+                     norm_cols: int) -> torch.Tensor | None:
+    """``linear(x, weight)`` with the first ``norm_cols`` columns taken as heads of 64 and each head
+    row RMS-normed with ``gain`` [64], in one kernel (``nori_linear_f16_head_norm``): the
+    projection and the per-head q/k norm of ``MultiheadAttention``, each rounded to fp16. Any row
+    count; None where the kernel does not take the operands."""
+    if gain.shape != (64,) or not gain.is_cuda or gain.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        return None
+    if norm_cols % 64 or not takes_kernel(x, weight, any_width=True, min_rows=1):
+        return None
+    n = int(weight.shape[0])
+    out = torch.empty(tuple(x.shape[:-1]) + (n,), dtype=torch.float16, device=x.device)
+    common = _common_grid(x, out)
+    if common is None:
+        return None
+    (no, nm, ni), sx, sy = common
+    gain = gain.contiguous()
+    nat.check(
+        nat.lib().nori_linear_f16_head_norm(
+            x.data_ptr(), no, nm, ni, int(x.shape[-1]), *sx, weight.data_ptr(), int(weight.stride(0)), n, out.data_ptr(),
+            *sy, gain.data_ptr(), nat.dtype_code(gain.dtype), float(eps), int(norm_cols), nat.stream_of(x.device),
+        ),
+        "linear_f16_head_norm",
     )
     return out
 

@@ -268,3 +268,29 @@ def test_two_phase_steps_take_the_fused_pass(cuda, monkeypatch):
     for got, ref in ((c1, c0), (t1, t0), (r1, r0)):
         scale = ref.abs().amax()
         assert float((got - ref).abs().amax()) <= 2e-3 * float(scale)
+
+
+@pytest.mark.parametrize("k", [128, 256])
+@pytest.mark.parametrize("rows", [1, 127, 129, 1359, 40000, 70001])
+@pytest.mark.parametrize("n,norm_cols", [(128, 128), (256, 128), (512, 256), (100, 64)])
+@pytest.mark.parametrize("gain_dtype", [torch.float32, torch.float16])
+def test_head_norm_against_the_separate_passes(cuda, k, rows, n, norm_cols, gain_dtype):
+    # nori_linear_f16_head_norm against nori_linear_f16 and the RMSNorm of each head of 64: row counts
+    # below, at and past the 128- and 256-row blocks and several blocks a workgroup, and widths with a
+    # part column chunk. Operands are dyadic, so both projections hold the same values; the mean of
+    # squares is summed in another order, so a normed value may round to the neighbouring fp16 and
+    # its product with the gain to one more: 2 ulps, 2^-9 of the value.
+    g = torch.Generator().manual_seed(rows + n + k)
+    x = dyadic((rows, k), 1 / 8, 4.0, g, cuda)
+    w = dyadic((n, k), 1 / 64, 1.0, g, cuda)
+    gain = (torch.rand(64, generator=g) + 0.5).to(gain_dtype).to(cuda)
+    got = projection.linear_head_norm(x, w, gain, 1e-6, norm_cols)
+    plain = kernel_linear(x, w)
+    assert torch.equal(got[:, norm_cols:], plain[:, norm_cols:])
+    heads = plain[:, :norm_cols].float().view(rows, -1, 64)
+    want = (heads * torch.rsqrt(heads.square().mean(-1, keepdim=True) + 1e-6)).half().float() * gain.float()
+    want = want.half().float().view(rows, norm_cols)
+    assert bool(((got[:, :norm_cols].float() - want).abs() <= 2.0**-9 * want.abs() + 2.0**-24).all())
+    strided = torch.zeros(3, rows, k + 8, dtype=torch.float16, device=cuda)
+    strided[1, :, :k] = x
+    assert torch.equal(projection.linear_head_norm(strided[1:2, :, :k], w, gain, 1e-6, norm_cols)[0], got)
