@@ -5,19 +5,28 @@
 // back for the gate and writes [rows, h], and the down projection reads that again; here the
 // hidden activations of a row tile never leave the CU.
 //
-// Workgroup: NW wavefronts of 32 rows each. Per chunk of 32 hidden units:
-//   1. up:   G^T, U^T [32 hidden x 32 rows] = W{g,u}[chunk] . X^T on v_mfma_f32_32x32x16_f16
-//            (A: weight rows staged in LDS; B: the wavefront's X fragments, held in registers
-//            for the whole kernel);
-//   2. gate: a = f16(f16(silu(f16(g))) * f16(u)) in registers; one v_permlane32_swap per word
+// Workgroup: four wavefronts of 32 rows each, two (width 128: three) of them on a CU. Per chunk of
+// 16 hidden units:
+//   1. up:   G^T, U^T [16 hidden x 32 rows] = W{g,u}[chunk] . X^T on v_mfma_f32_16x16x32_f16 (A:
+//            weight rows staged in LDS; B: the wavefront's X fragments, held in registers for the
+//            whole kernel);
+//   2. gate: a = f16(f16(silu(f16(g))) * f16(u)) in registers; one v_permlane16_swap per word
 //            pair turns the C layout into the B operand of step 3;
-//   3. down: Y^T [width x 32 rows] += Wd[:, chunk] . a^T, accumulated over every chunk.
-// The weight chunks (gate and up rows [64, width], down columns [width, 32]) go global -> LDS
-// directly (global_load_lds_dwordx4: no staging registers, no LDS write instructions) into a
+//   3. down: Y^T [width x 32 rows] += Wd[:, chunk] . a^T on v_mfma_f32_32x32x16_f16, accumulated
+//            over every chunk.
+// The weight chunks (gate and up rows [32, width], down columns [width, 16]) go global -> LDS
+// directly (buffer loads to LDS: no staging registers, no LDS write instructions) into a
 // double-buffered ring, the next chunk's loads in flight while the current chunk computes; one
-// barrier per chunk. The weight chunks stream through every workgroup: at width 256 the
-// staging costs about a third of the kernel's time (measured by leaving it out), the gate's
-// VALU work about an eighth.
+// barrier per chunk.
+//
+// What bounds it: an LDS read of a weight operand serves one 32-cycle MFMA of one wavefront, so the
+// LDS pipe and the matrix pipe of a CU are equally loaded (width 128: HBM as well, 8 to 20 bytes
+// an element of x). Chunks of 32 on 32x32x16 MFMAs took 32 registers for G^T and U^T, which left one
+// wavefront per SIMD at width 256 (one workgroup of 108 KB), each operand read just before its
+// MFMA: 163,840 rows of 256 (hidden 704) 315 us plain and 380 us with the residual epilogue, against
+// 210 us (845 TFLOP/s) and 246 us; 655,360 rows of 128 (256) 262 and 362 against 220 and 291 us
+// (3.5 TB/s); 33,792 rows of 352 (960) 185 against 151 us. Workgroups of eight wavefronts, which
+// stage a chunk for twice the rows: 230, 298, 251 and 355 us.
 //
 // nori_swiglu_mlp_residual_rms_norm ends the kernel with the deep-norm residual update of an
 // fp32 stream and the next sublayer's RMSNorm (no weight) instead of writing y: per row
@@ -25,7 +34,7 @@
 // groups of NW columns (the whole row, or 128-column tokens of a wider row) -- bit for bit
 // nori_swiglu_mlp followed by nori_residual_add_rms_norm: the sum of squares runs in that
 // kernel's order (an fma chain over each 4-column chunk, then pairwise over the chunk index
-// bits from the highest; a lane here holds every chunk of its half-row, chunk 8 t + 2 j + hh).
+// bits from the highest).
 //
 // Rounding: the projections sum in fp32 and round to fp16 as hipBLASLt's fp16 GEMMs do, but in
 // their own order, so a value can differ from the unfused sequence's by one fp16 ulp where the
@@ -42,35 +51,13 @@ namespace {
 
 using namespace nori;
 
-constexpr int HC = 32;  // hidden units per chunk
+// gate | up weights are addressed by 32-bit byte offsets (2 GiB)
+constexpr int64_t kMaxWeights = 0x7fffffff / 4;
 constexpr float kLog2eF = 1.4426950408889634f;
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
-
-// Wavefronts per workgroup: eight (two per SIMD) at width 128, whose Y^T accumulators
-// (width / 2 registers), X fragments (width / 4) and chunk G^T, U^T (32) leave the compiler
-// room in 256 registers; four above (at width 256 an eight-wavefront build spills and runs
-// 4-6 % slower).
-constexpr int waves_for(int e) { return e <= 128 ? 8 : 4; }
-
-template <int E>
-struct MlpGeom {
-    static_assert(E % 32 == 0, "width is a multiple of 32");
-    static constexpr int NW = waves_for(E);
-    static constexpr int THREADS = 64 * NW;
-    static constexpr int KS = E / 16;  // k-steps of the up projection
-    static constexpr int OT = E / 32;  // 32-row tiles of Y^T
-    // A chunk in LDS, in 16-byte granules: gate rows 0-31 then up rows 0-31, each E/8 granules
-    // and one of padding (the 16 lanes of a b128 read then land on distinct banks), then the
-    // down rows [E, 32 hidden], 4 granules and one of padding each.
-    static constexpr int GROW = E / 8 + 1;
-    static constexpr int NG = 2 * HC * GROW;
-    static constexpr int NDG = E * 5;
-    static constexpr int LOADS = (NG + NDG + 63) / 64;  // wavefront loads of 64 granules
-    static constexpr int BUF = LOADS * 64 * 8;           // f16 per ring buffer
-};
 
 __device__ __forceinline__ uint32_t pack_f16(float a, float b) {
     const f16x2 h = f16x2{(_Float16)pin_f32(a), (_Float16)pin_f32(b)};
@@ -98,190 +85,261 @@ struct ResEpi {
     int64_t y_group, y_group_stride, y_row_stride;
 };
 
-// NW: 0 writes y = the MLP's output (rows ys apart); else the residual epilogue with norm
-// groups of NW columns.
+// The epilogue for a wavefront's 32 rows from r0, from its Y^T tiles (element 4j + i of tile t is
+// output 32t + 8j + 4hh + i of row l32). u = f16(y) goes through the wavefront's LDS slice, 16 rows
+// at a time, into a row layout: a stream row moves in 256-byte pieces (lane l takes rows 4p + l/16
+// at columns 64q + 4 (l % 16)) and an output row whole, where the MFMA layout touched 32 rows in
+// 32-byte pieces an instruction. The slice is the wavefront's own: LDS runs its accesses in order.
 template <int E, int NW>
-__global__ void __launch_bounds__(MlpGeom<E>::THREADS)
+__device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r0, int64_t rows, int lane, _Float16* ut,
+                                           uint16_t* __restrict__ y, int64_t ys, const ResEpi& ep) {
+    constexpr int UP = E + 8, NCH = (E + 63) / 64;
+    const int l32 = lane & 31, hh = lane >> 5;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if ((l32 >> 4) == h) {
+            _Float16* ur = ut + (l32 & 15) * UP + 4 * hh;
+#pragma unroll
+            for (int t = 0; t < E / 32; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    *reinterpret_cast<u32x2*>(ur + 32 * t + 8 * j) =
+                        u32x2{pack_f16(yt[t][4 * j], yt[t][4 * j + 1]), pack_f16(yt[t][4 * j + 2], yt[t][4 * j + 3])};
+        }
+        asm volatile("" ::: "memory");
+        const int64_t rh = r0 + 16 * h;
+        if constexpr (NW == 0) {
+            constexpr int LPR = E / 8;  // 16-byte pieces per row
+#pragma unroll
+            for (int k = 0; k < (16 * LPR + 63) / 64; ++k) {
+                const int e = lane + 64 * k, rr = e / LPR, c = 8 * (e % LPR);
+                if (rr < 16 && rh + rr < rows)
+                    *reinterpret_cast<u32x4*>(y + (rh + rr) * ys + c) = *reinterpret_cast<const u32x4*>(ut + rr * UP + c);
+            }
+        } else {
+            static_assert(NW == 0 || (E % 64 == 0 && NW % 64 == 0), "norm groups of whole 64-column chunks");
+            constexpr int GC = NW > 0 ? NW / 64 : 1, GROUPS = NW > 0 ? E / NW : 1;
+            const int c4 = 4 * (lane & 15);
+            f32x4 v[4][NCH];
+            float part[4][NCH];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int rr = 4 * p + (lane >> 4);
+                const bool ok = rh + rr < rows;
+                const float* xr = ep.xs + (ok ? rh + rr : r0) * ep.xs_row + c4;
+#pragma unroll
+                for (int q = 0; q < NCH; ++q) v[p][q] = *reinterpret_cast<const f32x4*>(xr + 64 * q);
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int rr = 4 * p + (lane >> 4);
+                const bool ok = rh + rr < rows;
+                float* xr = ep.xs + (ok ? rh + rr : r0) * ep.xs_row + c4;
+#pragma unroll
+                for (int q = 0; q < NCH; ++q) {
+                    const u32x2 uw = *reinterpret_cast<const u32x2*>(ut + rr * UP + 64 * q + c4);
+                    float s = 0.f;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float u = f16_to_f32((uint16_t)(uw[e >> 1] >> (16 * (e & 1))));
+                        v[p][q][e] = v[p][q][e] + round_to<NORI_F16>(u * ep.alpha);
+                        s = fmaf(v[p][q][e], v[p][q][e], s);
+                    }
+                    part[p][q] = s;
+                    if (ok) *reinterpret_cast<f32x4*>(xr + 64 * q) = v[p][q];
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const int64_t row = rh + 4 * p + (lane >> 4);
+#pragma unroll
+                for (int k = 0; k < GROUPS; ++k) {
+                    // chunk 16 q + l % 16 of the group: pairs over its index bits from the highest, the
+                    // q's in the lane, then the 16 lanes
+                    float t[GC];
+#pragma unroll
+                    for (int q = 0; q < GC; ++q) t[q] = part[p][k * GC + q];
+#pragma unroll
+                    for (int st = GC / 2; st >= 1; st >>= 1) {
+#pragma unroll
+                        for (int q = 0; q < st; ++q) t[q] = t[q] + t[q + st];
+                    }
+                    float tot = t[0];
+#pragma unroll
+                    for (int off = 8; off > 0; off >>= 1) tot = tot + __shfl_xor(tot, off);
+                    const float inv = rsqrtf(tot / (float)(NW > 0 ? NW : 1) + ep.eps);
+                    if (row < rows) {
+                        const int64_t qr = row * GROUPS + k;
+                        uint16_t* yr = y + (qr / ep.y_group) * ep.y_group_stride + (qr % ep.y_group) * ep.y_row_stride + c4;
+#pragma unroll
+                        for (int q = 0; q < GC; ++q) {
+                            uint16_t o[4];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) o[e] = f32_to_f16(v[p][k * GC + q][e] * inv);
+                            *reinterpret_cast<u32x2*>(yr + 64 * q) =
+                                u32x2{o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16)};
+                        }
+                    }
+                }
+            }
+        }
+        asm volatile("" ::: "memory");
+    }
+}
+
+// Operand reads in flight: each LDS read is issued kAhead reads before its MFMA and the order is
+// fenced; left to itself the compiler reads an operand just before its MFMA and waits.
+constexpr int kAhead = 4;
+
+// 16 bytes per lane from byte voff + soff of a buffer to LDS at dst + 16 * lane (dst uniform)
+__device__ __forceinline__ void buffer_to_lds(__amdgpu_buffer_rsrc_t r, lds_void* dst, uint32_t voff, int soff) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, (int)voff, soff, 0, 0);
+#endif
+}
+
+template <int E>
+struct MlpGeom {
+    static constexpr int NWAVES = 4;
+    static constexpr int THREADS = 64 * NWAVES;
+    static constexpr int HC = 16;         // hidden units per chunk
+    static constexpr int S = E / 32;      // k-steps of the up projection
+    static constexpr int OT = E / 32;     // 32-row tiles of Y^T
+    // 16-byte granules of a chunk in LDS: 16 gate then 16 up rows of E/8 granules and one of padding,
+    // then E down rows of 2 granules and one of padding; both parts fill whole wavefront loads
+    static constexpr int GROW = E / 8 + 1;
+    static constexpr int GLOADS = (2 * HC * GROW + 63) / 64;
+    static constexpr int DLOADS = (3 * E + 63) / 64;
+    static constexpr int LOADS = GLOADS + DLOADS;
+    static constexpr int PER = (LOADS + NWAVES - 1) / NWAVES;
+    static constexpr int BUF = LOADS * 64 * 8;  // f16 per ring buffer
+    static_assert(NWAVES * 16 * (E + 8) <= 2 * BUF, "the epilogue's rows fit the ring");
+};
+
+template <int E, int NW>
+__global__ void __launch_bounds__(MlpGeom<E>::THREADS) __attribute__((amdgpu_waves_per_eu(E <= 128 ? 3 : (E <= 256 ? 2 : 1))))
 swiglu_mlp_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t xs, const uint16_t* __restrict__ wgu,
-                  const uint16_t* __restrict__ wd, int hp, uint16_t* __restrict__ y, int64_t ys, const ResEpi ep) {
+                    const uint16_t* __restrict__ wd, int hp, uint16_t* __restrict__ y, int64_t ys, const ResEpi ep) {
     using G = MlpGeom<E>;
     __shared__ __attribute__((aligned(16))) _Float16 ring[2 * G::BUF];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5, l16 = lane & 15, g4 = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t r0 = (int64_t)blockIdx.x * (G::NWAVES * 32) + wave * 32;
+    const int nch = hp / G::HC;
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-    const int64_t r0 = (int64_t)blockIdx.x * (G::NW * 32) + wave * 32;
-    const int nch = hp / HC;
-
-    // ---- staging: wavefront load i (i = wave, wave + NW, ...) fills granules [64i, 64i + 64)
-    // of a buffer, lane l granule 64i + l; padding granules (and the tail past the chunk) load
-    // a valid weight granule that nothing reads
-    auto fetch = [&](int h0, int b) {
+    // ---- staging: wavefront load i = wave, wave + NWAVES, ... of the chunk; padding granules load a
+    // valid weight granule that nothing reads. Byte offsets of the lane's granules in chunk 0.
+    const __amdgpu_buffer_rsrc_t rgu = __builtin_amdgcn_make_buffer_rsrc((void*)wgu, 0, 4 * hp * E, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)wd, 0, 2 * hp * E, 0x00020000);
+    uint32_t voff[G::PER];
 #pragma unroll
-        for (int k = 0; k < (G::LOADS + G::NW - 1) / G::NW; ++k) {
-            const int i = wave + k * G::NW;
-            if (i >= G::LOADS) break;  // uniform over the wavefront
-            const int q = 64 * i + lane;
-            const uint16_t* src;
-            if (q < G::NG) {
-                const int row = q / G::GROW, cp = min(q % G::GROW, E / 8 - 1);
-                src = wgu + ((int64_t)(row / HC) * hp + h0 + row % HC) * E + 8 * cp;
-            } else {
-                const int qd = min(q - G::NG, G::NDG - 1), e = qd / 5, cp = min(qd % 5, 3);
-                src = wd + (int64_t)e * hp + h0 + 8 * cp;
-            }
-            __builtin_amdgcn_global_load_lds(src, (lds_void*)(ring + b * G::BUF + 512 * i), 16, 0, 0);
-        }
-    };
-
-    // ---- X fragments (B operand of the up projection): lane holds x[row][16s + 8hh + 0..7]
-    f16x8 xf[G::KS];
-    {
-        const int64_t row = r0 + l32;
-        const bool ok = row < rows;
-#pragma unroll
-        for (int s = 0; s < G::KS; ++s) {
-            u32x4 v = u32x4{0u, 0u, 0u, 0u};
-            if (ok) v = *reinterpret_cast<const u32x4*>(x + row * xs + 16 * s + 8 * hh);
-            xf[s] = __builtin_bit_cast(f16x8, v);
+    for (int k = 0; k < G::PER; ++k) {
+        const int i = wave + k * G::NWAVES;
+        if (i < G::GLOADS) {
+            const int q = min(64 * i + lane, 2 * G::HC * G::GROW - 1);
+            const int row = q / G::GROW, cp = min(q % G::GROW, E / 8 - 1);
+            voff[k] = (uint32_t)((((row / G::HC) * hp + row % G::HC) * E + 8 * cp) * 2);
+        } else {
+            const int q = min(64 * (i - G::GLOADS) + lane, 3 * E - 1), e = q / 3, cp = min(q % 3, 1);
+            voff[k] = (uint32_t)((e * hp + 8 * cp) * 2);
         }
     }
+    auto fetch = [&](int c, int b) {
+#pragma unroll
+        for (int k = 0; k < G::PER; ++k) {
+            const int i = wave + k * G::NWAVES;
+            if (i >= G::LOADS) break;  // uniform over the wavefront
+            lds_void* dst = (lds_void*)(ring + b * G::BUF + 512 * i);
+            if (i < G::GLOADS) buffer_to_lds(rgu, dst, voff[k], c * G::HC * E * 2);
+            else buffer_to_lds(rd, dst, voff[k], c * G::HC * 2);
+        }
+    };
+    fetch(0, 0);
 
+    // ---- X fragments (B operands): row tile t holds x[r0 + 16t + l16][32s + 8 g4 + 0..7]
+    f16x8 xf[2][G::S];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int64_t row = r0 + 16 * t + l16;
+        const bool ok = row < rows;
+#pragma unroll
+        for (int s = 0; s < G::S; ++s) {
+            u32x4 v = u32x4{0u, 0u, 0u, 0u};
+            if (ok) v = *reinterpret_cast<const u32x4*>(x + row * xs + 32 * s + 8 * g4);
+            xf[t][s] = __builtin_bit_cast(f16x8, v);
+        }
+    }
     f32x16 yt[G::OT];
 #pragma unroll
     for (int t = 0; t < G::OT; ++t) yt[t] = f32x16{};
-
-    fetch(0, 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
 
+    const int up_lane = 8 * (l16 * G::GROW + g4);                 // gate row l16 (up rows: HC further)
+    const int dn_lane = 8 * (64 * G::GLOADS + 3 * l32 + hh);      // down row l32
     for (int c = 0; c < nch; ++c) {
         const int cur = c & 1;
-        // the next chunk into the other buffer, whose last reads were in chunk c-1 (before the
-        // previous barrier); it lands while this chunk computes
-        if (c + 1 < nch) fetch(HC * (c + 1), cur ^ 1);
-        const _Float16* Gc = ring + cur * G::BUF;
-        const _Float16* Dc = Gc + 8 * G::NG;
-
-        // 1. G^T and U^T of the chunk
-        f32x16 gt = f32x16{}, ut = f32x16{};
+        if (c + 1 < nch) fetch(c + 1, cur ^ 1);
+        const _Float16* Wc = ring + cur * G::BUF;
+        // operand reads of the chunk in order: gate and up rows of each k-step, then the down tiles
+        auto rd_op = [&](int i) {
+            const _Float16* p = i < 2 * G::S ? Wc + up_lane + 8 * ((i & 1) * G::HC * G::GROW + 4 * (i >> 1))
+                                             : Wc + dn_lane + 8 * 3 * 32 * (i - 2 * G::S);
+            return *reinterpret_cast<const f16x8*>(p);
+        };
+        f16x8 op[kAhead];
 #pragma unroll
-        for (int s = 0; s < G::KS; ++s) {
-            const f16x8 ag = *reinterpret_cast<const f16x8*>(Gc + 8 * (l32 * G::GROW + 2 * s + hh));
-            const f16x8 au = *reinterpret_cast<const f16x8*>(Gc + 8 * ((HC + l32) * G::GROW + 2 * s + hh));
-            gt = __builtin_amdgcn_mfma_f32_32x32x16_f16(ag, xf[s], gt, 0, 0, 0);
-            ut = __builtin_amdgcn_mfma_f32_32x32x16_f16(au, xf[s], ut, 0, 0, 0);
-        }
-
-        // 2. the gate, as words w[j][p] = hidden 8j + 4hh + 2p + {0, 1} of row l32, then the
-        //    B operands of the down projection: k-step ks holds hidden 16ks + 8hh + 0..7
-        uint32_t w[4][2];
+        for (int i = 0; i < kAhead; ++i) op[i] = rd_op(i);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 gt[2], ut[2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int t = 0; t < 2; ++t) gt[t] = ut[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
-                const int i0 = 4 * j + 2 * p;
-                w[j][p] = gate_pair(gt[i0], gt[i0 + 1], ut[i0], ut[i0 + 1]);
+        for (int s = 0; s < G::S; ++s) {
+            const int i = 2 * s;
+            const f16x8 ag = op[i % kAhead], au = op[(i + 1) % kAhead];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                gt[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ag, xf[t][s], gt[t], 0, 0, 0);
+                ut[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(au, xf[t][s], ut[t], 0, 0, 0);
             }
-        f16x8 af[2];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            // lanes 0-31 keep their words of hidden 16ks + 0..3 and take 4..7 from lane +32;
-            // lanes 32-63 keep 16ks + 12..15 and take 8..11 from lane -32
-            const auto s0 = __builtin_amdgcn_permlane32_swap(w[2 * ks][0], w[2 * ks + 1][0], false, false);
-            const auto s1 = __builtin_amdgcn_permlane32_swap(w[2 * ks][1], w[2 * ks + 1][1], false, false);
-            af[ks] = __builtin_bit_cast(f16x8, u32x4{s0[0], s1[0], s0[1], s1[1]});
+            op[i % kAhead] = rd_op(i + kAhead);
+            op[(i + 1) % kAhead] = rd_op(i + 1 + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
         }
-
-        // 3. Y^T += Wd[:, chunk] a^T
+        // the gate: word p of row tile t holds hidden 4 g4 + 2p + {0, 1} of row l16; swapping the tiles'
+        // words between 16-lane rows gives lane l the hidden units 8 hh + 0..7 of row l32
+        uint32_t w[2][2];
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int t = 0; t < G::OT; ++t) {
-                const f16x8 ad = *reinterpret_cast<const f16x8*>(Dc + 8 * ((32 * t + l32) * 5 + 2 * ks + hh));
-                yt[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ad, af[ks], yt[t], 0, 0, 0);
-            }
-
+            for (int p = 0; p < 2; ++p) w[t][p] = gate_pair(gt[t][2 * p], gt[t][2 * p + 1], ut[t][2 * p], ut[t][2 * p + 1]);
+        const auto s0 = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+        const auto s1 = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+        const f16x8 af = __builtin_bit_cast(f16x8, u32x4{s0[0], s1[0], s0[1], s1[1]});
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < G::OT; ++t) {
+            const int i = 2 * G::S + t;
+            const f16x8 ad = op[i % kAhead];
+            yt[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ad, af, yt[t], 0, 0, 0);
+            if (t + kAhead < G::OT) op[i % kAhead] = rd_op(i + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (c + 1 < nch) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's loads are in LDS
             __syncthreads();
         }
     }
-
-    // ---- y[row][e .. e+3] from Y^T: element 4j + i of tile t is e = 32t + 8j + 4hh + i
-    const int64_t row = r0 + l32;
-    if constexpr (NW > 0) {
-        static_assert(E % NW == 0 && NW % 32 == 0, "norm groups of whole tiles");
-        constexpr int TT = NW / 32;  // tiles per norm group
-        const bool ok = row < rows;
-        float* xr = ep.xs + (ok ? row : 0) * ep.xs_row;
-        float part[G::OT][4];
-#pragma unroll
-        for (int t = 0; t < G::OT; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = 32 * t + 8 * j + 4 * hh;
-                const f32x4 xv = ok ? *reinterpret_cast<const f32x4*>(xr + e) : f32x4{0.f, 0.f, 0.f, 0.f};
-                float p = 0.f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float u = round_to<NORI_F16>(yt[t][4 * j + i]);
-                    const float v = xv[i] + round_to<NORI_F16>(u * ep.alpha);
-                    yt[t][4 * j + i] = v;
-                    p = fmaf(v, v, p);
-                }
-                if (ok) *reinterpret_cast<f32x4*>(xr + e) = f32x4{yt[t][4 * j], yt[t][4 * j + 1], yt[t][4 * j + 2], yt[t][4 * j + 3]};
-                part[t][j] = p;
-            }
-#pragma unroll
-        for (int k = 0; k < E / NW; ++k) {
-            // chunk 8 t' + 2 j + hh of the group (t' = t - k TT): pairs over (t', j) from the
-            // highest bit in the lane, then over hh (lane bit 5)
-            float q[4 * TT];
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) q[4 * t + j] = part[k * TT + t][j];
-#pragma unroll
-            for (int st = 2 * TT; st >= 1; st >>= 1) {
-#pragma unroll
-                for (int i = 0; i < st; ++i) q[i] = q[i] + q[i + st];
-            }
-            float tot = q[0];
-            tot = tot + __shfl_xor(tot, 32);
-            const float inv = rsqrtf(tot / (float)NW + ep.eps);
-            if (ok) {
-                const int64_t qr = row * (E / NW) + k;
-                uint16_t* yr = y + (qr / ep.y_group) * ep.y_group_stride + (qr % ep.y_group) * ep.y_row_stride;
-#pragma unroll
-                for (int t = 0; t < TT; ++t)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const f32x16& v = yt[k * TT + t];
-                        uint16_t h[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) h[i] = f32_to_f16(v[4 * j + i] * inv);
-                        *reinterpret_cast<u32x2*>(yr + 32 * t + 8 * j + 4 * hh) =
-                            u32x2{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16)};
-                    }
-            }
-        }
-    } else if (row < rows) {
-        uint16_t* yr = y + row * ys;
-#pragma unroll
-        for (int t = 0; t < G::OT; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int e = 32 * t + 8 * j + 4 * hh;
-                const f32x16& v = yt[t];
-                *reinterpret_cast<u32x2*>(yr + e) = u32x2{pack_f16(v[4 * j], v[4 * j + 1]), pack_f16(v[4 * j + 2], v[4 * j + 3])};
-            }
-    }
+    __syncthreads();  // the ring's last reads are done: its memory takes the rows
+    write_rows<E, NW>(yt, r0, rows, lane, ring + wave * 16 * (E + 8), y, ys, ep);
 }
 
 template <int E, int NW = 0>
 void launch(const uint16_t* x, int64_t rows, int64_t xs, const uint16_t* wgu, const uint16_t* wd, int hp, uint16_t* y,
             int64_t ys, hipStream_t stream, const ResEpi& ep = ResEpi{}) {
     using G = MlpGeom<E>;
-    const int64_t per = G::NW * 32;
+    const int64_t per = G::NWAVES * 32;
     const dim3 grid((unsigned)((rows + per - 1) / per));
     hipLaunchKernelGGL((swiglu_mlp_kernel<E, NW>), grid, dim3(G::THREADS), 0, stream, x, rows, xs, wgu, wd, hp, y, ys,
                        ep);
@@ -306,6 +364,7 @@ extern "C" int nori_swiglu_mlp(const void* x, int dtype, int64_t rows, int32_t w
     if (!x || !w_gate_up || !w_down || !y) return fail(NORI_ERR_INVALID, "swiglu_mlp: null pointer");
     if ((uintptr_t)x % 16 || (uintptr_t)w_gate_up % 16 || (uintptr_t)w_down % 16 || (uintptr_t)y % 16)
         return fail(NORI_ERR_INVALID, "swiglu_mlp: x, the weights and y must be 16-byte aligned");
+    if ((int64_t)hidden * width > kMaxWeights) return fail(NORI_ERR_UNSUPPORTED, "swiglu_mlp: hidden width %d", hidden);
     hipStream_t stream = (hipStream_t)stream_v;
     auto xp = reinterpret_cast<const uint16_t*>(x);
     auto gp = reinterpret_cast<const uint16_t*>(w_gate_up);
@@ -344,6 +403,8 @@ extern "C" int nori_swiglu_mlp_residual_rms_norm(const void* x, int dtype, int64
         (uintptr_t)y % 8)
         return fail(NORI_ERR_INVALID, "swiglu_mlp_residual_rms_norm: x, the weights and the stream must be 16-byte "
                     "aligned, y 8-byte aligned");
+    if ((int64_t)hidden * width > kMaxWeights)
+        return fail(NORI_ERR_UNSUPPORTED, "swiglu_mlp_residual_rms_norm: hidden width %d", hidden);
     const ResEpi ep{stream_rows, stream_row_stride, alpha, eps, y_group, y_group_stride, y_row_stride};
     hipStream_t stream = (hipStream_t)stream_v;
     auto xp = reinterpret_cast<const uint16_t*>(x);
