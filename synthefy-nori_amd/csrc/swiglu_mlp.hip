@@ -125,8 +125,8 @@ __device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 const int rr = 4 * p + (lane >> 4);
-                const bool ok = rh + rr < rows;
-                const float* xr = ep.xs + (ok ? rh + rr : r0) * ep.xs_row + c4;
+                // (rows past the last, a whole wavefront's in the last workgroup, read the last again)
+                const float* xr = ep.xs + (rh + rr < rows ? rh + rr : rows - 1) * ep.xs_row + c4;
 #pragma unroll
                 for (int q = 0; q < NCH; ++q) v[p][q] = *reinterpret_cast<const f32x4*>(xr + 64 * q);
             }
@@ -134,7 +134,7 @@ __device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r
             for (int p = 0; p < 4; ++p) {
                 const int rr = 4 * p + (lane >> 4);
                 const bool ok = rh + rr < rows;
-                float* xr = ep.xs + (ok ? rh + rr : r0) * ep.xs_row + c4;
+                float* xr = ep.xs + (ok ? rh + rr : rows - 1) * ep.xs_row + c4;
 #pragma unroll
                 for (int q = 0; q < NCH; ++q) {
                     const u32x2 uw = *reinterpret_cast<const u32x2*>(ut + rr * UP + 64 * q + c4);
