@@ -34,6 +34,37 @@ int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t n_mid, int
                               int64_t y_row_stride, const void* gain, int gain_dtype, float eps, int32_t norm_cols,
                               void* stream);
 
+// One dense "smf" layer over query rows against its context cache, every launch from one call
+// (dense_layer.hip): x [tables, rows, groups, embed] fp32 contiguous is left as it is, out (the same
+// shape) takes the layer's output. Weights fp16, contiguous, as the module keeps them: w_q, w_out,
+// w_feat_out [embed, embed], w_qkv [3 embed, embed], the QASS MLPs ([64, 1 | head width], [64],
+// [embed | head width, 64], ...), gate_up [2 hidden, embed] and down [embed, hidden] with hidden a
+// multiple of 32. The cache as nori_icl_attention takes it; alpha the deep-norm factor as rounded to
+// fp16. embed is 128 or 256 (the norm after the MLP is over embed columns); two keys or more.
+typedef struct {
+    int64_t tables, rows, groups;
+    int32_t embed, heads;
+    const float* x;
+    float* out;
+    const void *w_q, *w_out, *w_qkv, *w_feat_out;
+    const void *base_w1, *base_b1, *base_w2, *base_b2, *gate_w1, *gate_b1, *gate_w2, *gate_b2;
+    int32_t qass_hidden;
+    const void *gate_up, *down;
+    int32_t hidden;
+    float eps_seq, eps_mlp, eps_feat, alpha, logit_scale, log_n;
+    const void* kv;
+    int32_t kv_dtype;
+    const float* kv_scales;
+    int64_t nk;
+    int32_t kv_heads;
+    int64_t kv_bg, kv_row, kv_half, sc_bg, sc_row, sc_half;
+    void* scratch;
+    int64_t scratch_bytes;
+} nori_dense_apply_args;
+
+int64_t nori_dense_apply_scratch_bytes(int64_t tables, int64_t rows, int64_t groups, int32_t embed, int32_t heads, int64_t nk);
+int nori_dense_apply(const nori_dense_apply_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -114,6 +114,21 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "nori_quant_f16_scale_probe": (ctypes.c_int, [_vp, _i64, _vp, _vp, _vp]),
 }
 
+class DenseApplyArgs(ctypes.Structure):
+    """``nori_dense_apply_args``."""
+
+    _fields_ = (
+        [(n, _i64) for n in ("tables", "rows", "groups")] + [("embed", _i32), ("heads", _i32)]
+        + [(n, _vp) for n in ("x", "out", "w_q", "w_out", "w_qkv", "w_feat_out", "base_w1", "base_b1", "base_w2", "base_b2",
+                              "gate_w1", "gate_b1", "gate_w2", "gate_b2")]
+        + [("qass_hidden", _i32), ("gate_up", _vp), ("down", _vp), ("hidden", _i32)]
+        + [(n, _f32) for n in ("eps_seq", "eps_mlp", "eps_feat", "alpha", "logit_scale", "log_n")]
+        + [("kv", _vp), ("kv_dtype", _i32), ("kv_scales", _vp), ("nk", _i64), ("kv_heads", _i32)]
+        + [(n, _i64) for n in ("kv_bg", "kv_row", "kv_half", "sc_bg", "sc_row", "sc_half")]
+        + [("scratch", _vp), ("scratch_bytes", _i64)]
+    )
+
+
 # The package's own entry points beyond the C ABI (csrc/nori_ops.h).
 OPS: dict[str, tuple[object, list]] = {
     "nori_qass_base": (ctypes.c_int, [_f32, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp]),
@@ -121,6 +136,8 @@ OPS: dict[str, tuple[object, list]] = {
         ctypes.c_int,
         [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _i32, _vp, _i64, _i64, _i64, _vp, _i32, _f32, _i32, _vp],
     ),
+    "nori_dense_apply_scratch_bytes": (_i64, [_i64, _i64, _i64, _i32, _i32, _i64]),
+    "nori_dense_apply": (ctypes.c_int, [ctypes.POINTER(DenseApplyArgs), _vp]),
     "nori_rms_norm_rows": (ctypes.c_int, [_vp, _i64, _i32, _i64, _i64, _i64, _i64, _i64, _f32, _vp, _i32, _vp]),
 }
 
@@ -195,7 +212,8 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream_of(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)  # current_stream(device).cuda_stream without the Stream object
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

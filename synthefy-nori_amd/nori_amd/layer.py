@@ -36,6 +36,7 @@ import torch.nn as nn
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .attention import attend_dense, compute_attention_blockwise, icl_attention, takes_prologue
+from . import _native as nat
 from . import kv_project
 from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
@@ -759,6 +760,15 @@ def _report_sdpa_once() -> None:
         )
 
 
+def _hooked(*modules: nn.Module) -> bool:
+    """Whether a call of any of the modules, or of one inside them, would run a forward hook."""
+    from torch.nn.modules import module as base
+
+    if base._global_forward_hooks or base._global_forward_pre_hooks:
+        return True
+    return any(m._forward_hooks or m._forward_pre_hooks for top in modules for m in top.modules())
+
+
 class EncoderBaseLayer(nn.Module):
     """Reference ``EncoderBaseLayer`` (layer.py:1164-1967), cached-inference paths."""
 
@@ -1213,8 +1223,90 @@ class EncoderBaseLayer(nn.Module):
                                   eval_pos)
         return self._add_then_steps(x, first, pre_steps[1:], feature_atten_mask, eval_pos, then_norm=seq_norm)
 
+    # small layers of the fused widths issue their launches from one native call
+    # (nori_dense_apply); False keeps the sublayers' own calls
+    native_apply = True
+    # Past this many tokens the kernels of a layer outlast the host's part of it, and its wider
+    # projections keep the library GEMM: 6m stack of 16 layers over 9 x 256 tokens 4.9 -> 1.6 ms; at
+    # 64 k tokens the two are level.
+    _NATIVE_TOKENS = 65536
+
+    def _apply_native(self, x: torch.Tensor, kv_cache, feature_atten_mask) -> torch.Tensor | None:
+        """``forward_test_with_cache`` as one native call, or None where that is not the same
+        computation: inference under fp16 autocast on an fp32 stream, the plain modules of an "smf"
+        pre-norm layer of 128 or 256 (SwiGLU, RMSNorm, QASS "full"), a resident cache."""
+        if not (self.native_apply and type(self) is EncoderBaseLayer and self.layer_arch == "smf" and self.pre_norm
+                and feature_atten_mask is None and x.is_cuda and x.dtype == torch.float32 and x.dim() == 4
+                and x.is_contiguous() and not torch.is_grad_enabled() and not self.training
+                and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.float16):
+            return None
+        b, r, g, e = x.shape
+        n = b * r * g
+        if e not in (128, 256) or e != self.embed_dim or not 0 < n <= self._NATIVE_TOKENS:
+            return None
+        if x.data_ptr() % 16 or type(kv_cache) is not ScalableSeqKV or kv_cache.offloaded:
+            return None
+        if int(kv_cache.batch) != b or int(kv_cache.groups) != g:
+            return None
+        seq = self.sequence_attentions[1 if self.seq_attn_isolated else 0]
+        feat, mlp, norms = self.feature_attentions[0], self.mlp[0], self.layer_norms
+        qass = seq.qassmax
+        if type(seq) is not MultiheadAttention or type(feat) is not MultiheadAttention or type(mlp) is not SwiGLUMLP \
+                or type(qass) is not QASSMaxScaling or qass.qass_mode != "full" or len(norms) != 3:
+            return None
+        if seq.qkv_combined or not feat.qkv_combined or feat.use_qassmax or seq.qk_norm or feat.qk_norm:
+            return None
+        for m in (seq, feat):
+            if m.use_logn_attention or m.use_learnable_attn_temperature or m.embed_dim != e or m.num_heads != self.nhead:
+                return None
+        for m in norms:
+            if type(m) is not RMSNorm or m.weight is not None or tuple(m.normalized_shape) != (e,):
+                return None
+        if _hooked(feat, mlp, qass, *norms):
+            return None
+        heads, d = seq.num_heads, seq.head_dim
+        payload, scales = kv_cache.device_payload()
+        if payload.device != x.device or payload.dim() != 5 or payload.dtype not in (torch.int8, torch.float16):
+            return None
+        n_keys, kv_heads = int(payload.shape[1]), int(payload.shape[3])
+        if payload.shape[0] != b * g or payload.shape[4] != d or not payload.is_contiguous() or n_keys < 2 or heads % kv_heads:
+            return None
+        if payload.dtype == torch.int8 and (scales is None or scales.dtype != torch.float32 or not scales.is_contiguous()
+                                            or tuple(scales.shape) != (*payload.shape[:-1], 1)):
+            return None
+        q16 = torch.empty(0, dtype=torch.float16, device=x.device)
+        if not (qass.fused and qass._fused_base_applies(q16) and d <= 64 and d % 4 == 0
+                and qass._fused_gate_applies(q16, q16) and mlp.fuses(x)):
+            return None
+        if any(p.device != x.device for p in (seq.qkv_proj_weight, feat.qkv_proj_weight, mlp.w_gate.weight)):
+            return None
+        w_q, _, w_out = seq._linear_weights(x.device)
+        _, _, _, w_feat_out, w_qkv = feat._cast_weights(x.device)
+        base, gate = qass._half_weights("_base16", qass.base_mlp), qass._gate_weights()
+        gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
+        lib = nat.lib()
+        scratch = torch.empty(lib.nori_dense_apply_scratch_bytes(b, r, g, e, heads, n_keys), dtype=torch.uint8, device=x.device)
+        out = torch.empty_like(x)
+        sc = (0, 0, 0) if payload.dtype != torch.int8 else scales.stride()[:3]
+        args = nat.DenseApplyArgs(
+            b, r, g, e, heads, x.data_ptr(), out.data_ptr(), w_q.data_ptr(), w_out.data_ptr(), w_qkv.data_ptr(),
+            w_feat_out.data_ptr(), *(t.data_ptr() for t in base), *(t.data_ptr() for t in gate), QASS_GATE_HIDDEN,
+            gate_up.data_ptr(), down.data_ptr(), hidden, *(float(m.eps) for m in norms), self._alpha_value(q16),
+            1.0 / math.sqrt(float(d)), math.log(float(n_keys)), payload.data_ptr(), nat.dtype_code(payload.dtype),
+            None if payload.dtype != torch.int8 else scales.data_ptr(), n_keys, kv_heads, *payload.stride()[:3], *sc,
+            scratch.data_ptr(), scratch.numel(),
+        )
+        rc = lib.nori_dense_apply(args, nat.stream_of(x.device))
+        if rc == nat.NORI_ERR_UNSUPPORTED:
+            return None
+        nat.check(rc, "dense_apply")
+        return out
+
     def forward_test_with_cache(self, x_test: torch.Tensor, cache: dict, feature_atten_mask: torch.Tensor | None = None):
         """Query rows through one layer against the layer's context cache (layer.py:1915-1967)."""
+        native = self._apply_native(x_test, cache["seq_kv"], feature_atten_mask)
+        if native is not None:
+            return native
         pre_steps, seq_step, post_steps, seq_index = self._cache_steps()
         eval_pos = x_test.shape[1]
         index1 = seq_index * 2 if self.seq_attn_isolated else seq_index

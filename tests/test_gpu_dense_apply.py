@@ -1,0 +1,79 @@
+"""A dense layer's cached apply as one native call (nori_dense_apply) against the same layer's own calls.
+
+Both run the same kernels, except that the projections of short operands go through
+``nori_linear_f16`` in one and the library GEMM in the other: fp32 sums in another order, so a value
+rounded to fp16 can land on its neighbour (2^-11 of it) and moves what follows by as much. Over the
+few such roundings of a layer the 2-norm of the difference stays below 4 * 2^-11 of the update's.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from nori_amd import ScalableSeqKV
+from nori_amd.layer import EncoderBaseLayer
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(embed, heads, shared, seed, device):
+    torch.manual_seed(seed)
+    layer = EncoderBaseLayer(heads, embed, 3 * embed, pre_norm=True, activation="swiglu", norm_type="rmsnorm",
+                             deepnorm_alpha=0.25, layer_arch="smf", seq_attn_isolated=True,
+                             cross_share_all_kv_heads=shared, use_qassmax=True, qass_mode="full")
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.normal_(0.0, p.shape[-1] ** -0.5 if p.dim() > 1 else 0.1)
+    return layer.eval().to(device)
+
+
+@pytest.mark.parametrize("embed,heads", [(128, 2), (128, 4), (256, 4)])
+@pytest.mark.parametrize("tables,rows,groups,keys", [(1, 1, 1, 2), (1, 37, 9, 300), (3, 130, 5, 129), (2, 64, 33, 1024)])
+@pytest.mark.parametrize("shared,quantized", [(False, True), (True, True), (False, False)])
+def test_native_apply_equals_the_layers_calls(cuda, embed, heads, tables, rows, groups, keys, shared, quantized):
+    layer = _layer(embed, heads, shared, embed + heads, cuda)
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(tables, rows, groups, embed, generator=g).to(cuda)
+    kv = torch.randn(tables * groups, keys, 2, 1 if shared else heads, embed // heads, generator=g).half().to(cuda)
+    cache = {"seq_kv": ScalableSeqKV(kv, tables, groups, quantize=quantized)}
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        before = x.clone()
+        taken = layer._apply_native(x, cache["seq_kv"], None) is not None
+        assert taken == (embed == 128 or layer.mlp[0].fuses(x))
+        got = layer.forward_test_with_cache(x, cache)
+        layer.native_apply = False
+        want = layer.forward_test_with_cache(x, cache)
+        assert torch.equal(x, before)
+    err = (got - want).double().norm() / (want - x).double().norm()
+    assert float(err) <= 4 * 2.0**-11
+
+
+def test_other_calls_keep_the_layers_own(cuda):
+    # what is not the plain inference computation, or what a user watches, is not taken over
+    layer = _layer(128, 2, False, 5, cuda)
+    x = torch.randn(1, 20, 4, 128, device=cuda)
+    kv = torch.randn(4, 50, 2, 2, 64, device=cuda).half()
+    cache = ScalableSeqKV(kv, 1, 4, quantize=True)
+
+    def taken(inp=x, c=cache, mask=None):
+        return layer._apply_native(inp, c, mask) is not None
+
+    with torch.inference_mode():
+        assert not taken()  # fp32 projections
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert not taken()
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not taken()  # gradients
+        with torch.inference_mode():
+            assert taken()
+            assert not taken(x.half()) and not taken(x.transpose(1, 2)) and not taken(c={"kv": kv, "batch": 1, "groups": 4})
+            assert not taken(x.expand(2, -1, -1, -1).contiguous())  # another batch than the cache's: the layer raises
+            seen = []
+            for module in (layer.mlp[0].w_down, layer.feature_attentions[0], layer.sequence_attentions[1].qassmax):
+                hook = module.register_forward_hook(lambda *a: seen.append(1))
+                assert not taken()
+                hook.remove()
+            assert taken()
+            layer.train()
+            assert not taken()
