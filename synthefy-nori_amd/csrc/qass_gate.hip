@@ -3,7 +3,7 @@
 //     out = q * base_scale[h] * (1 + tanh(W2 gelu(W1 q + b1) + b2))
 // as QASSMaxScaling.forward computes it under fp16 autocast (src/synthefy_nori/model/
 // layer.py:316-456: the gate MLP Linear(d, 64) -> GELU -> Linear(64, d), then the two
-// multiplies), rounded where torch's separate ops round: each linear's fp32 sum plus its bias
+// multiplies), rounded where torch's separate ops round: each linear's fp32 sum with its bias
 // rounded to fp16, GELU (erf form) and tanh evaluated in fp32 and rounded, 1 + t rounded, the
 // two products rounded in turn. base_scale = log n * (1 + tanh(base_mlp(log n))) is one
 // [heads, d] vector per call, formed by the caller. The separate ops make seven passes over
@@ -20,7 +20,16 @@
 // order, and the query elements a lane loads for the first GEMM are exactly the ones its
 // second-GEMM results belong to. So the epilogue multiplies each result by the query value
 // already in the lane's registers and writes 4 consecutive elements per 8-byte store.
+//
+// What bounds it: VALU issue (64 GELUs and up to 64 tanhs a query vector), a byte's worth of HBM time
+// three times over. With the math library's erf and tanh, a conversion for each rounding and 16,384
+// workgroups that each staged the weights two bytes at a time for one or two tiles, 153,000 rows of 10
+// heads of 56 took 235 us; a GELU of one polynomial and one exponential, packed fp16 products, the
+// biases as the accumulators' start, and resident workgroups that walk tiles with the next tile's
+// queries in flight take 156 us (0.34 GB; 68 us at the copy rate), 139,264 of 2 of 64 54 -> 32 us.
 #include <math.h>
+
+#include <algorithm>
 
 #include "nori_common.h"
 
@@ -34,7 +43,6 @@ using namespace nori;
 constexpr int kWaves = 4;
 constexpr int kHid = 64;    // the gate MLP's hidden width (QASSMaxScaling's hidden_dim)
 constexpr int kPitch = 72;  // f16 per LDS weight row (144 bytes: rows start on different banks)
-constexpr float kSqrtHalf = 0.70710678118654752440f;
 
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -50,28 +58,79 @@ __device__ __forceinline__ f16x8 join(u32x2_t lo, u32x2_t hi) {
     return __builtin_bit_cast(f16x8, u32x4_t{lo[0], lo[1], hi[0], hi[1]});
 }
 
-__device__ __forceinline__ float half_at(u32x2_t w, int i) {
-    return f16_to_f32((uint16_t)(w[i >> 1] >> (16 * (i & 1))));
+__device__ __forceinline__ f16x2 pair_at(u32x2_t w, int i) {
+    const uint32_t x = w[i];
+    return __builtin_bit_cast(f16x2, x);
 }
 
-// torch's GELU (approximate='none') on an fp16 value, in fp32, rounded to fp16
-__device__ __forceinline__ float gelu16(float x) { return r16(x * 0.5f * (1.0f + erff(x * kSqrtHalf))); }
+// two fp32 values rounded to fp16 (each product rounded to fp32 first)
+__device__ __forceinline__ f16x2 pair16(float a, float b) { return f16x2{(_Float16)pin_f32(a), (_Float16)pin_f32(b)}; }
+
+// GELU (the erf form) of an fp16 value in fp32: x Phi(x), with Phi(-|x|) = 2^L(|x|), L a polynomial of
+// degree 8 fitted to log2 Phi(-a) over [0, 5.8] (past it the fp16 result is zero; the leading
+// coefficient keeps L falling) by least squares reweighted towards the largest error: 1.4e-6. Of the
+// 63,488 finite fp16 x, 51 round to another fp16 value than the exact GELU does; x / 2 (1 + erf(x / sqrt
+// 2)) in fp32 with a correctly rounded erf misses 331, its sum cancelling for negative x. +-inf and NaN
+// give what that expression gives.
+__device__ __forceinline__ float gelu(float x) {
+    const float a = fabsf(x);
+    float p = fmaf(a, -4.04897598e-07f, 6.105983e-06f);
+    p = fmaf(p, a, -1.43313975e-06f);
+    p = fmaf(p, a, -0.00067129832f);
+    p = fmaf(p, a, 0.00792131722f);
+    p = fmaf(p, a, -0.0532461218f);
+    p = fmaf(p, a, -0.458885486f);
+    p = fmaf(p, a, -1.15115821f);
+    p = fmaf(p, a, -0.999998548f);
+    const float h = __builtin_amdgcn_exp2f(p);
+    return x * (x >= 0.0f ? 1.0f - h : h);
+}
+
+// tanh in fp32: 1 - 2 / (exp(2 v) + 1), within 2e-7
+__device__ __forceinline__ float tanh_f32(float v) {
+    return fmaf(-2.0f, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * 2.885390081777927f) + 1.0f), 1.0f);
+}
+
+// the biases of a 32 x 32 result's rows as a lane holds them (rows 8 g + 4 hh + 0..3; p at row 4 hh)
+__device__ __forceinline__ f32x16 bias_tile(const float* p) {
+    f32x16 r;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const f32x4 b = *reinterpret_cast<const f32x4*>(p + 8 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[4 * g + i] = b[i];
+    }
+    return r;
+}
 
 template <int KS1, int NT2>  // k-steps of the first GEMM (ceil(d / 16)), 32-row tiles of the second (ceil(d / 32))
 __global__ void __launch_bounds__(64 * kWaves, 4)
 qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, const uint16_t* w1,
                  const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, const uint16_t* bs, uint16_t* out,
-                 int64_t os, int64_t ntiles) {
+                 int64_t os, int64_t ntiles, int vec_w) {
     __shared__ __attribute__((aligned(16))) _Float16 w1s[kHid * kPitch];  // [hidden][k order], zeros past d
     __shared__ __attribute__((aligned(16))) _Float16 w2s[64 * kPitch];    // [output][k order], zero rows past d
     __shared__ __attribute__((aligned(16))) float b1s[kHid];
     __shared__ __attribute__((aligned(16))) float b2s[64];
     const int tid = threadIdx.x;
-    for (int i = tid; i < 64 * 64; i += 64 * kWaves) {
-        const int j = i >> 6, p = i & 63;
-        const int c = 16 * (p >> 4) + kperm((p >> 3) & 1, p & 7);  // source column of LDS column p
-        w1s[j * kPitch + p] = __builtin_bit_cast(_Float16, c < d ? w1[j * d + c] : (uint16_t)0);
-        w2s[j * kPitch + p] = __builtin_bit_cast(_Float16, j < d ? w2[j * kHid + c] : (uint16_t)0);
+    // 4 consecutive LDS columns are 4 consecutive source columns (d is a multiple of 4: all in or out)
+    if (vec_w) {
+#pragma unroll
+        for (int k = 0; k < 64 * 16 / (64 * kWaves); ++k) {
+            const int i = tid + 64 * kWaves * k, j = i >> 4, p = 4 * (i & 15);
+            const int c = 16 * (p >> 4) + kperm((p >> 3) & 1, p & 7);  // source column of LDS column p
+            const u32x2_t a = *reinterpret_cast<const u32x2_t*>(w1 + j * d + min(c, d - 4));
+            const u32x2_t b = *reinterpret_cast<const u32x2_t*>(w2 + min(j, d - 1) * kHid + c);
+            *reinterpret_cast<u32x2_t*>(w1s + j * kPitch + p) = c < d ? a : u32x2_t{0u, 0u};
+            *reinterpret_cast<u32x2_t*>(w2s + j * kPitch + p) = j < d ? b : u32x2_t{0u, 0u};
+        }
+    } else {
+        for (int i = tid; i < 64 * 64; i += 64 * kWaves) {
+            const int j = i >> 6, p = i & 63;
+            const int c = 16 * (p >> 4) + kperm((p >> 3) & 1, p & 7);
+            w1s[j * kPitch + p] = __builtin_bit_cast(_Float16, c < d ? w1[j * d + c] : (uint16_t)0);
+            w2s[j * kPitch + p] = __builtin_bit_cast(_Float16, j < d ? w2[j * kHid + c] : (uint16_t)0);
+        }
     }
     if (tid < 64) {
         b1s[tid] = f16_to_f32(b1[tid]);
@@ -79,18 +138,14 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
     }
     __syncthreads();
 
-    const int wave = tid >> 6, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
     const lds_f16* w1l = (const lds_f16*)w1s + l32 * kPitch + 8 * hh;
     const lds_f16* w2l = (const lds_f16*)w2s + l32 * kPitch + 8 * hh;
-    for (int64_t tile = (int64_t)blockIdx.x * kWaves + wave; tile < ntiles; tile += (int64_t)gridDim.x * kWaves) {
-        const int h = (int)(tile % heads);
-        const int64_t r = (tile / heads) * 32 + l32;  // this lane's row
-        const bool live = r < rows;
-        const uint16_t* qr = q + (live ? r : rows - 1) * qs + (int64_t)h * d;
-
-        // the lane's query elements: step s, half e holds q[16 s + 4 hh + 8 e + 0..3] (zeros
-        // past d; the address clamped inside the row)
-        u32x2_t qw[KS1][2];
+    // the lane's query elements of a tile: step s, half e holds q[16 s + 4 hh + 8 e + 0..3] (zeros
+    // past d; the address clamped inside the row)
+    auto load_q = [&](int64_t tile, u32x2_t (&qw)[KS1][2]) {
+        const int64_t block = tile / heads, r = block * 32 + l32;
+        const uint16_t* qr = q + min(r, rows - 1) * qs + (tile - block * heads) * d;
 #pragma unroll
         for (int s = 0; s < KS1; ++s)
 #pragma unroll
@@ -99,38 +154,48 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
                 const u32x2_t v = *reinterpret_cast<const u32x2_t*>(qr + min(c, d - 4));
                 qw[s][e] = c < d ? v : u32x2_t{0u, 0u};
             }
+    };
+    int64_t tile = (int64_t)blockIdx.x * kWaves + wave;
+    const int64_t step = (int64_t)gridDim.x * kWaves;
+    u32x2_t qw[KS1][2];
+    if (tile < ntiles) load_q(tile, qw);
+    for (; tile < ntiles; tile += step) {
+        const int64_t block = tile / heads;
+        const int h = (int)(tile - block * heads);
+        const int64_t r = block * 32 + l32;  // this lane's row
+        const bool live = r < rows;
+        u32x2_t qn[KS1][2];  // the next tile's (the last loads its own again, unused)
+        load_q(tile + step < ntiles ? tile + step : tile, qn);
 
         // H^T = W1 Q^T: acc1[t][4 g + i] is hidden unit 32 t + 8 g + 4 hh + i of row l32
         f32x16 acc1[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            acc1[t] = f32x16{};
+            acc1[t] = bias_tile(b1s + 32 * t + 4 * hh);
 #pragma unroll
             for (int s = 0; s < KS1; ++s) {
                 const f16x8 a = *reinterpret_cast<const lds_f16x8*>(w1l + 32 * t * kPitch + 16 * s);
                 acc1[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, join(qw[s][0], qw[s][1]), acc1[t], 0, 0, 0);
             }
         }
-        // bias, GELU, fp16: hw[t][g] holds hidden units 32 t + 8 g + 4 hh + 0..3
+        // fp16, GELU, fp16: hw[t][g] holds hidden units 32 t + 8 g + 4 hh + 0..3
         u32x2_t hw[2][4];
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 bb = *reinterpret_cast<const f32x4*>(&b1s[32 * t + 8 * g + 4 * hh]);
-                float y[4];
+            for (int g = 0; g < 4; ++g)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) y[i] = gelu16(r16(acc1[t][4 * g + i] + bb[i]));
-                hw[t][g] = u32x2_t{(uint32_t)f32_to_f16(y[0]) | ((uint32_t)f32_to_f16(y[1]) << 16),
-                                   (uint32_t)f32_to_f16(y[2]) | ((uint32_t)f32_to_f16(y[3]) << 16)};
-            }
+                for (int i = 0; i < 2; ++i) {
+                    const f16x2 x = pair16(acc1[t][4 * g + 2 * i], acc1[t][4 * g + 2 * i + 1]);
+                    hw[t][g][i] = __builtin_bit_cast(uint32_t, pair16(gelu((float)x[0]), gelu((float)x[1])));
+                }
 
         // G^T = W2 H^T: step s of the hidden units takes hw[s / 2][2 (s % 2) + 0..1] as its B
         // operand; acc2[t][4 g + i] is output 32 t + 8 g + 4 hh + i of row l32
         f32x16 acc2[NT2];
 #pragma unroll
         for (int t = 0; t < NT2; ++t) {
-            acc2[t] = f32x16{};
+            acc2[t] = bias_tile(b2s + 32 * t + 4 * hh);
 #pragma unroll
             for (int s = 0; s < kHid / 16; ++s) {
                 const f16x8 a = *reinterpret_cast<const lds_f16x8*>(w2l + 32 * t * kPitch + 16 * s);
@@ -139,29 +204,32 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
             }
         }
 
-        // out = (q * base_scale) * (1 + tanh(g + b2)); output o = 32 t + 8 g + 4 hh + i uses
-        // the query element in qw[2 t + g / 2][g % 2], lane slot i
-        if (live) {
-            uint16_t* orow = out + r * os + (int64_t)h * d;
-            const uint16_t* bsr = bs + (int64_t)h * d;
+        // out = (q * base_scale) * (1 + tanh(g + b2)); output o = 32 t + 8 g + 4 hh + i uses the
+        // query element in qw[2 t + g / 2][g % 2], lane slot i. The products and the sum of fp16
+        // values are packed fp16: each is rounded once from the exact value, as from fp32.
+        const uint16_t* bsr = bs + (int64_t)h * d;
+        uint16_t* orow = out + r * os + (int64_t)h * d;
 #pragma unroll
-            for (int t = 0; t < NT2; ++t)
+        for (int t = 0; t < NT2; ++t)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int o = 32 * t + 8 * g + 4 * hh;
-                    if (o >= d) continue;
-                    const u32x2_t qv = qw[2 * t + (g >> 1)][g & 1];
-                    const u32x2_t sv = *reinterpret_cast<const u32x2_t*>(bsr + o);
-                    const f32x4 bb = *reinterpret_cast<const f32x4*>(&b2s[o]);
-                    uint32_t ob[4];
+            for (int g = 0; g < 4; ++g) {
+                if (2 * t + (g >> 1) >= KS1) continue;  // past every head width of this kernel
+                const int o = 32 * t + 8 * g + 4 * hh;
+                const u32x2_t qv = qw[2 * t + (g >> 1)][g & 1];
+                const u32x2_t sv = *reinterpret_cast<const u32x2_t*>(bsr + min(o, d - 4));
+                u32x2_t ob;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float gs = r16(1.0f + r16(tanhf(r16(acc2[t][4 * g + i] + bb[i]))));
-                        ob[i] = f32_to_f16(r16(half_at(qv, i) * half_at(sv, i)) * gs);
-                    }
-                    *reinterpret_cast<u32x2_t*>(orow + o) = u32x2_t{ob[0] | (ob[1] << 16), ob[2] | (ob[3] << 16)};
+                for (int i = 0; i < 2; ++i) {
+                    const f16x2 v = pair16(acc2[t][4 * g + 2 * i], acc2[t][4 * g + 2 * i + 1]);
+                    const f16x2 gs = pair16(tanh_f32((float)v[0]), tanh_f32((float)v[1])) + f16x2{(_Float16)1.0f, (_Float16)1.0f};
+                    ob[i] = __builtin_bit_cast(uint32_t, (pair_at(qv, i) * pair_at(sv, i)) * gs);
                 }
-        }
+                if (live && o < d) *reinterpret_cast<u32x2_t*>(orow + o) = ob;
+            }
+#pragma unroll
+        for (int s = 0; s < KS1; ++s)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) qw[s][e] = qn[s][e];
     }
 }
 
@@ -175,7 +243,7 @@ qass_base_kernel(float log_n, const uint16_t* w1, const uint16_t* b1, const uint
     __shared__ float hid[kHid];
     const int tid = threadIdx.x;
     const float l = r16(log_n);
-    hid[tid] = gelu16(r16(f16_to_f32(w1[tid]) * l + f16_to_f32(b1[tid])));
+    hid[tid] = r16(gelu(r16(f16_to_f32(w1[tid]) * l + f16_to_f32(b1[tid]))));
     __syncthreads();
     const int o = blockIdx.x * 64 + tid;
     if (o >= n_out) return;
@@ -189,16 +257,18 @@ qass_base_kernel(float log_n, const uint16_t* w1, const uint16_t* b1, const uint
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc = fmaf(f16_to_f32((uint16_t)(w[c][i >> 1] >> (16 * (i & 1)))), hid[8 * c + i], acc);
     const float delta = r16(acc + f16_to_f32(b2[o]));
-    out[o] = f32_to_f16(l * r16(1.0f + r16(tanhf(delta))));
+    out[o] = f32_to_f16(l * r16(1.0f + r16(tanh_f32(delta))));
 }
 
 template <int KS1, int NT2>
 void launch(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, const uint16_t* w1, const uint16_t* b1,
             const uint16_t* w2, const uint16_t* b2, const uint16_t* bs, uint16_t* out, int64_t os, hipStream_t stream) {
     const int64_t ntiles = (rows + 31) / 32 * heads;
-    const int64_t grid = std::min<int64_t>((ntiles + kWaves - 1) / kWaves, 16384);
+    // resident workgroups (four a CU): each stages the weights once and walks tiles
+    const int64_t grid = std::min<int64_t>((ntiles + kWaves - 1) / kWaves, (int64_t)device_cus() * 4);
     hipLaunchKernelGGL((qass_gate_kernel<KS1, NT2>), dim3((unsigned)grid), dim3(64 * kWaves), 0, stream, q, rows,
-                       heads, d, qs, w1, b1, w2, b2, bs, out, os, ntiles);
+                       heads, d, qs, w1, b1, w2, b2, bs, out, os, ntiles,
+                       (int)((uintptr_t)w1 % 8 == 0 && (uintptr_t)w2 % 8 == 0));
 }
 
 }  // namespace
