@@ -1,12 +1,12 @@
 // One dense layer over query rows against its context cache (EncoderBaseLayer.forward_test_with_cache,
-// src/synthefy_nori/model/layer.py:1915-1967, layer_arch "smf"), its eleven launches issued by one call.
+// src/synthefy_nori/model/layer.py:1915-1967, layer_arch "smf"), its nine launches issued by one call.
 //
 // For small tables a layer's kernels take a few microseconds each and the Python between them two to
 // three times that: the 6m stack over 256 x 9 query tokens spent 4.9 ms of host time on 1.4 ms of
 // kernels. The kernels are the ones the module issues one by one -- row norm, q projection, QASS base
-// and gate, cached attention, output projection, residual + norm, SwiGLU with residual + norm, q|k|v
-// projection, feature attention, output projection, residual -- with the projections on
-// nori_linear_f16 at every row count.
+// and gate, cached attention, SwiGLU, q|k|v projection, feature attention -- with the projections on
+// nori_linear_f16 at every row count and the residual updates and norms inside the output
+// projections and the SwiGLU kernel.
 #include "nori_common.h"
 
 namespace {
@@ -61,21 +61,19 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
     NORI_STEP(nori_icl_attention(a0, NORI_F16, B * G, R, h, d, R * e, e, d, p->kv, p->kv_dtype, p->kv_scales, p->nk,
                                  p->kv_heads, p->kv_bg, p->kv_row, p->kv_half, p->sc_bg, p->sc_row, p->sc_half, scale, a1,
                                  NORI_F16, R * e, e, d, nullptr, 0, ws, ws_bytes, stream));
-    NORI_STEP(nori_linear_f16(a1, 1, 1, n, e, 0, 0, e, p->w_out, e, e, a0, 0, 0, e, stream));
     // x + alpha u into the new stream, then the MLP with its residual, each with the next norm
-    const int64_t u_rows[5] = {R, G, R * G * e, e, R * (int64_t)e};
-    NORI_STEP(nori_residual_add_rms_norm(p->x, a0, NORI_F16, u_rows, p->alpha, n, e, p->eps_mlp, p->out, a1, NORI_F16, n,
-                                         0, e, stream));
-    NORI_STEP(nori_swiglu_mlp_residual_rms_norm(a1, NORI_F16, n, e, e, p->gate_up, p->down, p->hidden, p->alpha, p->out, e,
-                                                e, p->eps_feat, a0, n, 0, e, stream));
+    NORI_STEP(nori_linear_f16_residual(a1, B, R, G, e, R * G * e, e, R * (int64_t)e, p->w_out, e, p->alpha, p->x, R * G * e,
+                                       G * (int64_t)e, e, p->out, p->eps_mlp, a0, R * G * e, G * (int64_t)e, e, stream));
+    NORI_STEP(nori_swiglu_mlp_residual_rms_norm(a0, NORI_F16, n, e, e, p->gate_up, p->down, p->hidden, p->alpha, p->out, e,
+                                                e, p->eps_feat, a1, n, 0, e, stream));
     // feature attention over each row's groups
-    NORI_STEP(nori_linear_f16(a0, 1, 1, n, e, 0, 0, e, p->w_qkv, e, 3 * e, qkv, 0, 0, 3 * e, stream));
+    NORI_STEP(nori_linear_f16(a1, 1, 1, n, e, 0, 0, e, p->w_qkv, e, 3 * e, qkv, 0, 0, 3 * e, stream));
     const uint16_t* q3 = reinterpret_cast<const uint16_t*>(qkv);
     NORI_STEP(nori_icl_attention(q3, NORI_F16, B * R, G, h, d, 3 * G * e, 3 * e, d, q3 + e, NORI_F16, nullptr, G, h,
                                  3 * G * e, 3 * e, e, 0, 0, 0, scale, a0, NORI_F16, G * e, e, d, nullptr, 0, ws, ws_bytes,
                                  stream));
-    NORI_STEP(nori_linear_f16(a0, 1, 1, n, e, 0, 0, e, p->w_feat_out, e, e, a1, 0, 0, e, stream));
-    NORI_STEP(nori_residual_add(p->out, a1, NORI_F16, p->alpha, n * e, p->out, stream));
+    NORI_STEP(nori_linear_f16_residual(a0, 1, 1, n, e, 0, 0, e, p->w_feat_out, e, p->alpha, p->out, 0, 0, e, p->out, 0.f,
+                                       nullptr, 0, 0, 0, stream));
 #undef NORI_STEP
     return NORI_OK;
 }

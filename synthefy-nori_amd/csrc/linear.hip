@@ -259,8 +259,10 @@ int launch(LinArgs a, hipStream_t stream) {
 struct ResArgs {
     const _Float16* a; int64_t rows, n_mid, n_inner, a_outer, a_mid, a_row;
     const _Float16* w; int64_t w_row;
-    float* x; int64_t x_outer, x_mid, x_row;
-    _Float16* y; int64_t y_outer, y_mid, y_row;
+    const float* x; int64_t x_outer, x_mid, x_row;
+    float* xo;    // the updated stream, at x's strides (may be x)
+    _Float16* y;  // null: no norm
+    int64_t y_outer, y_mid, y_row;
     float alpha, eps;
     int64_t nblocks;
 };
@@ -363,9 +365,10 @@ __global__ void __launch_bounds__(WAVES * 64, KS == 4 ? 4 : 2) linear_residual_n
                 }
                 part[p][q] = pp;
                 const int64_t xop = __shfl(xo, rr) + c4 + 64 * q;
-                if (row0 + rr < a.rows) *reinterpret_cast<f32x4*>(a.x + xop) = v[p][q];
+                if (row0 + rr < a.rows) *reinterpret_cast<f32x4*>(a.xo + xop) = v[p][q];
             }
         }
+        if (a.y) {  // uniform over the launch
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
             // pairs over the chunk index bits from the highest: q's in the lane, then l % 16's
@@ -390,6 +393,7 @@ __global__ void __launch_bounds__(WAVES * 64, KS == 4 ? 4 : 2) linear_residual_n
                         uint2{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16)};
                 }
             }
+        }
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) xf[ks] = xn[ks];
@@ -491,12 +495,12 @@ extern "C" int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t
 }
 
 
-extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner,
-                                                 int32_t k, int64_t a_outer_stride, int64_t a_mid_stride,
-                                                 int64_t a_row_stride, const void* weight, int64_t w_row_stride,
-                                                 float alpha, float* x, int64_t x_outer_stride, int64_t x_mid_stride,
-                                                 int64_t x_row_stride, float eps, void* y, int64_t y_outer_stride,
-                                                 int64_t y_mid_stride, int64_t y_row_stride, void* stream) {
+namespace {
+
+int run_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k, int64_t a_outer_stride,
+                 int64_t a_mid_stride, int64_t a_row_stride, const void* weight, int64_t w_row_stride, float alpha,
+                 const float* x, int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, float* x_out,
+                 float eps, void* y, int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, void* stream) {
     clear_error();
     if (n_outer < 0 || n_mid < 0 || n_inner < 0 || k <= 0)
         return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: bad shape n_outer=%lld n_mid=%lld n_inner=%lld k=%d",
@@ -507,10 +511,10 @@ extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer,
     if (n_inner > INT64_MAX / n_mid || n_mid * n_inner > INT64_MAX / n_outer)
         return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: %lld x %lld x %lld rows overflow",
                     (long long)n_outer, (long long)n_mid, (long long)n_inner);
-    if (!a || !weight || !x || !y) return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: null pointer");
+    if (!a || !weight || !x || !x_out) return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: null pointer");
     // 16-byte operand and weight chunks, 16-byte pieces of x, 8-byte pieces of y
     if ((uintptr_t)a % 16 || a_row_stride % 8 || a_mid_stride % 8 || a_outer_stride % 8 || (uintptr_t)weight % 16 ||
-        w_row_stride % 8 || w_row_stride < k || (uintptr_t)x % 16 || x_row_stride % 4 || x_mid_stride % 4 ||
+        w_row_stride % 8 || w_row_stride < k || (uintptr_t)x % 16 || (uintptr_t)x_out % 16 || x_row_stride % 4 || x_mid_stride % 4 ||
         x_outer_stride % 4 || (uintptr_t)y % 8 || y_row_stride % 4 || y_mid_stride % 4 || y_outer_stride % 4)
         return fail(NORI_ERR_UNSUPPORTED, "linear_f16_residual_rms_norm: operand and weight rows must be 16-byte "
                     "aligned, stream rows 16-byte aligned, output rows 8-byte aligned");
@@ -525,6 +529,7 @@ extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer,
     r.w = reinterpret_cast<const _Float16*>(weight);
     r.w_row = w_row_stride;
     r.x = x;
+    r.xo = x_out;
     r.x_outer = x_outer_stride;
     r.x_mid = x_mid_stride;
     r.x_row = x_row_stride;
@@ -536,4 +541,32 @@ extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer,
     r.eps = eps;
     hipStream_t s = (hipStream_t)stream;
     return k == 128 ? launch_residual<4, 8>(r, s) : launch_residual<8, 8>(r, s);
+}
+
+}  // namespace
+
+extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner,
+                                                 int32_t k, int64_t a_outer_stride, int64_t a_mid_stride,
+                                                 int64_t a_row_stride, const void* weight, int64_t w_row_stride,
+                                                 float alpha, float* x, int64_t x_outer_stride, int64_t x_mid_stride,
+                                                 int64_t x_row_stride, float eps, void* y, int64_t y_outer_stride,
+                                                 int64_t y_mid_stride, int64_t y_row_stride, void* stream) {
+    if (!y && n_outer > 0 && n_mid > 0 && n_inner > 0 && (k == 128 || k == 256)) {
+        clear_error();
+        return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: null pointer");
+    }
+    return run_residual(a, n_outer, n_mid, n_inner, k, a_outer_stride, a_mid_stride, a_row_stride, weight, w_row_stride,
+                        alpha, x, x_outer_stride, x_mid_stride, x_row_stride, x, eps, y, y_outer_stride, y_mid_stride,
+                        y_row_stride, stream);
+}
+
+extern "C" int nori_linear_f16_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
+                                        int64_t a_outer_stride, int64_t a_mid_stride, int64_t a_row_stride,
+                                        const void* weight, int64_t w_row_stride, float alpha, const float* x,
+                                        int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, float* x_out,
+                                        float eps, void* y, int64_t y_outer_stride, int64_t y_mid_stride,
+                                        int64_t y_row_stride, void* stream) {
+    return run_residual(a, n_outer, n_mid, n_inner, k, a_outer_stride, a_mid_stride, a_row_stride, weight, w_row_stride,
+                        alpha, x, x_outer_stride, x_mid_stride, x_row_stride, x_out, eps, y, y_outer_stride, y_mid_stride,
+                        y_row_stride, stream);
 }

@@ -34,6 +34,19 @@ int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t n_mid, int
                               int64_t y_row_stride, const void* gain, int gain_dtype, float eps, int32_t norm_cols,
                               void* stream);
 
+// nori_linear_f16_residual_rms_norm with the updated stream written to x_out, at x's strides (x_out may
+// be x), and with y NULL without the norm.
+int nori_linear_f16_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
+                             int64_t a_outer_stride, int64_t a_mid_stride, int64_t a_row_stride, const void* weight,
+                             int64_t w_row_stride, float alpha, const float* x, int64_t x_outer_stride,
+                             int64_t x_mid_stride, int64_t x_row_stride, float* x_out, float eps, void* y,
+                             int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, void* stream);
+
+// nori_swiglu_mlp_residual_rms_norm without the norm (fp16 x, width 128 or 256).
+int nori_swiglu_mlp_residual(const void* x, int64_t rows, int32_t width, int64_t x_row_stride, const void* w_gate_up,
+                             const void* w_down, int32_t hidden, float alpha, float* stream_rows,
+                             int64_t stream_row_stride, void* stream);
+
 // One dense "smf" layer over query rows against its context cache, every launch from one call
 // (dense_layer.hip): x [tables, rows, groups, embed] fp32 contiguous is left as it is, out (the same
 // shape) takes the layer's output. Weights fp16, contiguous, as the module keeps them: w_q, w_out,

@@ -149,6 +149,7 @@ __device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r
                     if (ok) *reinterpret_cast<f32x4*>(xr + 64 * q) = v[p][q];
                 }
             }
+            if (y) {  // uniform over the launch (null: no norm)
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 const int64_t row = rh + 4 * p + (lane >> 4);
@@ -181,6 +182,7 @@ __device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r
                         }
                     }
                 }
+            }
             }
         }
         asm volatile("" ::: "memory");
@@ -415,4 +417,30 @@ extern "C" int nori_swiglu_mlp_residual_rms_norm(const void* x, int dtype, int64
     else if (norm_width == 128) launch<256, 128>(xp, rows, x_row_stride, gp, dp, hidden, yp, 0, stream, ep);
     else launch<256, 256>(xp, rows, x_row_stride, gp, dp, hidden, yp, 0, stream, ep);
     return launch_status("swiglu_mlp_residual_rms_norm");
+}
+
+extern "C" int nori_swiglu_mlp_residual(const void* x, int64_t rows, int32_t width, int64_t x_row_stride,
+                                        const void* w_gate_up, const void* w_down, int32_t hidden, float alpha,
+                                        float* stream_rows, int64_t stream_row_stride, void* stream_v) {
+    clear_error();
+    if (width != 128 && width != 256)
+        return fail(NORI_ERR_UNSUPPORTED, "swiglu_mlp_residual: width %d is not 128 or 256", width);
+    if (rows < 0 || rows > 0x7fffffffLL || hidden <= 0 || hidden % 32 != 0)
+        return fail(NORI_ERR_INVALID, "swiglu_mlp_residual: bad shape (%lld rows, hidden %d)", (long long)rows, hidden);
+    if (x_row_stride < width || x_row_stride % 8 || stream_row_stride < width || stream_row_stride % 4)
+        return fail(NORI_ERR_INVALID, "swiglu_mlp_residual: row strides must be multiples of 8 (x) or 4");
+    if (rows == 0) return NORI_OK;
+    if (!x || !w_gate_up || !w_down || !stream_rows) return fail(NORI_ERR_INVALID, "swiglu_mlp_residual: null pointer");
+    if ((uintptr_t)x % 16 || (uintptr_t)w_gate_up % 16 || (uintptr_t)w_down % 16 || (uintptr_t)stream_rows % 16)
+        return fail(NORI_ERR_INVALID, "swiglu_mlp_residual: x, the weights and the stream must be 16-byte aligned");
+    if ((int64_t)hidden * width > kMaxWeights)
+        return fail(NORI_ERR_UNSUPPORTED, "swiglu_mlp_residual: hidden width %d", hidden);
+    const ResEpi ep{stream_rows, stream_row_stride, alpha, 0.f, 1, 0, 0};
+    hipStream_t stream = (hipStream_t)stream_v;
+    auto xp = reinterpret_cast<const uint16_t*>(x);
+    auto gp = reinterpret_cast<const uint16_t*>(w_gate_up);
+    auto dp = reinterpret_cast<const uint16_t*>(w_down);
+    if (width == 128) launch<128, 128>(xp, rows, x_row_stride, gp, dp, hidden, nullptr, 0, stream, ep);
+    else launch<256, 256>(xp, rows, x_row_stride, gp, dp, hidden, nullptr, 0, stream, ep);
+    return launch_status("swiglu_mlp_residual");
 }

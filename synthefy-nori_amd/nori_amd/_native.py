@@ -136,6 +136,12 @@ OPS: dict[str, tuple[object, list]] = {
         ctypes.c_int,
         [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _i32, _vp, _i64, _i64, _i64, _vp, _i32, _f32, _i32, _vp],
     ),
+    "nori_linear_f16_residual": (
+        ctypes.c_int,
+        [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _f32, _vp, _i64, _i64, _i64, _vp, _f32, _vp, _i64, _i64,
+         _i64, _vp],
+    ),
+    "nori_swiglu_mlp_residual": (ctypes.c_int, [_vp, _i64, _i32, _i64, _vp, _vp, _i32, _f32, _vp, _i64, _vp]),
     "nori_dense_apply_scratch_bytes": (_i64, [_i64, _i64, _i64, _i32, _i32, _i64]),
     "nori_dense_apply": (ctypes.c_int, [ctypes.POINTER(DenseApplyArgs), _vp]),
     "nori_rms_norm_rows": (ctypes.c_int, [_vp, _i64, _i32, _i64, _i64, _i64, _i64, _i64, _f32, _vp, _i32, _vp]),

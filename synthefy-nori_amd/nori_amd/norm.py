@@ -430,6 +430,29 @@ def swiglu_mlp_residual_norm(x: torch.Tensor, gate_up: torch.Tensor, down: torch
     return out
 
 
+def swiglu_mlp_residual(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, hidden: int, stream: torch.Tensor,
+                        alpha: float) -> bool:
+    """``stream += alpha * swiglu_mlp(x, ...)`` in place in one kernel (``nori_swiglu_mlp_residual``),
+    bit for bit ``swiglu_mlp`` followed by ``residual_add``; whether the kernel took the operands
+    (``swiglu_mlp_residual_norm``'s without the norm)."""
+    width = int(x.shape[-1])
+    if not (x.is_cuda and x.dtype == torch.float16 and stream.dtype == torch.float32 and stream.is_contiguous()
+            and stream.device == x.device and stream.numel() == x.numel() and width in (128, 256)
+            and gate_up.shape == (2 * hidden, width) and down.shape == (width, hidden)):
+        return False
+    x2 = x.reshape(-1, width)
+    if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16 or stream.data_ptr() % 16:
+        return False
+    nat.check(
+        nat.lib().nori_swiglu_mlp_residual(
+            x2.data_ptr(), x2.shape[0], width, x2.stride(0), gate_up.contiguous().data_ptr(), down.contiguous().data_ptr(),
+            hidden, float(alpha), stream.data_ptr(), width, nat.stream_of(x.device),
+        ),
+        "swiglu_mlp_residual",
+    )
+    return True
+
+
 QASS_GATE_HIDDEN = 64
 
 

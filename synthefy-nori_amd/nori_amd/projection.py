@@ -20,7 +20,7 @@ import torch
 
 from . import _native as nat
 
-__all__ = ["linear", "linear_head_norm", "linear_residual_norm", "takes_kernel"]
+__all__ = ["linear", "linear_head_norm", "linear_residual", "linear_residual_norm", "takes_kernel"]
 
 _WIDTHS = (128,)  # inner widths routed to the kernel (it also takes 256, where the library GEMM was faster)
 _MAX_N = 256      # output widths up to this (past it the library GEMM was as fast or faster)
@@ -163,39 +163,57 @@ def linear_head_norm(x: torch.Tensor, weight: torch.Tensor, gain: torch.Tensor, 
 
 
 def linear_residual_norm(a: torch.Tensor, weight: torch.Tensor, stream: torch.Tensor, alpha: float, eps: float,
-                         out: torch.Tensor | None = None) -> torch.Tensor | None:
+                         out: torch.Tensor | None = None, dest: torch.Tensor | None = None) -> torch.Tensor | None:
     """``stream += alpha * F.linear(a, weight)`` in place, then the RMSNorm (no weight, ``eps``)
     of the updated stream rows in fp16, in one kernel (``nori_linear_f16_residual_rms_norm``):
     bit for bit ``linear`` followed by the fused residual + norm pass. ``a`` [..., K] fp16,
     ``weight`` [K, K] fp16 (K 128 or 256), ``stream`` [..., K] fp32 with ``a``'s leading shape
     (any row strides: e.g. the [table, row, group] cells beside an attention output in
     [table, group, row] order), ``out`` the same shape in fp16 (new and laid out like
-    ``stream`` when None). Returns the normalized rows, or None where the kernel does not take
-    the operands (nothing is then written)."""
+    ``stream`` when None). ``dest`` (``stream``'s shape and strides) takes the sum in ``stream``'s
+    place. Returns the normalized rows, or None where the kernel does not take the operands
+    (nothing is then written)."""
+    if out is None:
+        if a.shape != stream.shape:
+            return None
+        out = torch.empty_like(stream, dtype=torch.float16)
+    elif tuple(out.shape) != tuple(a.shape) or out.dtype != torch.float16 or out.stride(-1) != 1:
+        return None
+    return out if _linear_residual(a, weight, stream, alpha, eps, out, dest) else None
+
+
+def linear_residual(a: torch.Tensor, weight: torch.Tensor, stream: torch.Tensor, alpha: float,
+                    dest: torch.Tensor | None = None) -> bool:
+    """``linear_residual_norm`` without the norm; whether the kernel took the operands."""
+    return _linear_residual(a, weight, stream, alpha, 0.0, None, dest)
+
+
+def _linear_residual(a, weight, stream, alpha, eps, out, dest) -> bool:
     k = int(a.shape[-1])
     if not (a.is_cuda and a.dtype == torch.float16 and weight.dtype == torch.float16 and stream.dtype == torch.float32
             and k in (128, 256) and tuple(weight.shape) == (k, k) and tuple(stream.shape) == tuple(a.shape)
             and stream.device == a.device and weight.device == a.device):
-        return None
+        return False
     if a.stride(-1) != 1 or stream.stride(-1) != 1 or weight.stride(-1) != 1:
-        return None
-    if out is None:
-        out = torch.empty_like(stream, dtype=torch.float16)
-    elif tuple(out.shape) != tuple(a.shape) or out.dtype != torch.float16 or out.stride(-1) != 1:
-        return None
-    common = _common_grid(a, stream, out)
+        return False
+    if dest is None:
+        dest = stream
+    elif dest.shape != stream.shape or dest.stride() != stream.stride() or dest.dtype != stream.dtype \
+            or dest.device != stream.device:
+        return False
+    common = _common_grid(a, stream) if out is None else _common_grid(a, stream, out)
     if common is None:
-        return None
-    (no, nm, ni), sa, sx, sy = common
+        return False
+    (no, nm, ni), sa, sx = common[:3]
+    sy = (0, 0, 0) if out is None else common[3]
     if (a.data_ptr() % 16 or any(st % 8 for st in sa) or weight.data_ptr() % 16 or weight.stride(0) % 8
-            or stream.data_ptr() % 16 or any(st % 4 for st in sx) or out.data_ptr() % 8 or any(st % 4 for st in sy)):
-        return None
-    nat.check(
-        nat.lib().nori_linear_f16_residual_rms_norm(
-            ctypes.c_void_p(a.data_ptr()), no, nm, ni, k, *sa, ctypes.c_void_p(weight.data_ptr()), int(weight.stride(0)),
-            float(alpha), ctypes.c_void_p(stream.data_ptr()), *sx, float(eps), ctypes.c_void_p(out.data_ptr()), *sy,
-            nat.stream_of(a.device),
-        ),
-        "linear_f16_residual_rms_norm",
-    )
-    return out
+            or stream.data_ptr() % 16 or dest.data_ptr() % 16 or any(st % 4 for st in sx)
+            or (out is not None and (out.data_ptr() % 8 or any(st % 4 for st in sy)))):
+        return False
+    head = (a.data_ptr(), no, nm, ni, k, *sa, weight.data_ptr(), int(weight.stride(0)), float(alpha), stream.data_ptr(), *sx)
+    tail = (float(eps), nat.ptr(out), *sy, nat.stream_of(a.device))
+    if out is not None and dest is stream:
+        nat.check(nat.lib().nori_linear_f16_residual_rms_norm(*head, *tail), "linear_f16_residual_rms_norm")
+    else:
+        nat.check(nat.lib().nori_linear_f16_residual(*head, dest.data_ptr(), *tail), "linear_f16_residual")
+    return True

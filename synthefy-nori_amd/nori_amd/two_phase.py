@@ -34,9 +34,10 @@ import torch
 from torch import nn
 
 from .layer import MultiheadAttention, SwiGLUMLP
-from .norm import RMSNorm, operand_dtype, projection_operand, residual_add, residual_add_norm, swiglu_mlp_residual_norm
+from .norm import (RMSNorm, operand_dtype, projection_operand, residual_add, residual_add_norm, swiglu_mlp_residual,
+                   swiglu_mlp_residual_norm)
 from .projection import linear as proj_linear
-from .projection import linear_residual_norm, takes_kernel
+from .projection import linear_residual, linear_residual_norm, takes_kernel
 
 __all__ = [
     "CellLayer2P",
@@ -75,30 +76,41 @@ def _accumulate(stream: torch.Tensor, update: torch.Tensor, alpha: float, then: 
 
 
 def _linear_accumulate(a: torch.Tensor, weight: torch.Tensor, stream: torch.Tensor, alpha: float, then: RMSNorm | None,
-                       project, *, operand: bool = True, out: torch.Tensor | None = None) -> torch.Tensor | None:
+                       project, *, operand: bool = True, out: torch.Tensor | None = None,
+                       dest: torch.Tensor | None = None) -> torch.Tensor | None:
     """``_accumulate(stream, project(), alpha, then, ...)`` where ``project()`` is ``F.linear(a,
     weight)`` under fp16 autocast: ``a`` [..., K] with ``stream``'s leading shape (any row
-    strides), ``weight`` [K, K] in the projection dtype. When the next norm is formed in the
-    fp16 operand dtype, the projection, the residual update and the norm run as one kernel
-    (``linear_residual_norm``: u never reaches memory) wherever it takes the operands."""
-    if (then is not None and operand and a.is_cuda and then.weight is None
-            and tuple(then.normalized_shape) == (int(stream.shape[-1]),)
-            and operand_dtype(stream) == torch.float16 and weight.dtype == torch.float16):
-        y = linear_residual_norm(a, weight, stream, alpha, then.eps, out=out)
-        if y is not None:
-            return y
-    return _accumulate(stream, project(), alpha, then, operand=operand, out=out)
+    strides), ``weight`` [K, K] in the projection dtype. The projection, the residual update and
+    the next norm, when it is formed in the fp16 operand dtype, run as one kernel
+    (``linear_residual_norm``, ``linear_residual``: u never reaches memory) wherever it takes the
+    operands. ``dest`` (laid out like ``stream``) takes the sum, and ``stream`` is left as it is."""
+    if a.is_cuda and operand_dtype(stream) == torch.float16 and weight.dtype == torch.float16:
+        if then is None:
+            if linear_residual(a, weight, stream, alpha, dest):
+                return None
+        elif operand and then.weight is None and tuple(then.normalized_shape) == (int(stream.shape[-1]),):
+            y = linear_residual_norm(a, weight, stream, alpha, then.eps, out=out, dest=dest)
+            if y is not None:
+                return y
+    return _accumulate(_moved(stream, dest), project(), alpha, then, operand=operand, out=out)
+
+
+def _moved(stream: torch.Tensor, dest: torch.Tensor | None) -> torch.Tensor:
+    """``stream``, or its copy in ``dest``."""
+    return stream if dest is None else dest.copy_(stream)
 
 
 def _attend_accumulate(attn: MultiheadAttention, atten: torch.Tensor, stream: torch.Tensor, alpha: float,
-                       then: RMSNorm | None = None, *, operand: bool = True) -> torch.Tensor | None:
-    """``stream += alpha * attn.project_out(atten)`` (then the next norm, as ``_accumulate``):
-    ``atten`` the attention output [..., H, D] with ``stream``'s leading shape, any row strides."""
+                       then: RMSNorm | None = None, *, operand: bool = True,
+                       dest: torch.Tensor | None = None) -> torch.Tensor | None:
+    """``stream += alpha * attn.project_out(atten)`` (then the next norm, as ``_accumulate``; into
+    ``dest``, as ``_linear_accumulate``): ``atten`` the attention output [..., H, D] with ``stream``'s
+    leading shape, any row strides."""
     a = atten.reshape(*atten.shape[:-2], -1)
     w_o = attn._linear_weights(atten.device)[2] if atten.is_cuda else None
     if w_o is None:
-        return _accumulate(stream, attn.project_out(atten), alpha, then, operand=operand)
-    return _linear_accumulate(a, w_o, stream, alpha, then, lambda: attn.project_out(atten), operand=operand)
+        return _accumulate(_moved(stream, dest), attn.project_out(atten), alpha, then, operand=operand)
+    return _linear_accumulate(a, w_o, stream, alpha, then, lambda: attn.project_out(atten), operand=operand, dest=dest)
 
 
 def _mlp_accumulate(mlp: SwiGLUMLP, x: torch.Tensor, stream: torch.Tensor, alpha: float, then: RMSNorm | None,
@@ -107,6 +119,10 @@ def _mlp_accumulate(mlp: SwiGLUMLP, x: torch.Tensor, stream: torch.Tensor, alpha
     operand dtype, the fused SwiGLU kernel applies the residual update and the norm itself
     (``swiglu_mlp_residual_norm``: the MLP output never reaches memory) wherever it takes the
     operands. ``stream`` holds x's rows (its last axis the norm's width)."""
+    if then is None and x.is_cuda and mlp.fuses(x) and operand_dtype(stream) == torch.float16:
+        gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
+        if swiglu_mlp_residual(x.to(torch.float16), gate_up, down, hidden, stream, alpha):
+            return None
     if (then is not None and operand and x.is_cuda and then.weight is None and mlp.fuses(x)
             and tuple(then.normalized_shape) == (int(stream.shape[-1]),)
             and operand_dtype(stream) == torch.float16):
@@ -298,41 +314,45 @@ class CellLayer2P(nn.Module):
 
     def forward(self, cells: torch.Tensor, targets: torch.Tensor, eval_pos: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Out-of-place form: returns the updated (cells, targets); the inputs are left as they are."""
-        cells, targets = cells.clone(), targets.contiguous().clone()
-        cell_op = self.column_step(cells, eval_pos, then=True)
+        # the first update of each stream writes the new one, so neither is copied first
+        new_cells, targets = torch.empty_like(cells), targets.contiguous()
+        new_targets = torch.empty_like(targets)
+        cell_op = self.column_step(cells, eval_pos, then=True, dest=new_cells)
         rows = _row_vectors(targets)
-        row_op = self.target_row_step(rows, self.row_operand(rows), eval_pos, then=True)
-        self.row_local_steps(cells, targets, cell_op, row_op)
-        return cells, targets
+        row_op = self.target_row_step(rows, self.row_operand(rows), eval_pos, then=True, dest=_row_vectors(new_targets))
+        self.row_local_steps(new_cells, new_targets, cell_op, row_op)
+        return new_cells, new_targets
 
     # --- steps on the streams (in place). Each step may take its normalized input, and with
     # ``then`` returns the normalized input of the step after it from the same pass as its
     # residual update (so a stream is not read again for the next norm).
     def column_step(self, cells: torch.Tensor, eval_pos: int, normed: torch.Tensor | None = None,
-                    then: bool = False) -> torch.Tensor | None:
+                    then: bool = False, dest: torch.Tensor | None = None) -> torch.Tensor | None:
         """Each cell reads its column's context cells. Reads whole columns: a slice of the
         groups axis may be passed. ``normed``: the cells through ``cell_norms[0]``; ``then``:
-        return the cells through ``cell_norms[1]`` (the cell MLP's operand)."""
+        return the cells through ``cell_norms[1]`` (the cell MLP's operand). ``dest`` (laid out like
+        ``cells``) takes the updated cells."""
         if normed is None:
             normed = projection_operand(self.cell_norms[0], cells)
         atten = self.column_attention.attend(normed, eval_pos)
         del normed
         return _attend_accumulate(self.column_attention.sequence_attentions[0], atten, cells, self.deepnorm_alpha,
-                                  self.cell_norms[1] if then else None)
+                                  self.cell_norms[1] if then else None, dest=dest)
 
     def row_operand(self, rows: torch.Tensor) -> torch.Tensor:
         """The normalized row vectors the target-stream row attention reads, [batch, 1, n, width]."""
         return projection_operand(self.target_norms[0], rows).unsqueeze(1)
 
     def target_row_step(self, rows: torch.Tensor, normed: torch.Tensor, eval_pos: int | None = None,
-                        context: torch.Tensor | None = None, then: bool = False) -> torch.Tensor | None:
+                        context: torch.Tensor | None = None, then: bool = False,
+                        dest: torch.Tensor | None = None) -> torch.Tensor | None:
         """The row vectors ``rows`` [batch, n, width] (normalized: ``normed``) read the context
         rows' normalized vectors: ``context``, or the first ``eval_pos`` of ``normed``. ``then``:
         return the rows through ``target_norms[1]`` (the target MLP's operand)."""
         keys = normed[:, :, :eval_pos] if context is None else context
         attn = self.sequence_attentions[0]
         atten = attn.attend(normed, keys).view(*rows.shape[:-1], attn.num_heads, attn.head_dim)
-        return _attend_accumulate(attn, atten, rows, self.deepnorm_alpha, self.target_norms[1] if then else None)
+        return _attend_accumulate(attn, atten, rows, self.deepnorm_alpha, self.target_norms[1] if then else None, dest=dest)
 
     def row_local_steps(self, cells: torch.Tensor, targets: torch.Tensor, cell_operand: torch.Tensor | None = None,
                         row_operand: torch.Tensor | None = None,
@@ -385,23 +405,24 @@ class RowLayer2P(nn.Module):
 
     def forward(self, rows: torch.Tensor, eval_pos: int, cell_memory: torch.Tensor) -> torch.Tensor:
         """Out-of-place form: returns the updated rows; ``rows`` is left as it is."""
-        rows = rows.clone()
-        query = self.context_step(rows, self.row_operand(rows), eval_pos, then=True)
-        self.readback_steps(rows, cell_memory, query)
-        return rows
+        new_rows = torch.empty_like(rows)
+        query = self.context_step(rows, self.row_operand(rows), eval_pos, then=True, dest=new_rows)
+        self.readback_steps(new_rows, cell_memory, query)
+        return new_rows
 
     def row_operand(self, rows: torch.Tensor) -> torch.Tensor:
         return projection_operand(self.attn_norm, rows).unsqueeze(1)
 
     def context_step(self, rows: torch.Tensor, normed: torch.Tensor, eval_pos: int | None = None,
-                     context: torch.Tensor | None = None, then: bool = False) -> torch.Tensor | None:
+                     context: torch.Tensor | None = None, then: bool = False,
+                     dest: torch.Tensor | None = None) -> torch.Tensor | None:
         """``rows`` [batch, n, width] (normalized: ``normed``) read the context rows' normalized
         vectors: ``context``, or the first ``eval_pos`` of ``normed``. ``then``: return the rows
         through ``readback_norm`` (the read-back query)."""
         keys = normed[:, :, :eval_pos] if context is None else context
         attn = self.sequence_attentions[0]
         atten = attn.attend(normed, keys).view(*rows.shape[:-1], attn.num_heads, attn.head_dim)
-        return _attend_accumulate(attn, atten, rows, self.deepnorm_alpha, self.readback_norm if then else None)
+        return _attend_accumulate(attn, atten, rows, self.deepnorm_alpha, self.readback_norm if then else None, dest=dest)
 
     def readback_steps(self, rows: torch.Tensor, cell_memory: torch.Tensor, query: torch.Tensor | None = None,
                        then: RMSNorm | None = None, operand: bool = True) -> torch.Tensor | None:

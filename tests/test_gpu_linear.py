@@ -294,3 +294,26 @@ def test_head_norm_against_the_separate_passes(cuda, k, rows, n, norm_cols, gain
     strided = torch.zeros(3, rows, k + 8, dtype=torch.float16, device=cuda)
     strided[1, :, :k] = x
     assert torch.equal(projection.linear_head_norm(strided[1:2, :, :k], w, gain, 1e-6, norm_cols)[0], got)
+
+
+@pytest.mark.parametrize("k", [128, 256])
+@pytest.mark.parametrize("rows", [1, 129, 5001])
+def test_residual_into_another_stream_and_without_the_norm(cuda, k, rows):
+    # nori_linear_f16_residual: bit for bit the in-place kernel, the source left as it is, nothing
+    # past the last row written; without the norm the same sums
+    g = torch.Generator(device=cuda).manual_seed(rows + k)
+    a = torch.randn(rows, k, generator=g, device=cuda).to(torch.float16)
+    w = (torch.randn(k, k, generator=g, device=cuda) / k ** 0.5).to(torch.float16)
+    x = torch.randn(rows, k, generator=g, device=cuda)
+    want = x.clone()
+    y_ref = projection.linear_residual_norm(a, w, want, ALPHA, 1e-5)
+    buf = torch.full((rows + 2, k), 7.0, device=cuda)
+    before = x.clone()
+    y = projection.linear_residual_norm(a, w, x, ALPHA, 1e-5, dest=buf[1:-1])
+    assert torch.equal(y, y_ref) and torch.equal(buf[1:-1], want) and torch.equal(x, before)
+    buf[1:-1] = 0.0
+    assert projection.linear_residual(a, w, x, ALPHA, buf[1:-1])
+    assert torch.equal(buf[1:-1], want) and torch.equal(x, before)
+    assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
+    assert projection.linear_residual(a, w, x, ALPHA) and torch.equal(x, want)
+    assert not projection.linear_residual(a, w, x, ALPHA, torch.empty(rows, k + 8, device=cuda)[:, :k])  # other strides

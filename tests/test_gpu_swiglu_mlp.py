@@ -216,3 +216,20 @@ def test_residual_norm_epilogue_declines_what_it_does_not_take():
     x = torch.randn(64, 128, device=DEV).half()
     assert swiglu_mlp_residual_norm(x, gate_up, down, hp, torch.randn(64, 128, device=DEV).half(), ALPHA, 1e-5,
                                     128) is None  # fp16 stream
+
+
+@pytest.mark.parametrize("width,hidden", [(128, 256), (256, 682)])
+@pytest.mark.parametrize("rows", [1, 31, 97, 128, 4133])
+def test_residual_without_a_norm_equals_the_separate_passes(width, hidden, rows):
+    # row counts that leave whole wavefronts of the last workgroup without rows; nothing past the
+    # stream is written
+    from nori_amd.norm import residual_add, swiglu_mlp_residual
+
+    gate_up, down, hp = _weights(width, hidden, seed=rows)
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, width, generator=g).half().to(DEV)
+    buf = torch.randn(rows + 1, width, generator=g).to(DEV)
+    stream, guard = buf[:rows], buf[rows].clone()
+    want = residual_add(stream, swiglu_mlp(x, gate_up, down, hp), 0.2)
+    assert swiglu_mlp_residual(x, gate_up, down, hp, stream, 0.2)
+    assert torch.equal(stream, want) and torch.equal(buf[rows], guard)
