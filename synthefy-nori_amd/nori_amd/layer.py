@@ -40,9 +40,10 @@ from . import _native as nat
 from . import kv_project
 from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
-from .projection import linear_head_norm
+from .projection import linear_head_norm, linear_residual, linear_residual_norm
 from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, group_major_operand, operand_dtype, projection_operand,
-                   qass_base, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp)
+                   qass_base, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp,
+                   swiglu_mlp_residual_norm)
 
 ACTIVATION_FN = {"gelu": nn.GELU(), "relu": nn.ReLU(), "silu": nn.SiLU()}
 _SDPA_BACKENDS_WITHOUT_CUDNN = [SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION, SDPBackend.MATH]
@@ -931,6 +932,49 @@ class EncoderBaseLayer(nn.Module):
             stream.copy_(residual_add(src, update, self._alpha_value(update)))
         return stream
 
+    def _fused_after_attention(self, x: torch.Tensor, seq: MultiheadAttention, atten: torch.Tensor) -> torch.Tensor | None:
+        """The rest of an "smf" pre-norm layer after its sequence attention, from the attention's
+        output [B * G, R, H, D] before its projection: each output projection and the MLP apply
+        their residual update and the next norm themselves (``linear_residual_norm``,
+        ``swiglu_mlp_residual_norm``), so no update reaches memory. x [B, R, G, E] is left as it
+        is; None where those kernels do not take the layer, with nothing written."""
+        feat, mlp, norms = self.feature_attentions[0], self.mlp[0], self.layer_norms
+        b, r, g, e = x.shape
+        if any(type(m) is not RMSNorm or m.weight is not None or tuple(m.normalized_shape) != (e,) for m in norms):
+            return None
+        if atten.dtype != torch.float16 or not x.is_contiguous() or not mlp.fuses(x) or feat.qk_norm or feat.use_qassmax:
+            return None
+        alpha = self._alpha_value(atten)
+        a = atten.view(b, g, r, e).transpose(1, 2)
+        stream = torch.empty_like(x)
+        operand = linear_residual_norm(a, seq._linear_weights(x.device)[2], x, alpha, norms[1].eps, dest=stream)
+        if operand is None:
+            return None
+        gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
+        tokens = swiglu_mlp_residual_norm(operand, gate_up, down, hidden, stream, alpha, norms[2].eps, e)
+        if tokens is None:
+            return None
+        del operand
+        w = feat._cast_weights(x.device)
+        qkv = proj_linear(tokens.view(b * r, g, e), w[4]).view(b * r, g, 3, feat.num_heads, feat.head_dim)
+        del tokens
+        out = icl_attention(feat._apply_extra_attn_scale(qkv[:, :, 0], g), qkv[:, :, 1:]).view(x.shape)
+        if not linear_residual(out, w[3], stream, alpha):
+            residual_add(stream, proj_linear(out, w[3]), alpha, inplace=True)
+        return stream
+
+    def _takes_fused_steps(self, x: torch.Tensor, seq: MultiheadAttention, feature_atten_mask) -> bool:
+        """Whether ``_fused_after_attention`` may stand for the modules' own calls: inference under
+        fp16 autocast on an fp32 stream, the plain modules, nothing watching their calls."""
+        return (
+            type(self) is EncoderBaseLayer and self.layer_arch == "smf" and self.pre_norm and feature_atten_mask is None
+            and x.is_cuda and x.dtype == torch.float32 and x.shape[-1] in (128, 256) and not torch.is_grad_enabled()
+            and operand_dtype(x) == torch.float16 and type(seq) is MultiheadAttention
+            and type(self.feature_attentions[0]) is MultiheadAttention and type(self.mlp[0]) is SwiGLUMLP
+            and self.feature_attentions[0]._attention_dropout_p() == 0.0
+            and not _hooked(seq, self.feature_attentions[0], self.mlp[0], *self.layer_norms)
+        )
+
     def _run_non_sequence_step(self, x, *, step_idx, feature_atten_mask, eval_pos):
         sublayer, norm = self.layer_steps[step_idx], self.layer_norms[step_idx]
         if self.pre_norm:
@@ -1182,9 +1226,16 @@ class EncoderBaseLayer(nn.Module):
         seq_norm = self.layer_norms[seq_step]
         x_train, src = self._pre_steps_then_operand(x_train, pre_steps, seq_norm, feature_atten_mask, eval_pos)
         residual = x_train
-        train_attn = seq_attn_train(
-            x=src.transpose(1, 2), x_kv=src.transpose(1, 2), copy_first_head_kv=self.self_share_all_kv_heads
-        )[0].transpose(1, 2)
+        fused_steps = not self.seq_attn_serial and self._takes_fused_steps(x_train, seq_attn_train, feature_atten_mask)
+        rows_t = src.transpose(1, 2)
+        atten = None
+        if fused_steps:
+            atten = seq_attn_train.attend(rows_t, rows_t, self.self_share_all_kv_heads)
+            train_attn = None
+        else:
+            train_attn = seq_attn_train(x=rows_t, x_kv=rows_t, copy_first_head_kv=self.self_share_all_kv_heads)[0]
+            train_attn = train_attn.transpose(1, 2)
+        del rows_t
         kv_source = (train_attn if self.seq_attn_serial else src).transpose(1, 2)
         fused = None
         if quantize_kv_cache and fused_cache_write:
@@ -1198,7 +1249,15 @@ class EncoderBaseLayer(nn.Module):
         else:
             seq_kv_cache = seq_attn_test.project_kv_cache(kv_source, copy_first_head_kv=self.cross_share_all_kv_heads)
         del kv_source
-        if self.pre_norm:
+        done = None
+        if fused_steps:
+            done = self._fused_after_attention(residual, seq_attn_train, atten)
+            if done is None:
+                out = seq_attn_train.project_out(atten)
+                train_attn = out.view(src.shape[0], src.shape[2], *out.shape[1:]).transpose(1, 2)
+        if done is not None:
+            x_train = done
+        elif self.pre_norm:
             x_train = self._add_then_steps(residual, train_attn, post_steps, feature_atten_mask, eval_pos)
         else:
             x_train = seq_norm(train_attn + residual)

@@ -5,10 +5,10 @@ reference's projections compute under the GPU's fp16 autocast, layer.py:651-683,
 fp32 sums of fp16 products, rounded once to fp16. ``nori_linear_f16`` (csrc/linear.hip) reads
 x and writes the output through strides -- a token subset of each row, a slice of a stacked
 output buffer (``out``), the transposed [table, group, row] view of a cell buffer -- without
-copies. ``linear`` routes to it the shapes where it is the faster of the two (same-box A/B
-against the library GEMM: inner width 128 and up to 256 output columns, e.g. 655,360 rows x
-128 -> 128 in 78 against 110 us; at inner width 256 or wider outputs the library GEMM was as
-fast or faster); everything else (other dtypes, widths or shapes, short operands, CPU
+copies. ``linear`` routes to it the shapes where it is the faster of the two (same-box A/B against the
+library GEMM at inner width 128: 139,264 rows x 128 -> 128 in 20 against 26 us, -> 256 in 25.5
+against 28, -> 384 in 32 against 59.5; 655,360 rows 67 against 101, 114 against 126, 157 against 261.
+At inner width 256 the library was level or faster up to 256 columns); everything else (other dtypes, widths or shapes, short operands, CPU
 tensors) is ``F.linear``. The two differ only in the order of the fp32 sums.
 """
 
@@ -23,7 +23,7 @@ from . import _native as nat
 __all__ = ["linear", "linear_head_norm", "linear_residual", "linear_residual_norm", "takes_kernel"]
 
 _WIDTHS = (128,)  # inner widths routed to the kernel (it also takes 256, where the library GEMM was faster)
-_MAX_N = 256      # output widths up to this (past it the library GEMM was as fast or faster)
+_MAX_N = 384      # output widths up to this
 _MIN_ROWS = 4096  # below this the library GEMM's launch is as cheap
 
 

@@ -77,3 +77,26 @@ def test_other_calls_keep_the_layers_own(cuda):
             assert taken()
             layer.train()
             assert not taken()
+
+
+@pytest.mark.parametrize("embed,heads", [(128, 2), (256, 4), (352, 8)])
+@pytest.mark.parametrize("tables,rows,groups", [(1, 40, 1), (1, 300, 9), (3, 701, 5)])
+def test_fused_build_equals_the_modules_calls(cuda, embed, heads, tables, rows, groups):
+    # the cache build's steps after its attention (residuals and norms inside the projections and the
+    # SwiGLU kernel) against the modules' own calls, which a forward hook keeps; the cache does not
+    # depend on them. Width 352 has no such kernels and takes the modules' calls both times.
+    layer = _layer(embed, heads, False, embed, cuda)
+    x = torch.randn(tables, rows, groups, embed, generator=torch.Generator().manual_seed(rows)).to(cuda)
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        before = x.clone()
+        fused = []
+        real = layer._fused_after_attention
+        layer._fused_after_attention = lambda *a: fused.append(real(*a)) or fused[-1]
+        got, cache = layer.forward_train_cache(x, quantize_kv_cache=True)
+        assert (len(fused) == 1 and fused[0] is not None) == (embed != 352)
+        handle = layer.mlp[0].register_forward_hook(lambda *a: None)
+        want, ref = layer.forward_train_cache(x, quantize_kv_cache=True)
+        handle.remove()
+        assert len(fused) <= 1 and torch.equal(x, before)
+    assert torch.equal(cache["seq_kv"]["kv"], ref["seq_kv"]["kv"])
+    assert float((got - want).double().norm() / (want - x).double().norm()) <= 4 * 2.0**-11
