@@ -85,73 +85,57 @@ struct ResEpi {
     int64_t y_group, y_group_stride, y_row_stride;
 };
 
-// The epilogue for a wavefront's 32 rows from r0, from its Y^T tiles (element 4j + i of tile t is
-// output 32t + 8j + 4hh + i of row l32). u = f16(y) goes through the wavefront's LDS slice, 16 rows
-// at a time, into a row layout: a stream row moves in 256-byte pieces (lane l takes rows 4p + l/16
-// at columns 64q + 4 (l % 16)) and an output row whole, where the MFMA layout touched 32 rows in
-// 32-byte pieces an instruction. The slice is the wavefront's own: LDS runs its accesses in order.
-template <int E, int NW>
-__device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r0, int64_t rows, int lane, _Float16* ut,
-                                           uint16_t* __restrict__ y, int64_t ys, const ResEpi& ep) {
-    constexpr int UP = E + 8, NCH = (E + 63) / 64;
-    const int l32 = lane & 31, hh = lane >> 5;
+// The epilogue's rows: PASSES * 4 rows from rh, their u = f16(y) in LDS at ut (rows E + 8 f16 apart),
+// written as y, or into the stream and its norm (NW > 0). A stream row moves in 256-byte pieces (lane
+// l takes rows 4p + l/16 at columns 64q + 4 (l % 16)) and an output row whole.
+template <int E, int NW, int PASSES>
+__device__ __forceinline__ void emit_rows(const _Float16* ut, int64_t rh, int64_t rows, int lane, uint16_t* __restrict__ y,
+                                          int64_t ys, const ResEpi& ep) {
+    constexpr int UP = E + 8, NCH = (E + 63) / 64, ROWS = 4 * PASSES;
+    if constexpr (NW == 0) {
+        constexpr int LPR = E / 8;  // 16-byte pieces per row
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        if ((l32 >> 4) == h) {
-            _Float16* ur = ut + (l32 & 15) * UP + 4 * hh;
-#pragma unroll
-            for (int t = 0; t < E / 32; ++t)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    *reinterpret_cast<u32x2*>(ur + 32 * t + 8 * j) =
-                        u32x2{pack_f16(yt[t][4 * j], yt[t][4 * j + 1]), pack_f16(yt[t][4 * j + 2], yt[t][4 * j + 3])};
+        for (int k = 0; k < (ROWS * LPR + 63) / 64; ++k) {
+            const int e = lane + 64 * k, rr = e / LPR, c = 8 * (e % LPR);
+            if (rr < ROWS && rh + rr < rows)
+                *reinterpret_cast<u32x4*>(y + (rh + rr) * ys + c) = *reinterpret_cast<const u32x4*>(ut + rr * UP + c);
         }
-        asm volatile("" ::: "memory");
-        const int64_t rh = r0 + 16 * h;
-        if constexpr (NW == 0) {
-            constexpr int LPR = E / 8;  // 16-byte pieces per row
+    } else {
+        static_assert(NW == 0 || (E % 64 == 0 && NW % 64 == 0), "norm groups of whole 64-column chunks");
+        constexpr int GC = NW > 0 ? NW / 64 : 1, GROUPS = NW > 0 ? E / NW : 1;
+        const int c4 = 4 * (lane & 15);
+        f32x4 v[PASSES][NCH];
+        float part[PASSES][NCH];
 #pragma unroll
-            for (int k = 0; k < (16 * LPR + 63) / 64; ++k) {
-                const int e = lane + 64 * k, rr = e / LPR, c = 8 * (e % LPR);
-                if (rr < 16 && rh + rr < rows)
-                    *reinterpret_cast<u32x4*>(y + (rh + rr) * ys + c) = *reinterpret_cast<const u32x4*>(ut + rr * UP + c);
-            }
-        } else {
-            static_assert(NW == 0 || (E % 64 == 0 && NW % 64 == 0), "norm groups of whole 64-column chunks");
-            constexpr int GC = NW > 0 ? NW / 64 : 1, GROUPS = NW > 0 ? E / NW : 1;
-            const int c4 = 4 * (lane & 15);
-            f32x4 v[4][NCH];
-            float part[4][NCH];
+        for (int p = 0; p < PASSES; ++p) {
+            const int rr = 4 * p + (lane >> 4);
+            // (rows past the last, a whole wavefront's in the last workgroup, read the last again)
+            const float* xr = ep.xs + (rh + rr < rows ? rh + rr : rows - 1) * ep.xs_row + c4;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const int rr = 4 * p + (lane >> 4);
-                // (rows past the last, a whole wavefront's in the last workgroup, read the last again)
-                const float* xr = ep.xs + (rh + rr < rows ? rh + rr : rows - 1) * ep.xs_row + c4;
+            for (int q = 0; q < NCH; ++q) v[p][q] = *reinterpret_cast<const f32x4*>(xr + 64 * q);
+        }
 #pragma unroll
-                for (int q = 0; q < NCH; ++q) v[p][q] = *reinterpret_cast<const f32x4*>(xr + 64 * q);
-            }
+        for (int p = 0; p < PASSES; ++p) {
+            const int rr = 4 * p + (lane >> 4);
+            const bool ok = rh + rr < rows;
+            float* xr = ep.xs + (ok ? rh + rr : rows - 1) * ep.xs_row + c4;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const int rr = 4 * p + (lane >> 4);
-                const bool ok = rh + rr < rows;
-                float* xr = ep.xs + (ok ? rh + rr : rows - 1) * ep.xs_row + c4;
+            for (int q = 0; q < NCH; ++q) {
+                const u32x2 uw = *reinterpret_cast<const u32x2*>(ut + rr * UP + 64 * q + c4);
+                float s = 0.f;
 #pragma unroll
-                for (int q = 0; q < NCH; ++q) {
-                    const u32x2 uw = *reinterpret_cast<const u32x2*>(ut + rr * UP + 64 * q + c4);
-                    float s = 0.f;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float u = f16_to_f32((uint16_t)(uw[e >> 1] >> (16 * (e & 1))));
-                        v[p][q][e] = v[p][q][e] + round_to<NORI_F16>(u * ep.alpha);
-                        s = fmaf(v[p][q][e], v[p][q][e], s);
-                    }
-                    part[p][q] = s;
-                    if (ok) *reinterpret_cast<f32x4*>(xr + 64 * q) = v[p][q];
+                for (int e = 0; e < 4; ++e) {
+                    const float u = f16_to_f32((uint16_t)(uw[e >> 1] >> (16 * (e & 1))));
+                    v[p][q][e] = v[p][q][e] + round_to<NORI_F16>(u * ep.alpha);
+                    s = fmaf(v[p][q][e], v[p][q][e], s);
                 }
+                part[p][q] = s;
+                if (ok) *reinterpret_cast<f32x4*>(xr + 64 * q) = v[p][q];
             }
-            if (y) {  // uniform over the launch (null: no norm)
+        }
+        if (y) {  // uniform over the launch (null: no norm)
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < PASSES; ++p) {
                 const int64_t row = rh + 4 * p + (lane >> 4);
 #pragma unroll
                 for (int k = 0; k < GROUPS; ++k) {
@@ -183,11 +167,43 @@ __device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r
                     }
                 }
             }
-            }
         }
+    }
+}
+
+// u = f16(y) of a lane's tile t (element 4j + i is output 32t + 8j + 4hh + i of its row) into its row at ur
+__device__ __forceinline__ void stage_tile(const f32x16& v, _Float16* ur) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<u32x2*>(ur + 8 * j) = u32x2{pack_f16(v[4 * j], v[4 * j + 1]), pack_f16(v[4 * j + 2], v[4 * j + 3])};
+}
+
+// The epilogue for a wavefront's 32 rows from r0, from its Y^T tiles. u goes through the wavefront's
+// LDS slice, 16 rows at a time, into a row layout, where the MFMA layout touched 32 rows in 32-byte
+// pieces an instruction. The slice is the wavefront's own: LDS runs its accesses in order.
+template <int E, int NW>
+__device__ __forceinline__ void write_rows(const f32x16 (&yt)[E / 32], int64_t r0, int64_t rows, int lane, _Float16* ut,
+                                           uint16_t* __restrict__ y, int64_t ys, const ResEpi& ep) {
+    const int l32 = lane & 31, hh = lane >> 5;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if ((l32 >> 4) == h) {
+#pragma unroll
+            for (int t = 0; t < E / 32; ++t) stage_tile(yt[t], ut + (l32 & 15) * (E + 8) + 4 * hh + 32 * t);
+        }
+        asm volatile("" ::: "memory");
+        emit_rows<E, NW, 4>(ut, r0 + 16 * h, rows, lane, y, ys, ep);
         asm volatile("" ::: "memory");
     }
 }
+
+// Few rows (SPLIT kernels, width 128): up to this many per CU, a workgroup owns 32 rows and its four
+// wavefronts take every fourth chunk each, from buffers of their own, so no barrier orders them; their
+// partial sums meet in LDS in the order of the wavefronts. With a whole workgroup to 128 rows, 2,304
+// rows are 18 workgroups, each one chain of 16 chunks: 17.1 us (hidden 256, with the residual epilogue)
+// against 13.6 us here, 13.2 against 10.0 us plain; 9,513 rows are past the line, at 19.6 us.
+constexpr int kSplitRowsPerCu = 32;
+constexpr int split_width(int e) { return e == 128; }
 
 // Operand reads in flight: each LDS read is issued kAhead reads before its MFMA and the order is
 // fenced; left to itself the compiler reads an operand just before its MFMA and waits.
@@ -213,30 +229,35 @@ struct MlpGeom {
     static constexpr int GLOADS = (2 * HC * GROW + 63) / 64;
     static constexpr int DLOADS = (3 * E + 63) / 64;
     static constexpr int LOADS = GLOADS + DLOADS;
-    static constexpr int PER = (LOADS + NWAVES - 1) / NWAVES;
     static constexpr int BUF = LOADS * 64 * 8;  // f16 per ring buffer
     static_assert(NWAVES * 16 * (E + 8) <= 2 * BUF, "the epilogue's rows fit the ring");
 };
 
-template <int E, int NW>
-__global__ void __launch_bounds__(MlpGeom<E>::THREADS) __attribute__((amdgpu_waves_per_eu(E <= 128 ? 3 : (E <= 256 ? 2 : 1))))
+template <int E, int NW, bool SPLIT>
+__global__ void __launch_bounds__(MlpGeom<E>::THREADS)
+__attribute__((amdgpu_waves_per_eu(SPLIT ? 1 : (E <= 128 ? 3 : (E <= 256 ? 2 : 1)))))
 swiglu_mlp_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t xs, const uint16_t* __restrict__ wgu,
                     const uint16_t* __restrict__ wd, int hp, uint16_t* __restrict__ y, int64_t ys, const ResEpi ep) {
     using G = MlpGeom<E>;
-    __shared__ __attribute__((aligned(16))) _Float16 ring[2 * G::BUF];
+    constexpr int SHARE = SPLIT ? 1 : G::NWAVES;  // wavefronts that stage and read a buffer together
+    constexpr int CSTEP = SPLIT ? G::NWAVES : 1;  // chunks from one of a wavefront's to its next
+    constexpr int PER = (G::LOADS + SHARE - 1) / SHARE;
+    __shared__ __attribute__((aligned(16))) _Float16 ring[(SPLIT ? G::NWAVES : 1) * 2 * G::BUF];
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5, l16 = lane & 15, g4 = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t r0 = (int64_t)blockIdx.x * (G::NWAVES * 32) + wave * 32;
-    const int nch = hp / G::HC;
+    const int64_t r0 = (int64_t)blockIdx.x * (SHARE * 32) + (SPLIT ? 0 : wave * 32);
+    const int nch = hp / G::HC, c0 = SPLIT ? wave : 0;
+    const int w0 = SPLIT ? 0 : wave;  // first of the wavefront's loads of a chunk
+    _Float16* const bufs = ring + (SPLIT ? wave * 2 * G::BUF : 0);
 
     // ---- staging: wavefront load i = wave, wave + NWAVES, ... of the chunk; padding granules load a
     // valid weight granule that nothing reads. Byte offsets of the lane's granules in chunk 0.
     const __amdgpu_buffer_rsrc_t rgu = __builtin_amdgcn_make_buffer_rsrc((void*)wgu, 0, 4 * hp * E, 0x00020000);
     const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void*)wd, 0, 2 * hp * E, 0x00020000);
-    uint32_t voff[G::PER];
+    uint32_t voff[PER];
 #pragma unroll
-    for (int k = 0; k < G::PER; ++k) {
-        const int i = wave + k * G::NWAVES;
+    for (int k = 0; k < PER; ++k) {
+        const int i = w0 + k * SHARE;
         if (i < G::GLOADS) {
             const int q = min(64 * i + lane, 2 * G::HC * G::GROW - 1);
             const int row = q / G::GROW, cp = min(q % G::GROW, E / 8 - 1);
@@ -248,15 +269,15 @@ swiglu_mlp_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t xs, cons
     }
     auto fetch = [&](int c, int b) {
 #pragma unroll
-        for (int k = 0; k < G::PER; ++k) {
-            const int i = wave + k * G::NWAVES;
+        for (int k = 0; k < PER; ++k) {
+            const int i = w0 + k * SHARE;
             if (i >= G::LOADS) break;  // uniform over the wavefront
-            lds_void* dst = (lds_void*)(ring + b * G::BUF + 512 * i);
+            lds_void* dst = (lds_void*)(bufs + b * G::BUF + 512 * i);
             if (i < G::GLOADS) buffer_to_lds(rgu, dst, voff[k], c * G::HC * E * 2);
             else buffer_to_lds(rd, dst, voff[k], c * G::HC * 2);
         }
     };
-    fetch(0, 0);
+    if (c0 < nch) fetch(c0, 0);
 
     // ---- X fragments (B operands): row tile t holds x[r0 + 16t + l16][32s + 8 g4 + 0..7]
     f16x8 xf[2][G::S];
@@ -275,14 +296,13 @@ swiglu_mlp_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t xs, cons
 #pragma unroll
     for (int t = 0; t < G::OT; ++t) yt[t] = f32x16{};
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    if constexpr (!SPLIT) __syncthreads();
 
     const int up_lane = 8 * (l16 * G::GROW + g4);                 // gate row l16 (up rows: HC further)
     const int dn_lane = 8 * (64 * G::GLOADS + 3 * l32 + hh);      // down row l32
-    for (int c = 0; c < nch; ++c) {
-        const int cur = c & 1;
-        if (c + 1 < nch) fetch(c + 1, cur ^ 1);
-        const _Float16* Wc = ring + cur * G::BUF;
+    for (int c = c0, cur = 0; c < nch; c += CSTEP, cur ^= 1) {
+        if (c + CSTEP < nch) fetch(c + CSTEP, cur ^ 1);
+        const _Float16* Wc = bufs + cur * G::BUF;
         // operand reads of the chunk in order: gate and up rows of each k-step, then the down tiles
         auto rd_op = [&](int i) {
             const _Float16* p = i < 2 * G::S ? Wc + up_lane + 8 * ((i & 1) * G::HC * G::GROW + 4 * (i >> 1))
@@ -328,23 +348,58 @@ swiglu_mlp_kernel(const uint16_t* __restrict__ x, int64_t rows, int64_t xs, cons
             if (t + kAhead < G::OT) op[i % kAhead] = rd_op(i + kAhead);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (c + 1 < nch) {
+        if (c + CSTEP < nch) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's loads are in LDS
-            __syncthreads();
+            if constexpr (!SPLIT) __syncthreads();
         }
     }
-    __syncthreads();  // the ring's last reads are done: its memory takes the rows
-    write_rows<E, NW>(yt, r0, rows, lane, ring + wave * 16 * (E + 8), y, ys, ep);
+    __syncthreads();  // the ring's last reads are done: its memory takes the sums or the rows
+    if constexpr (SPLIT) {
+        // wavefront w sums tile w over the wavefronts' partials, stages its columns of the 32 rows, and
+        // after those of all four takes rows 8w..8w+7
+        static_assert(G::OT == G::NWAVES, "a tile per wavefront");
+        f32x4* red = reinterpret_cast<f32x4*>(ring);  // [wavefront][tile][j][lane]
+        _Float16* ut = ring + G::NWAVES * G::OT * 4 * 64 * 8;
+        static_assert((G::NWAVES * G::OT * 4 * 64 * 8 + 32 * (E + 8)) <= G::NWAVES * 2 * G::BUF, "sums and rows fit");
+#pragma unroll
+        for (int t = 0; t < G::OT; ++t)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                red[((wave * G::OT + t) * 4 + j) * 64 + lane] =
+                    f32x4{yt[t][4 * j], yt[t][4 * j + 1], yt[t][4 * j + 2], yt[t][4 * j + 3]};
+        __syncthreads();
+        f32x16 sum = f32x16{};
+#pragma unroll
+        for (int w = 0; w < G::NWAVES; ++w)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 v = red[((w * G::OT + wave) * 4 + j) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sum[4 * j + i] = sum[4 * j + i] + v[i];
+            }
+        stage_tile(sum, ut + l32 * (E + 8) + 4 * hh + 32 * wave);
+        __syncthreads();
+        emit_rows<E, NW, 2>(ut + 8 * wave * (E + 8), r0 + 8 * wave, rows, lane, y, ys, ep);
+    } else {
+        write_rows<E, NW>(yt, r0, rows, lane, ring + wave * 16 * (E + 8), y, ys, ep);
+    }
 }
 
 template <int E, int NW = 0>
 void launch(const uint16_t* x, int64_t rows, int64_t xs, const uint16_t* wgu, const uint16_t* wd, int hp, uint16_t* y,
             int64_t ys, hipStream_t stream, const ResEpi& ep = ResEpi{}) {
     using G = MlpGeom<E>;
+    if constexpr (split_width(E)) {
+        if (rows <= (int64_t)kSplitRowsPerCu * device_cus()) {
+            hipLaunchKernelGGL((swiglu_mlp_kernel<E, NW, true>), dim3((unsigned)((rows + 31) / 32)), dim3(G::THREADS), 0,
+                               stream, x, rows, xs, wgu, wd, hp, y, ys, ep);
+            return;
+        }
+    }
     const int64_t per = G::NWAVES * 32;
     const dim3 grid((unsigned)((rows + per - 1) / per));
-    hipLaunchKernelGGL((swiglu_mlp_kernel<E, NW>), grid, dim3(G::THREADS), 0, stream, x, rows, xs, wgu, wd, hp, y, ys,
-                       ep);
+    hipLaunchKernelGGL((swiglu_mlp_kernel<E, NW, false>), grid, dim3(G::THREADS), 0, stream, x, rows, xs, wgu, wd, hp, y,
+                       ys, ep);
 }
 
 }  // namespace
