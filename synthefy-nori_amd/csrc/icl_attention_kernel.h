@@ -60,7 +60,7 @@ constexpr float kLn2 = 0.6931471805599453f;
 // log2 units a checked step may exceed the running max by: of the folded kernels, whose scan
 // checks one block in kAnchorBlocks (the less the max may lag, the more room a key in the blocks
 // between has below the f16 range), and of the VALU kernels, which check every step
-constexpr float kFoldSlack = 4.0f, kRescaleSlack = 8.0f;
+constexpr float kFoldSlack = 2.0f, kRescaleSlack = 8.0f;
 // Blocks from one checked block of a folded scan to the next (see the block loop).
 constexpr int kAnchorBlocks = 8;
 
@@ -804,9 +804,9 @@ icl_attention_kernel(const Args a) {
     // channels (2 % of them eight times the rest: logits of 6 log2 units' spread) sent most
     // workgroups through both scans: 6.46 -> 3.53 ms at d 44, 33 x 8 x 1024 queries x 65536 keys,
     // 1.50 -> 0.92 ms at 16384 keys. Unit-normal caches, which never rescan, pay for the added
-    // tests: 3.52 -> 3.59 ms. (16 blocks apart, the same cache rescans again: 4.2 ms; a slack of
-    // 8: 4.3 ms; a test in one step of every block: 3.59-3.63 ms.) The two scans do the same
-    // arithmetic
+    // tests: 3.52 -> 3.59 ms. (Slack: over ten such caches 3.60 ms on average at 2, 3.85 at 4 (one in
+    // three rescans somewhere), 4.3 at 8; four blocks apart at 2 or 4 3.62, 16 apart 4.2; a test in
+    // one step of every block 3.59-3.63.) The two scans do the same arithmetic
     // otherwise. (The VALU-mode kernels scan once with the test on: at DP 64 the second pass's
     // live state spills inside their loop and costs more than the test.)
     if constexpr (resident(NW)) {
