@@ -17,9 +17,9 @@ for the parts of the ICL stage that run per layer:
 Every sequence attention -- the context self-attention of the cache build and the
 query -> context attention over the (int8) cache -- runs on the HIP kernel
 (``nori_amd.attention``); RMSNorm runs on the HIP kernel (``nori_amd.norm``); the int8
-cache is written by the HIP quantizer (``nori_amd.kv_cache_scaling``). The projections are
-the reference's own GEMMs (einsum / F.linear, hipBLASLt on ROCm). The feature attention
-over a row's few tokens and the MLPs are the reference's torch expressions.
+cache is written by the HIP quantizer (``nori_amd.kv_cache_scaling``). Projections run on the
+library GEMM or, at the widths it is built for, on ``nori_linear_f16`` (``nori_amd.projection``); the
+feature attention over a row's tokens runs on the HIP kernel and the SwiGLU MLPs on the fused one.
 """
 
 from __future__ import annotations
@@ -122,7 +122,7 @@ class QASSMaxScaling(nn.Module):
         first, last = self.base_mlp[0], self.base_mlp[-1]
         if not (self.fused and q.is_cuda and q.dtype == torch.float16 and first.weight.is_cuda):
             return False
-        if first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None:
+        if first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None or _hooked(self.base_mlp):
             return False
         return self._computes_in_fp16(q, first)
 
@@ -197,7 +197,7 @@ class SwiGLUMLP(nn.Module):
         return (
             x.is_cuda and self.fused and self._projection_dtype() == torch.float16 and self.w_gate.bias is None
             and self.w_down.bias is None and x.shape[-1] == self.w_down.out_features
-            and x.shape[-1] in FUSED_MLP_WIDTHS
+            and x.shape[-1] in FUSED_MLP_WIDTHS and self.w_gate.weight.numel() < 1 << 28  # the kernel's 32-bit weight offsets
         )
 
     def _projection_dtype(self) -> torch.dtype:
