@@ -1285,10 +1285,10 @@ class EncoderBaseLayer(nn.Module):
     # small layers of the fused widths issue their launches from one native call
     # (nori_dense_apply); False keeps the sublayers' own calls
     native_apply = True
-    # Past this many tokens the kernels of a layer outlast the host's part of it, and its wider
-    # projections keep the library GEMM: 6m stack of 16 layers over 9 x 256 tokens 4.9 -> 1.6 ms; at
-    # 64 k tokens the two are level.
-    _NATIVE_TOKENS = 65536
+    # Up to this many tokens. One 6m layer, native against its own calls: 2,304 tokens 116 / 349 us,
+    # 32,768 152 / 271, 65,280 197 / 268, 204,000 592 / 632. Past that the kernels outlast the host,
+    # and the own calls free each operand as they go where the native scratch holds 10 bytes an element.
+    _NATIVE_TOKENS = 262144
 
     def _apply_native(self, x: torch.Tensor, kv_cache, feature_atten_mask) -> torch.Tensor | None:
         """``forward_test_with_cache`` as one native call, or None where that is not the same
