@@ -85,7 +85,8 @@ def _common_grid(*tensors: torch.Tensor) -> tuple | None:
 def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = False, min_rows: int = _MIN_ROWS) -> bool:
     """Whether ``linear(x, weight)`` runs on the HIP kernel (``any_width``: whether the kernel
     can take the operands at all, whatever the routing rule says)."""
-    if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == torch.float16 and weight.dim() == 2):
+    if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == torch.float16 and weight.dim() == 2
+            and weight.device == x.device):  # (F.linear refuses a weight on another device)
         return False
     k = int(x.shape[-1])
     widths = (128, 256) if any_width else _WIDTHS
@@ -141,7 +142,7 @@ def linear_head_norm(x: torch.Tensor, weight: torch.Tensor, gain: torch.Tensor, 
     row RMS-normed with ``gain`` [64], in one kernel (``nori_linear_f16_head_norm``): the
     projection and the per-head q/k norm of ``MultiheadAttention``, each rounded to fp16. Any row
     count; None where the kernel does not take the operands."""
-    if gain.shape != (64,) or not gain.is_cuda or gain.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+    if gain.shape != (64,) or gain.device != x.device or gain.dtype not in (torch.float32, torch.float16, torch.bfloat16):
         return None
     if norm_cols % 64 or not takes_kernel(x, weight, any_width=True, min_rows=1):
         return None

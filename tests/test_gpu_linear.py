@@ -317,3 +317,15 @@ def test_residual_into_another_stream_and_without_the_norm(cuda, k, rows):
     assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
     assert projection.linear_residual(a, w, x, ALPHA) and torch.equal(x, want)
     assert not projection.linear_residual(a, w, x, ALPHA, torch.empty(rows, k + 8, device=cuda)[:, :k])  # other strides
+
+
+def test_weights_on_another_device_are_refused(cuda):
+    # the kernel takes raw pointers: a weight or gain left on the host goes to the library GEMM,
+    # which raises
+    x = torch.randn(5000, 128, device=cuda).half()
+    w, gain = torch.randn(128, 128).half(), torch.ones(64)
+    assert not projection.takes_kernel(x, w) and not projection.takes_kernel(x, w, any_width=True)
+    assert projection.linear_head_norm(x, w.to(cuda), gain, 1e-6, 64) is None
+    assert projection.linear_head_norm(x, w, gain.to(cuda), 1e-6, 64) is None
+    with pytest.raises(RuntimeError):
+        projection.linear(x, w)
