@@ -436,12 +436,11 @@ class MultiheadAttention(nn.Module):
         mult = float(torch.tensor(math.log(float(max(n_keys, 2))), dtype=dtype)) if n_keys > 1 else 1.0
         return mult / math.sqrt(float(self.head_dim))
 
-    def _cast_weights(self, device: torch.device):
-        """(key, q weight [H*D, E], k|v weight [2*H*D, E], output weight [E, H*D], q|k|v weight
-        [3*H*D, E]) as F.linear takes them, in the dtype the projections compute in (the autocast
-        dtype under GPU autocast), cached until a weight changes. Autocast does not keep casts of
-        these reshaped views, so without the cache every call would cast them again; the values
-        are the same casts."""
+    def _linear_weights(self, device: torch.device):
+        """(q weight [H*D, E], k|v weight [2*H*D, E], output weight [E, H*D]) as F.linear takes
+        them, in the dtype the projections compute in (the autocast dtype under GPU autocast),
+        cached until a weight changes. Autocast does not keep casts of these reshaped views, so
+        without the cache every call would cast them again; the values are the same casts."""
         dtype = self.qkv_proj_weight.dtype
         if device.type == "cuda" and torch.is_autocast_enabled("cuda"):
             dtype = torch.get_autocast_dtype("cuda")
@@ -453,16 +452,22 @@ class MultiheadAttention(nn.Module):
             with torch.no_grad():
                 w = self.qkv_proj_weight.to(device=device, dtype=dtype)
                 out_w = self.out_proj_weight.reshape(hd, self.embed_dim).t().to(device=device, dtype=dtype).contiguous()
-                cached = self._cast = (key, w[0].reshape(hd, self.embed_dim), w[1:].reshape(2 * hd, self.embed_dim), out_w,
-                                       w.reshape(3 * hd, self.embed_dim))
-        return cached
+                cached = self._cast = (key, w[0].reshape(hd, self.embed_dim), w[1:].reshape(2 * hd, self.embed_dim), out_w)
+        return cached[1:]
 
-    def _linear_weights(self, device: torch.device):
-        """(q weight, k|v weight, output weight) of ``_cast_weights``."""
-        return self._cast_weights(device)[1:4]
+    def _live_weight(self, first: int, last: int) -> torch.Tensor:
+        """Projections ``first`` to ``last - 1`` of (q, k, v) as one F.linear weight
+        [(last - first) * H * D, E], in the dtype autocast casts it to. Cast by each call, on its own
+        stream, from the parameter as it is then: a kept cast misses an edit through ``.data``,
+        which moves neither address nor version, and is not ordered with calls on other streams."""
+        w = self.qkv_proj_weight[first:last].reshape(-1, self.embed_dim)
+        if torch.is_autocast_enabled("cuda") and w.dtype in (torch.float32, torch.float16, torch.bfloat16):
+            w = w.to(torch.get_autocast_dtype("cuda"))
+        return w
 
-    def _projects_with_cast_weights(self, x: torch.Tensor) -> bool:
-        """Whether a projection of x may take the cached casts (which carry no gradient)."""
+    def _projects_by_linear(self, x: torch.Tensor) -> bool:
+        """Whether a projection of x on the GPU takes the F.linear form for models without q/k norms
+        too (the projection kernel, which carries no gradient, may then take it)."""
         return x.is_cuda and not torch.is_grad_enabled()
 
     def _apply_extra_attn_scale(self, q: torch.Tensor, n_keys: int) -> torch.Tensor:
@@ -535,10 +540,6 @@ class MultiheadAttention(nn.Module):
         kv_proj_weight = self.qkv_proj_weight[1:]
         if copy_first_head_kv:
             kv = torch.einsum("... s, j h d s -> ... j h d", x_kv_flat, kv_proj_weight[:, :1])
-        elif self._projects_with_cast_weights(x_kv_flat):
-            # the same library GEMM on the same casts of the weight, not cast again on each call
-            kv = torch.nn.functional.linear(x_kv_flat, self._cast_weights(x_kv_flat.device)[2])
-            kv = kv.view(*x_kv_flat.shape[:-1], 2, self.num_heads, self.head_dim)
         else:
             kv = torch.nn.functional.linear(
                 x_kv_flat, kv_proj_weight.reshape(2 * self.num_heads * self.head_dim, self.embed_dim)
@@ -610,8 +611,8 @@ class MultiheadAttention(nn.Module):
         BS = B * S
         if self.qkv_combined:
             x = x.reshape(-1, *x.shape[-2:])
-            if self._projects_with_cast_weights(x):
-                qkv = proj_linear(x, self._cast_weights(x.device)[4])
+            if self._projects_by_linear(x):
+                qkv = proj_linear(x, self._live_weight(0, 3))
                 qkv = qkv.view(*x.shape[:-1], 3, self.num_heads, self.head_dim)
             else:
                 qkv = torch.einsum("... s, j h d s -> ... j h d", x, self.qkv_proj_weight)
@@ -641,7 +642,8 @@ class MultiheadAttention(nn.Module):
         B, S, F, _ = x.shape
         BS = B * S
         n_kv = int(x_kv.shape[-2])
-        use_linear = self._is_linear_projection_used(x.device) or self._projects_with_cast_weights(x)
+        kept = self._is_linear_projection_used(x.device)
+        use_linear = kept or self._projects_by_linear(x)
         # the projections read x and x_kv as they lie: a strided view such as the column
         # attention's [table, group, row] transpose of the cells goes through the projection
         # kernel without the copy its flattening would make (the result is contiguous)
@@ -652,7 +654,11 @@ class MultiheadAttention(nn.Module):
                                              normed[1].view(BS, n_kv, 2, self.num_heads, self.head_dim), attn_mask,
                                              normed=True)
         if use_linear:
-            w_q, w_kv, _ = self._linear_weights(x.device)
+            if kept:
+                w_q, w_kv, _ = self._linear_weights(x.device)
+            else:
+                w = self._live_weight(0, 1 if copy_first_head_kv else 3)
+                w_q, w_kv = w[: self.num_heads * self.head_dim], w[self.num_heads * self.head_dim:]
             q = proj_linear(x, w_q).view(BS, F, self.num_heads, self.head_dim)
         else:
             q = torch.einsum("... s, h d s -> ... h d", x.reshape(BS, F, -1), self.qkv_proj_weight[0])
@@ -668,7 +674,7 @@ class MultiheadAttention(nn.Module):
     def _project_normed(self, x: torch.Tensor, x_kv: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor] | None:
         """The q and k|v projections with their q/k norms formed in the same kernels, or None where
         those do not take them (heads other than 64 wide, other dtypes or widths, gradients)."""
-        if not (self.qk_norm and self.head_dim == 64 and self._projects_with_cast_weights(x)):
+        if not (self.qk_norm and self.head_dim == 64 and self._projects_by_linear(x)):
             return None
         if self.q_norm.weight is None or self.k_norm.weight is None:
             return None
@@ -955,12 +961,12 @@ class EncoderBaseLayer(nn.Module):
         if tokens is None:
             return None
         del operand
-        w = feat._cast_weights(x.device)
-        qkv = proj_linear(tokens.view(b * r, g, e), w[4]).view(b * r, g, 3, feat.num_heads, feat.head_dim)
+        w_out = feat._linear_weights(x.device)[2]
+        qkv = proj_linear(tokens.view(b * r, g, e), feat._live_weight(0, 3)).view(b * r, g, 3, feat.num_heads, feat.head_dim)
         del tokens
         out = icl_attention(feat._apply_extra_attn_scale(qkv[:, :, 0], g), qkv[:, :, 1:]).view(x.shape)
-        if not linear_residual(out, w[3], stream, alpha):
-            residual_add(stream, proj_linear(out, w[3]), alpha, inplace=True)
+        if not linear_residual(out, w_out, stream, alpha):
+            residual_add(stream, proj_linear(out, w_out), alpha, inplace=True)
         return stream
 
     def _takes_fused_steps(self, x: torch.Tensor, seq: MultiheadAttention, feature_atten_mask) -> bool:
@@ -1340,7 +1346,9 @@ class EncoderBaseLayer(nn.Module):
         if any(p.device != x.device for p in (seq.qkv_proj_weight, feat.qkv_proj_weight, mlp.w_gate.weight)):
             return None
         w_q, _, w_out = seq._linear_weights(x.device)
-        _, _, _, w_feat_out, w_qkv = feat._cast_weights(x.device)
+        w_feat_out, w_qkv = feat._linear_weights(x.device)[2], feat._live_weight(0, 3)
+        if w_qkv.dtype != torch.float16 or not w_qkv.is_contiguous():
+            return None
         base, gate = qass._half_weights("_base16", qass.base_mlp), qass._gate_weights()
         gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
         lib = nat.lib()

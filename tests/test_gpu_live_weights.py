@@ -11,8 +11,7 @@ import pytest
 import torch
 
 from nori_amd import ScalableSeqKV
-from nori_amd.layer import EncoderBaseLayer, MultiheadAttention, QASSMaxScaling
-from nori_amd.two_phase import CellLayer2P
+from nori_amd.layer import EncoderBaseLayer, MultiheadAttention
 
 pytestmark = pytest.mark.gpu
 
@@ -77,3 +76,29 @@ def test_dense_layer_reads_the_edited_projections(cuda, part):
         cache = {"seq_kv": ScalableSeqKV(kv, 1, 5, quantize=True)}
         got, before, want = _after_edit(layer, part, lambda m: m.forward_test_with_cache(x, cache))
         assert torch.equal(got, want) and not torch.equal(got, before)
+
+
+def test_cache_projection_of_weights_without_a_version_counter(cuda):
+    x = torch.randn(1, 3, 40, 128, generator=torch.Generator().manual_seed(7)).to(cuda)
+    with torch.inference_mode():
+        made = MultiheadAttention(128, 2, qkv_combined=False).to(cuda)
+        plain = torch.nn.functional.linear(x.view(3, 40, 128), made.qkv_proj_weight[1:].reshape(256, 128))
+        assert torch.equal(made.project_kv_cache(x)["kv"].view(3, 40, 256), plain)
+
+
+def test_a_call_on_another_stream_does_not_read_the_first_ones_casts(cuda):
+    # the first call's casts wait behind a long kernel on its own stream; a call on another stream
+    # must not read what they have not written yet
+    x = torch.randn(2, 60, 3, 128, generator=torch.Generator().manual_seed(8)).to(cuda).transpose(1, 2)
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        for call in (lambda m: m.attend(x, x), lambda m: m.project_kv_cache(x)["kv"]):
+            attn = _normal(MultiheadAttention(128, 2, qkv_combined=False), 9, cuda)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(busy):
+                torch.cuda._sleep(200_000_000)
+                want = call(attn)
+            with torch.cuda.stream(other):
+                got = call(attn)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
