@@ -13,7 +13,7 @@ extern "C" {
 // layer.py:316-456, under fp16 autocast): with l = T(log n), T the rounding to fp16,
 //     out[o] = T(l * T(1 + T(tanh(T(W2 h + b2)[o])))),  h = T(gelu(T(w1 l + b1))),
 // fp32 sums, gelu the erf form. w1, b1 [hidden], w2 [n_out, hidden], b2 [n_out], out [n_out], all
-// fp16 and contiguous; hidden is 64; w2 16-byte aligned.
+// fp16 and contiguous; hidden is 64.
 int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int32_t hidden,
                    int32_t n_out, void* out, void* stream);
 

@@ -234,28 +234,31 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
 }
 
 // The base scale: one output per thread. Every workgroup forms the 64 hidden units anew (one erf a
-// lane) rather than pass them through memory. As torch ops this vector of a few hundred values
+// lane) rather than pass them through memory, and takes its 64 rows of w2 through LDS: element loads,
+// so that weights of any alignment are taken (a parameter may be a view into a flat buffer), each
+// 64 consecutive elements of the wavefront. As torch ops this vector of a few hundred values
 // took eleven launches a layer (fill, two GEMMs with their bias copies, GELU, tanh, add, multiply,
 // weight casts), 37 us of device time and three times that on the host; as one kernel about 3 us.
 __global__ void __launch_bounds__(64)
 qass_base_kernel(float log_n, const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, int n_out,
                  uint16_t* out) {
     __shared__ float hid[kHid];
-    const int tid = threadIdx.x;
+    __shared__ float wt[64][kHid + 1];
+    const int tid = threadIdx.x, o0 = blockIdx.x * 64, o = o0 + tid;
+    const uint16_t* rows = w2 + (int64_t)o0 * kHid;
+    const int left = min(64, n_out - o0) * kHid;  // elements of this workgroup's rows
+    float w[kHid];
+#pragma unroll
+    for (int i = 0; i < kHid; ++i) w[i] = kHid * i + tid < left ? f16_to_f32(rows[kHid * i + tid]) : 0.0f;
     const float l = r16(log_n);
     hid[tid] = r16(gelu(r16(f16_to_f32(w1[tid]) * l + f16_to_f32(b1[tid]))));
-    __syncthreads();
-    const int o = blockIdx.x * 64 + tid;
-    if (o >= n_out) return;
-    const u32x4_t* wr = reinterpret_cast<const u32x4_t*>(w2 + (int64_t)o * kHid);
-    u32x4_t w[kHid / 8];
 #pragma unroll
-    for (int c = 0; c < kHid / 8; ++c) w[c] = wr[c];
+    for (int i = 0; i < kHid; ++i) wt[i][tid] = w[i];
+    __syncthreads();
+    if (o >= n_out) return;
     float acc = 0.0f;
 #pragma unroll
-    for (int c = 0; c < kHid / 8; ++c)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc = fmaf(f16_to_f32((uint16_t)(w[c][i >> 1] >> (16 * (i & 1)))), hid[8 * c + i], acc);
+    for (int j = 0; j < kHid; ++j) acc = fmaf(wt[tid][j], hid[j], acc);
     const float delta = r16(acc + f16_to_f32(b2[o]));
     out[o] = f32_to_f16(l * r16(1.0f + r16(tanh_f32(delta))));
 }
@@ -315,7 +318,6 @@ extern "C" int nori_qass_base(float log_n, const void* w1, const void* b1, const
     if (hidden != kHid) return fail(NORI_ERR_UNSUPPORTED, "qass_base: hidden width %d (64 only)", hidden);
     if (n_out <= 0) return fail(NORI_ERR_INVALID, "qass_base: %d outputs", n_out);
     if (!w1 || !b1 || !w2 || !b2 || !out) return fail(NORI_ERR_INVALID, "qass_base: null pointer");
-    if ((uintptr_t)w2 % 16) return fail(NORI_ERR_INVALID, "qass_base: w2 must be 16-byte aligned");
     hipLaunchKernelGGL(qass_base_kernel, dim3((unsigned)((n_out + 63) / 64)), dim3(64), 0, (hipStream_t)stream_v, log_n,
                        reinterpret_cast<const uint16_t*>(w1), reinterpret_cast<const uint16_t*>(b1),
                        reinterpret_cast<const uint16_t*>(w2), reinterpret_cast<const uint16_t*>(b2), n_out,

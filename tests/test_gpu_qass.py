@@ -137,3 +137,26 @@ def test_base_scale_against_the_separate_ops(heads, d, n_keys):
         assert float((got.double() - want.view(-1).double()).abs().max()) <= 3 * 2.0**-10 * float(log_n)
         m.base_mlp[-1].bias.add_(1.0)  # in place: the fp16 copies follow
         assert not torch.equal(layer_mod.qass_base(math.log(float(n_keys)), *m._half_weights("_base16", m.base_mlp)), got)
+
+
+@pytest.mark.parametrize("offset", [1, 4])
+def test_base_scale_of_weights_in_a_flat_buffer(offset):
+    # an fp16 module whose parameters are views into one buffer: rows of w2 on 2- and 8-byte
+    # boundaries, which the separate ops took. Against them: the base scale's bar of 3 * 2^-10 * T(log n)
+    # times the gate's factor (below 2), 2 ulps of the gate times |q * base| (base below 2 log n) and
+    # 4 ulps of the output (below 4 log n |q|): 18 * 2^-10 * log n * |q|
+    m = _module(2, 64, seed=3).to(DEV).half()
+    with torch.no_grad():
+        flat = torch.empty(offset + sum(p.numel() for p in m.parameters()), dtype=torch.float16, device=DEV)
+        at = offset
+        for p in m.parameters():
+            view = flat[at : at + p.numel()].view(p.shape)
+            view.copy_(p)
+            p.data = view
+            at += p.numel()
+    q = torch.randn(40, 3, 2, 64, generator=torch.Generator().manual_seed(2)).half().to(DEV)
+    with torch.inference_mode():
+        got = m(q, 300)
+        m.fused = False
+        want = m(q, 300)
+    assert bool(((got.float() - want.float()).abs() <= 18 * 2.0**-10 * math.log(300.0) * q.float().abs() + 2.0**-14).all())
