@@ -55,7 +55,8 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
     // sequence attention, in [table, group, row] order
     NORI_STEP(nori_rms_norm_rows(p->x, n, e, G, R, R * G * e, e, G * (int64_t)e, p->eps_seq, a0, NORI_F16, stream));
     NORI_STEP(nori_linear_f16(a0, 1, 1, n, e, 0, 0, e, p->w_q, e, e, a1, 0, 0, e, stream));
-    NORI_STEP(nori_qass_base(p->log_n, p->base_w1, p->base_b1, p->base_w2, p->base_b2, p->qass_hidden, e, base, stream));
+    NORI_STEP(nori_qass_base(p->log_n, p->base_w1, p->base_b1, p->base_w2, p->base_b2, p->base_dtype, p->qass_hidden, e,
+                             base, stream));
     NORI_STEP(nori_qass_gate(a1, NORI_F16, n, h, d, e, p->gate_w1, p->gate_b1, p->gate_w2, p->gate_b2, p->qass_hidden,
                              base, a0, e, stream));
     NORI_STEP(nori_icl_attention(a0, NORI_F16, B * G, R, h, d, R * e, e, d, p->kv, p->kv_dtype, p->kv_scales, p->nk,

@@ -12,10 +12,10 @@ extern "C" {
 // QASS base scale of one key count (QASSMaxScaling.forward's base branch, src/synthefy_nori/model/
 // layer.py:316-456, under fp16 autocast): with l = T(log n), T the rounding to fp16,
 //     out[o] = T(l * T(1 + T(tanh(T(W2 h + b2)[o])))),  h = T(gelu(T(w1 l + b1))),
-// fp32 sums, gelu the erf form. w1, b1 [hidden], w2 [n_out, hidden], b2 [n_out], out [n_out], all
-// fp16 and contiguous; hidden is 64.
-int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int32_t hidden,
-                   int32_t n_out, void* out, void* stream);
+// fp32 sums, gelu the erf form. w1, b1 [hidden], w2 [n_out, hidden], b2 [n_out], contiguous, of
+// w_dtype (fp32, fp16 or bf16), each rounded by T first; out [n_out] fp16; hidden is 64.
+int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int w_dtype,
+                   int32_t hidden, int32_t n_out, void* out, void* stream);
 
 // nori_rms_norm_to (no weight) of fp32 rows at three strides, written as contiguous fp16 or bf16
 // rows: row r = (i0 * d1 + i1) * d2 + i2 of x starts at element i0 * s0 + i1 * s1 + i2 * s2. Bit for
@@ -49,7 +49,7 @@ int nori_swiglu_mlp_residual(const void* x, int64_t rows, int32_t width, int64_t
 
 // One dense "smf" layer over query rows against its context cache, every launch from one call
 // (dense_layer.hip): x [tables, rows, groups, embed] fp32 contiguous is left as it is, out (the same
-// shape) takes the layer's output. Weights fp16, contiguous, as the module keeps them: w_q, w_out,
+// shape) takes the layer's output. Weights fp16 (the QASS base MLP's of base_dtype), contiguous: w_q, w_out,
 // w_feat_out [embed, embed], w_qkv [3 embed, embed], the QASS MLPs ([64, 1 | head width], [64],
 // [embed | head width, 64], ...), gate_up [2 hidden, embed] and down [embed, hidden] with hidden a
 // multiple of 32. The cache as nori_icl_attention takes it; alpha the deep-norm factor as rounded to
@@ -61,7 +61,7 @@ typedef struct {
     float* out;
     const void *w_q, *w_out, *w_qkv, *w_feat_out;
     const void *base_w1, *base_b1, *base_w2, *base_b2, *gate_w1, *gate_b1, *gate_w2, *gate_b2;
-    int32_t qass_hidden;
+    int32_t base_dtype, qass_hidden;
     const void *gate_up, *down;
     int32_t hidden;
     float eps_seq, eps_mlp, eps_feat, alpha, logit_scale, log_n;

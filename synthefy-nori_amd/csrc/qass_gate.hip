@@ -236,22 +236,24 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
 // The base scale: one output per thread. Every workgroup forms the 64 hidden units anew (one erf a
 // lane) rather than pass them through memory, and takes its 64 rows of w2 through LDS: element loads,
 // so that weights of any alignment are taken (a parameter may be a view into a flat buffer), each
-// 64 consecutive elements of the wavefront. As torch ops this vector of a few hundred values
+// 64 consecutive elements of the wavefront. Weights are rounded to fp16 here, as autocast casts them, so
+// the caller passes the parameters themselves: no cast to keep or to launch. As torch ops this vector of a few hundred values
 // took eleven launches a layer (fill, two GEMMs with their bias copies, GELU, tanh, add, multiply,
 // weight casts), 37 us of device time and three times that on the host; as one kernel about 3 us.
+template <int WT>
 __global__ void __launch_bounds__(64)
-qass_base_kernel(float log_n, const uint16_t* w1, const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, int n_out,
-                 uint16_t* out) {
+qass_base_kernel(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int n_out, uint16_t* out) {
     __shared__ float hid[kHid];
     __shared__ float wt[64][kHid + 1];
     const int tid = threadIdx.x, o0 = blockIdx.x * 64, o = o0 + tid;
-    const uint16_t* rows = w2 + (int64_t)o0 * kHid;
+    auto cast = [](const void* p, int64_t i) { return r16(load_elem<WT>(p, i)); };
+    const int64_t first = (int64_t)o0 * kHid;
     const int left = min(64, n_out - o0) * kHid;  // elements of this workgroup's rows
     float w[kHid];
 #pragma unroll
-    for (int i = 0; i < kHid; ++i) w[i] = kHid * i + tid < left ? f16_to_f32(rows[kHid * i + tid]) : 0.0f;
+    for (int i = 0; i < kHid; ++i) w[i] = kHid * i + tid < left ? cast(w2, first + kHid * i + tid) : 0.0f;
     const float l = r16(log_n);
-    hid[tid] = r16(gelu(r16(f16_to_f32(w1[tid]) * l + f16_to_f32(b1[tid]))));
+    hid[tid] = r16(gelu(r16(cast(w1, tid) * l + cast(b1, tid))));
 #pragma unroll
     for (int i = 0; i < kHid; ++i) wt[i][tid] = w[i];
     __syncthreads();
@@ -259,7 +261,7 @@ qass_base_kernel(float log_n, const uint16_t* w1, const uint16_t* b1, const uint
     float acc = 0.0f;
 #pragma unroll
     for (int j = 0; j < kHid; ++j) acc = fmaf(wt[tid][j], hid[j], acc);
-    const float delta = r16(acc + f16_to_f32(b2[o]));
+    const float delta = r16(acc + cast(b2, o));
     out[o] = f32_to_f16(l * r16(1.0f + r16(tanh_f32(delta))));
 }
 
@@ -312,15 +314,22 @@ extern "C" int nori_qass_gate(const void* q, int dtype, int64_t rows, int32_t he
     return launch_status("qass_gate");
 }
 
-extern "C" int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2,
+extern "C" int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int w_dtype,
                               int32_t hidden, int32_t n_out, void* out, void* stream_v) {
     clear_error();
     if (hidden != kHid) return fail(NORI_ERR_UNSUPPORTED, "qass_base: hidden width %d (64 only)", hidden);
+    if (w_dtype != NORI_F32 && w_dtype != NORI_F16 && w_dtype != NORI_BF16)
+        return fail(NORI_ERR_UNSUPPORTED, "qass_base: unsupported weight dtype %s", dtype_name(w_dtype));
     if (n_out <= 0) return fail(NORI_ERR_INVALID, "qass_base: %d outputs", n_out);
     if (!w1 || !b1 || !w2 || !b2 || !out) return fail(NORI_ERR_INVALID, "qass_base: null pointer");
-    hipLaunchKernelGGL(qass_base_kernel, dim3((unsigned)((n_out + 63) / 64)), dim3(64), 0, (hipStream_t)stream_v, log_n,
-                       reinterpret_cast<const uint16_t*>(w1), reinterpret_cast<const uint16_t*>(b1),
-                       reinterpret_cast<const uint16_t*>(w2), reinterpret_cast<const uint16_t*>(b2), n_out,
-                       reinterpret_cast<uint16_t*>(out));
+    const dim3 grid((unsigned)((n_out + 63) / 64)), block(64);
+    hipStream_t stream = (hipStream_t)stream_v;
+    auto o = reinterpret_cast<uint16_t*>(out);
+    if (w_dtype == NORI_F32)
+        hipLaunchKernelGGL((qass_base_kernel<NORI_F32>), grid, block, 0, stream, log_n, w1, b1, w2, b2, n_out, o);
+    else if (w_dtype == NORI_F16)
+        hipLaunchKernelGGL((qass_base_kernel<NORI_F16>), grid, block, 0, stream, log_n, w1, b1, w2, b2, n_out, o);
+    else
+        hipLaunchKernelGGL((qass_base_kernel<NORI_BF16>), grid, block, 0, stream, log_n, w1, b1, w2, b2, n_out, o);
     return launch_status("qass_base");
 }

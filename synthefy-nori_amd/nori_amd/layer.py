@@ -42,7 +42,7 @@ from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
 from .projection import linear_head_norm, linear_residual, linear_residual_norm
 from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, group_major_operand, operand_dtype, projection_operand,
-                   qass_base, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp,
+                   qass_base, qass_base_weights, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp,
                    swiglu_mlp_residual_norm)
 
 ACTIVATION_FN = {"gelu": nn.GELU(), "relu": nn.ReLU(), "silu": nn.SiLU()}
@@ -93,7 +93,7 @@ class QASSMaxScaling(nn.Module):
         if key_len <= 1:
             return q
         if self.qass_mode == "full" and self._fused_base_applies(q):
-            base_scale = qass_base(math.log(float(max(key_len, 2))), *self._half_weights("_base16", self.base_mlp))
+            base_scale = qass_base(math.log(float(max(key_len, 2))), *self._base_weights())
             base_scale = base_scale.view(1, 1, self.num_heads, self.head_dim)
             if self._fused_gate_applies(q, base_scale):
                 return qass_gate(q, *self._gate_weights(), base_scale)
@@ -156,6 +156,11 @@ class QASSMaxScaling(nn.Module):
                 cached = (key, tuple(p.detach().to(torch.float16).contiguous() for p in params))
             setattr(self, slot, cached)
         return cached[1]
+
+    def _base_weights(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+        """The base MLP's own parameters (w1, b1, w2, b2): the kernel rounds them itself."""
+        first, last = self.base_mlp[0], self.base_mlp[-1]
+        return first.weight, first.bias, last.weight, last.bias
 
     def _gate_weights(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         return self._half_weights("_gate16", self.gate_mlp)
@@ -1349,7 +1354,7 @@ class EncoderBaseLayer(nn.Module):
         w_feat_out, w_qkv = feat._linear_weights(x.device)[2], feat._live_weight(0, 3)
         if w_qkv.dtype != torch.float16 or not w_qkv.is_contiguous():
             return None
-        base, gate = qass._half_weights("_base16", qass.base_mlp), qass._gate_weights()
+        base, gate = qass_base_weights(*qass._base_weights()), qass._gate_weights()
         gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
         lib = nat.lib()
         scratch = torch.empty(lib.nori_dense_apply_scratch_bytes(b, r, g, e, heads, n_keys), dtype=torch.uint8, device=x.device)
@@ -1357,7 +1362,8 @@ class EncoderBaseLayer(nn.Module):
         sc = (0, 0, 0) if payload.dtype != torch.int8 else scales.stride()[:3]
         args = nat.DenseApplyArgs(
             b, r, g, e, heads, x.data_ptr(), out.data_ptr(), w_q.data_ptr(), w_out.data_ptr(), w_qkv.data_ptr(),
-            w_feat_out.data_ptr(), *(t.data_ptr() for t in base), *(t.data_ptr() for t in gate), QASS_GATE_HIDDEN,
+            w_feat_out.data_ptr(), *(t.data_ptr() for t in base), *(t.data_ptr() for t in gate),
+            nat.dtype_code(base[0].dtype), QASS_GATE_HIDDEN,
             gate_up.data_ptr(), down.data_ptr(), hidden, *(float(m.eps) for m in norms), self._alpha_value(q16),
             1.0 / math.sqrt(float(d)), math.log(float(n_keys)), payload.data_ptr(), nat.dtype_code(payload.dtype),
             None if payload.dtype != torch.int8 else scales.data_ptr(), n_keys, kv_heads, *payload.stride()[:3], *sc,

@@ -456,16 +456,29 @@ def swiglu_mlp_residual(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tens
 QASS_GATE_HIDDEN = 64
 
 
+def qass_base_weights(*weights: torch.Tensor) -> list[torch.Tensor]:
+    """The base MLP's parameters (w1, b1, w2, b2) as ``nori_qass_base`` reads them: themselves where they
+    are contiguous and of one dtype it takes, else fp16 casts made by this call."""
+    dtype = weights[0].dtype
+    if dtype in (torch.float32, torch.float16, torch.bfloat16) and all(w.dtype == dtype and w.is_contiguous() for w in weights):
+        return list(weights)
+    return [w.to(torch.float16).contiguous() for w in weights]
+
+
 def qass_base(log_n: float, w1: torch.Tensor, b1: torch.Tensor, w2: torch.Tensor, b2: torch.Tensor) -> torch.Tensor:
     """The QASS base scale ``T(log n) * (1 + tanh(base_mlp(T(log n))))`` as fp16 [n_out] in one launch
     (``nori_qass_base``), T the rounding to fp16, rounded where the separate fp16 ops round: w1
-    [64, 1], b1 [64], w2 [n_out, 64], b2 [n_out], fp16 and contiguous."""
+    [64, 1], b1 [64], w2 [n_out, 64], b2 [n_out], each rounded by T first."""
+    if w1.shape != (QASS_GATE_HIDDEN, 1) or b1.shape != (QASS_GATE_HIDDEN,) or w2.dim() != 2 \
+            or w2.shape[1] != QASS_GATE_HIDDEN or b2.shape != w2.shape[:1]:
+        raise ValueError(f"qass_base: weights {tuple(w1.shape)}, {tuple(w2.shape)} are not a 1 -> 64 -> n MLP's")
     device = nat.require_device(w1, b1, w2, b2)
+    w1, b1, w2, b2 = qass_base_weights(w1, b1, w2, b2)
     out = torch.empty(w2.shape[0], dtype=torch.float16, device=device)
     nat.check(
         nat.lib().nori_qass_base(
-            float(log_n), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), w2.shape[1], w2.shape[0],
-            out.data_ptr(), nat.stream_of(device),
+            float(log_n), w1.data_ptr(), b1.data_ptr(), w2.data_ptr(), b2.data_ptr(), nat.dtype_code(w1.dtype),
+            w2.shape[1], w2.shape[0], out.data_ptr(), nat.stream_of(device),
         ),
         "qass_base",
     )

@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from nori_amd import ScalableSeqKV
-from nori_amd.layer import EncoderBaseLayer, MultiheadAttention
+from nori_amd.layer import EncoderBaseLayer, MultiheadAttention, QASSMaxScaling
 
 pytestmark = pytest.mark.gpu
 
@@ -102,3 +102,21 @@ def test_a_call_on_another_stream_does_not_read_the_first_ones_casts(cuda):
                 got = call(attn)
             torch.cuda.synchronize()
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("param", ["base_mlp.0.weight", "base_mlp.0.bias", "base_mlp.2.weight", "base_mlp.2.bias"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_qass_reads_the_edited_base_mlp(cuda, param, dtype):
+    module = _normal(QASSMaxScaling(num_heads=2, head_dim=64, qass_mode="full"), 10, cuda).to(dtype)
+    q = torch.randn(40, 3, 2, 64, generator=torch.Generator().manual_seed(11)).half().to(cuda)
+    got, before, want = _after_edit(module, param, lambda m: m(q, 300))
+    assert torch.equal(got, want) and not torch.equal(got, before)
+
+
+def test_dense_layer_reads_the_edited_base_mlp(cuda):
+    x = torch.randn(1, 40, 5, 128, generator=torch.Generator().manual_seed(12)).to(cuda)
+    kv = torch.randn(5, 50, 2, 2, 64, generator=torch.Generator().manual_seed(13)).half().to(cuda)
+    cache = {"seq_kv": ScalableSeqKV(kv, 1, 5, quantize=True)}
+    got, before, want = _after_edit(_dense_layer(14, cuda), "sequence_attentions.1.qassmax.base_mlp.2.bias",
+                                    lambda m: m.forward_test_with_cache(x, cache))
+    assert torch.equal(got, want) and not torch.equal(got, before)

@@ -160,3 +160,14 @@ def test_base_scale_of_weights_in_a_flat_buffer(offset):
         m.fused = False
         want = m(q, 300)
     assert bool(((got.float() - want.float()).abs() <= 18 * 2.0**-10 * math.log(300.0) * q.float().abs() + 2.0**-14).all())
+
+
+def test_base_scale_rounds_its_weights_as_autocast_does():
+    # fp32 and bf16 parameters read by the kernel: bit for bit its result on their fp16 casts
+    for dtype in (torch.float32, torch.bfloat16):
+        m = _module(3, 44, seed=5).to(DEV).to(dtype)
+        params = [p.detach() for lin in (m.base_mlp[0], m.base_mlp[-1]) for p in (lin.weight, lin.bias)]
+        got = layer_mod.qass_base(math.log(777.0), *params)
+        assert torch.equal(got, layer_mod.qass_base(math.log(777.0), *[p.half() for p in params]))
+        mixed = [params[0].half(), params[1], params[2].t().contiguous().t(), params[3].half()]
+        assert torch.equal(got, layer_mod.qass_base(math.log(777.0), *mixed))
