@@ -124,14 +124,14 @@ class QASSMaxScaling(nn.Module):
             return False
         if first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None or _hooked(self.base_mlp):
             return False
-        return self._computes_in_fp16(q, first)
-
-    @staticmethod
-    def _computes_in_fp16(q: torch.Tensor, first: nn.Linear) -> bool:
-        autocast16 = torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.float16
-        if not (autocast16 or first.weight.dtype == torch.float16):
+        params = self._base_weights()
+        if torch.is_autocast_enabled("cuda"):  # which casts these dtypes, to its own
+            if torch.get_autocast_dtype("cuda") != torch.float16 \
+                    or any(p.dtype not in (torch.float32, torch.float16, torch.bfloat16) for p in params):
+                return False
+        elif any(p.dtype != torch.float16 for p in params):
             return False
-        return not (torch.is_grad_enabled() and (q.requires_grad or first.weight.requires_grad))
+        return not (torch.is_grad_enabled() and (q.requires_grad or any(p.requires_grad for p in params)))
 
     def _fused_gate_applies(self, q: torch.Tensor, base_scale: torch.Tensor) -> bool:
         """The gate MLP as one HIP pass: inference on fp16 queries whose gate linears compute in
@@ -142,7 +142,10 @@ class QASSMaxScaling(nn.Module):
         if first.out_features != QASS_GATE_HIDDEN or self.head_dim > 64 or self.head_dim % 4 or first.bias is None \
                 or last.bias is None:
             return False
-        return self._computes_in_fp16(q, first)
+        autocast16 = torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.float16
+        if not (autocast16 or first.weight.dtype == torch.float16):
+            return False
+        return not (torch.is_grad_enabled() and (q.requires_grad or first.weight.requires_grad))
 
     def _half_weights(self, slot: str, mlp: nn.Sequential) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """(w1, b1, w2, b2) of a two-layer MLP in fp16 (the casts autocast makes), kept in ``slot``

@@ -171,3 +171,19 @@ def test_base_scale_rounds_its_weights_as_autocast_does():
         assert torch.equal(got, layer_mod.qass_base(math.log(777.0), *[p.half() for p in params]))
         mixed = [params[0].half(), params[1], params[2].t().contiguous().t(), params[3].half()]
         assert torch.equal(got, layer_mod.qass_base(math.log(777.0), *mixed))
+
+
+def test_base_scale_follows_the_dtype_its_linears_compute_in():
+    # fp16 parameters under bf16 autocast compute in bf16, and the scaled queries come out as torch
+    # promotes them; parameters of two dtypes without autocast are refused
+    q = torch.randn(40, 3, 2, 64, generator=torch.Generator().manual_seed(4)).half().to(DEV)
+    m = _module(2, 64, seed=6).to(DEV).half()
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+        got = m(q, 300)
+        m.fused = False
+        want = m(q, 300)
+    assert got.dtype == want.dtype and torch.equal(got, want)
+    m.fused = True
+    m.base_mlp[-1].float()
+    with torch.inference_mode(), pytest.raises(RuntimeError):
+        m(q, 300)
