@@ -1332,6 +1332,8 @@ class EncoderBaseLayer(nn.Module):
         for m in (seq, feat):
             if m.use_logn_attention or m.use_learnable_attn_temperature or m.embed_dim != e or m.num_heads != self.nhead:
                 return None
+            if m._attention_dropout_p() != 0.0:  # a sublayer in training mode: its own call drops out, or refuses
+                return None
         for m in norms:
             if type(m) is not RMSNorm or m.weight is not None or tuple(m.normalized_shape) != (e,):
                 return None

@@ -100,3 +100,22 @@ def test_fused_build_equals_the_modules_calls(cuda, embed, heads, tables, rows, 
         assert len(fused) <= 1 and torch.equal(x, before)
     assert torch.equal(cache["seq_kv"]["kv"], ref["seq_kv"]["kv"])
     assert float((got - want).double().norm() / (want - x).double().norm()) <= 4 * 2.0**-11
+
+
+def test_sublayers_in_training_mode_keep_the_layers_own_calls(cuda):
+    # dropout follows each attention's own mode, not the layer's: the feature attention drops out and
+    # the cached attention refuses
+    layer = _layer(128, 2, False, 6, cuda)
+    x = torch.randn(1, 20, 4, 128, device=cuda)
+    cache = ScalableSeqKV(torch.randn(4, 50, 2, 2, 64, device=cuda).half(), 1, 4, quantize=True)
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        for attn in (layer.sequence_attentions[1], layer.feature_attentions[0]):
+            attn.train()
+            assert layer._apply_native(x, cache, None) is not None  # no dropout to apply
+            attn.dropout = 0.5
+            assert layer._apply_native(x, cache, None) is None
+            if attn is layer.sequence_attentions[1]:
+                with pytest.raises(RuntimeError, match="inference-only"):
+                    layer.forward_test_with_cache(x, {"seq_kv": cache})
+            attn.eval()
+            assert layer._apply_native(x, cache, None) is not None
