@@ -1353,7 +1353,7 @@ class EncoderBaseLayer(nn.Module):
         if not (qass.fused and qass._fused_base_applies(q16) and d <= 64 and d % 4 == 0
                 and qass._fused_gate_applies(q16, q16) and mlp.fuses(x)):
             return None
-        if any(p.device != x.device for p in (seq.qkv_proj_weight, feat.qkv_proj_weight, mlp.w_gate.weight)):
+        if any(p.device != x.device for p in (seq.qkv_proj_weight, mlp.w_gate.weight)):
             return None
         w_q, _, w_out = seq._linear_weights(x.device)
         w_feat_out, w_qkv = feat._linear_weights(x.device)[2], feat._live_weight(0, 3)
@@ -1361,6 +1361,15 @@ class EncoderBaseLayer(nn.Module):
             return None
         base, gate = qass_base_weights(*qass._base_weights()), qass._gate_weights()
         gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
+        # the call passes raw pointers: what the sublayers' own calls check, or refuse, is checked here
+        hid = QASS_GATE_HIDDEN
+        shaped = ((w_q, (e, e)), (w_out, (e, e)), (w_qkv, (3 * e, e)), (w_feat_out, (e, e)), (gate_up, (2 * hidden, e)),
+                  (down, (e, hidden)), *zip(base, ((hid, 1), (hid,), (e, hid), (e,))),
+                  *zip(gate, ((hid, d), (hid,), (d, hid), (d,))))
+        if any(t.device != x.device or tuple(t.shape) != shape for t, shape in shaped):
+            return None
+        if scales is not None and scales.device != x.device:
+            return None
         lib = nat.lib()
         scratch = torch.empty(lib.nori_dense_apply_scratch_bytes(b, r, g, e, heads, n_keys), dtype=torch.uint8, device=x.device)
         out = torch.empty_like(x)

@@ -119,3 +119,30 @@ def test_sublayers_in_training_mode_keep_the_layers_own_calls(cuda):
                     layer.forward_test_with_cache(x, {"seq_kv": cache})
             attn.eval()
             assert layer._apply_native(x, cache, None) is not None
+
+
+def test_parameters_on_another_device_or_of_another_shape_are_refused(cuda):
+    # the native call passes pointers, so it leaves such a layer to the sublayers' own calls, which raise
+    x = torch.randn(1, 20, 4, 128, device=cuda)
+    cache = ScalableSeqKV(torch.randn(4, 50, 2, 2, 64, device=cuda).half(), 1, 4, quantize=True)
+
+    def spoil_base(layer):
+        layer.sequence_attentions[1].qassmax.base_mlp[-1].cpu()
+
+    def spoil_gate(layer):
+        layer.sequence_attentions[1].qassmax.gate_mlp[-1].cpu()
+
+    def spoil_feature(layer):
+        layer.feature_attentions[0].qkv_proj_weight.data = layer.feature_attentions[0].qkv_proj_weight.data.cpu()
+
+    def shrink_base(layer):
+        layer.sequence_attentions[1].qassmax.base_mlp[-1] = torch.nn.Linear(64, 64).to(cuda)
+
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        for spoil in (spoil_base, spoil_gate, spoil_feature, shrink_base):
+            layer = _layer(128, 2, False, 7, cuda)
+            assert layer._apply_native(x, cache, None) is not None
+            spoil(layer)
+            assert layer._apply_native(x, cache, None) is None, spoil.__name__
+            with pytest.raises((RuntimeError, ValueError)):
+                layer.forward_test_with_cache(x, {"seq_kv": cache})
