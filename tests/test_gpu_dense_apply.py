@@ -138,11 +138,12 @@ def test_parameters_on_another_device_or_of_another_shape_are_refused(cuda):
     def shrink_base(layer):
         layer.sequence_attentions[1].qassmax.base_mlp[-1] = torch.nn.Linear(64, 64).to(cuda)
 
-    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
-        for spoil in (spoil_base, spoil_gate, spoil_feature, shrink_base):
-            layer = _layer(128, 2, False, 7, cuda)
+    for spoil in (spoil_base, spoil_gate, spoil_feature, shrink_base):
+        layer = _layer(128, 2, False, 7, cuda)
+        spoiled = _layer(128, 2, False, 7, cuda)
+        spoil(spoiled)
+        with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
             assert layer._apply_native(x, cache, None) is not None
-            spoil(layer)
-            assert layer._apply_native(x, cache, None) is None, spoil.__name__
+            assert spoiled._apply_native(x, cache, None) is None, spoil.__name__
             with pytest.raises((RuntimeError, ValueError)):
-                layer.forward_test_with_cache(x, {"seq_kv": cache})
+                spoiled.forward_test_with_cache(x, {"seq_kv": cache})
