@@ -33,7 +33,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from .layer import MultiheadAttention, SwiGLUMLP
+from .layer import MultiheadAttention, SwiGLUMLP, _hooked
 from .norm import (RMSNorm, operand_dtype, projection_operand, residual_add, residual_add_norm, swiglu_mlp_residual,
                    swiglu_mlp_residual_norm)
 from .projection import linear as proj_linear
@@ -117,13 +117,15 @@ def _mlp_accumulate(mlp: SwiGLUMLP, x: torch.Tensor, stream: torch.Tensor, alpha
                     *, operand: bool = True, out: torch.Tensor | None = None) -> torch.Tensor | None:
     """``_accumulate(stream, mlp(x), alpha, then, ...)``: with the next norm formed in the fp16
     operand dtype, the fused SwiGLU kernel applies the residual update and the norm itself
-    (``swiglu_mlp_residual_norm``: the MLP output never reaches memory) wherever it takes the
-    operands. ``stream`` holds x's rows (its last axis the norm's width)."""
-    if then is None and x.is_cuda and mlp.fuses(x) and operand_dtype(stream) == torch.float16:
+    (``swiglu_mlp_residual_norm``, ``swiglu_mlp_residual`` without a norm: the MLP output never
+    reaches memory) wherever it takes the operands; an MLP that is watched by hooks, or another
+    module, is called. ``stream`` holds x's rows (its last axis the norm's width)."""
+    fuses = x.is_cuda and type(mlp) is SwiGLUMLP and not _hooked(mlp) and mlp.fuses(x)
+    if then is None and fuses and operand_dtype(stream) == torch.float16:
         gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
         if swiglu_mlp_residual(x.to(torch.float16), gate_up, down, hidden, stream, alpha):
             return None
-    if (then is not None and operand and x.is_cuda and then.weight is None and mlp.fuses(x)
+    if (then is not None and operand and fuses and then.weight is None
             and tuple(then.normalized_shape) == (int(stream.shape[-1]),)
             and operand_dtype(stream) == torch.float16):
         gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
@@ -381,7 +383,8 @@ class CellLayer2P(nn.Module):
         del tokens
         cell_norm, row_norm, operand = (None, None, True) if then is None else then
         cell_next = _attend_accumulate(fa.feature_attentions[0], cell_out, cells, alpha, cell_norm, operand=operand)
-        mix = fa.mix_weight(readout.dtype, readout.device) if readout.is_cuda else None
+        plain_mix = type(fa.target_mix) is nn.Linear and fa.target_mix.bias is None and not _hooked(fa.target_mix)
+        mix = fa.mix_weight(readout.dtype, readout.device) if readout.is_cuda and plain_mix else None
         row_next = _linear_accumulate(readout, mix, rows, alpha, row_norm, lambda: fa.target_mix(readout),
                                       operand=operand) if mix is not None else \
             _accumulate(rows, fa.target_mix(readout), alpha, row_norm, operand=operand)

@@ -1,0 +1,91 @@
+"""The two-phase layers' fused updates stand for module calls: where a hook watches or replaces a
+module's output, or the module is another one, the module is called."""
+
+from __future__ import annotations
+
+import copy
+
+import pytest
+import torch
+
+from nori_amd.layer import SwiGLUMLP
+from nori_amd.two_phase import CellLayer2P, RowLayer2P
+
+pytestmark = pytest.mark.gpu
+
+
+def _filled(module, seed, device):
+    g = torch.Generator().manual_seed(seed)
+    with torch.no_grad():
+        for p in module.parameters():
+            p.copy_(torch.empty(p.shape).normal_(0.0, p.shape[-1] ** -0.5 if p.dim() > 1 else 0.1, generator=g))
+    return module.eval().to(device)
+
+
+def _cell(device):
+    layer = _filled(CellLayer2P(128, 2, 384, target_tokens=2, target_heads=4, target_hidden_dim=1024, deepnorm_alpha=0.25), 1, device)
+    g = torch.Generator().manual_seed(2)
+    cells, targets = (torch.randn(3, 41, n, 128, generator=g).to(device) for n in (5, 2))
+    return layer, lambda m: m(cells, targets, 30)
+
+
+def _row(device):
+    layer = _filled(RowLayer2P(256, 4, 1024, deepnorm_alpha=0.25), 3, device)
+    g = torch.Generator().manual_seed(4)
+    rows = torch.randn(3, 41, 256, generator=g).to(device)
+    memory = torch.randn(3, 41, 5, 256, generator=g).half().to(device)
+    return layer, lambda m: (m(rows, 30, memory),)
+
+
+def _run(layer, call):
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        return call(layer)
+
+
+@pytest.mark.parametrize("make,module,last", [
+    (_row, "mlp.0", "w_down"), (_cell, "mlp.0", "w_down"), (_cell, "mlp.1", "w_down"), (_cell, "feature_attention.target_mix", None),
+])
+def test_a_hook_replaces_the_update(cuda, make, module, last):
+    # a hook that returns zeros gives what zero weights give, bit for bit
+    layer, call = make(cuda)
+    zeroed = copy.deepcopy(layer)
+    target = zeroed.get_submodule(module)
+    with torch.no_grad():
+        (target if last is None else getattr(target, last)).weight.zero_()
+    plain, want = _run(layer, call), _run(zeroed, call)
+    seen = []
+    handle = layer.get_submodule(module).register_forward_hook(lambda m, args, out: seen.append(1) or torch.zeros_like(out))
+    got = _run(layer, call)
+    handle.remove()
+    assert len(seen) == 1
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and not all(torch.equal(a, b) for a, b in zip(got, plain))
+    assert all(torch.equal(a, b) for a, b in zip(_run(layer, call), plain))
+
+
+def test_another_mlp_class_is_called(cuda):
+    class Silent(SwiGLUMLP):
+        def forward(self, x):
+            return torch.zeros_like(super().forward(x))
+
+    layer, call = _row(cuda)
+    zeroed = copy.deepcopy(layer)
+    with torch.no_grad():
+        zeroed.mlp[0].w_down.weight.zero_()
+    layer.mlp[0].__class__ = Silent
+    assert torch.equal(_run(layer, call)[0], _run(zeroed, call)[0])
+
+
+def test_a_biased_target_mix_keeps_its_bias(cuda):
+    # (cells, targets): the bias moves the targets by alpha times itself, to the fp16 rounding of the update
+    layer, call = _cell(cuda)
+    mix = layer.feature_attention.target_mix
+    plain = _run(layer, call)
+    biased = torch.nn.Linear(256, 256).to(cuda)
+    with torch.no_grad():
+        biased.weight.copy_(mix.weight)
+        biased.bias.normal_(0.0, 1.0, generator=torch.Generator(device=cuda).manual_seed(5))
+    layer.feature_attention.target_mix = biased
+    got = _run(layer, call)
+    assert torch.equal(got[0], plain[0])
+    moved = got[1] - plain[1] - 0.25 * biased.bias.detach().view(2, 128)
+    assert float(moved.abs().max()) <= 2.0**-11 * 16  # updates below 8, two roundings of each of the two
