@@ -246,15 +246,10 @@ class DecoupledFeatureAttention(nn.Module):
         cells_out = self.feature_attentions[0].project_out(cell_out)
         return cells_out, self.target_mix(readout).view(b, r, self.target_tokens, width)
 
-    def mix_weight(self, dtype: torch.dtype, device) -> torch.Tensor:
-        """``target_mix``'s weight in ``dtype`` (the projection dtype), cached until it changes."""
-        p = self.target_mix.weight
-        key = (dtype, device, p.data_ptr(), p._version)
-        cached = getattr(self, "_mix", None)
-        if cached is None or cached[0] != key:
-            with torch.no_grad():
-                cached = self._mix = (key, p.to(device=device, dtype=dtype).contiguous())
-        return cached[1]
+    def mix_weight(self, dtype: torch.dtype) -> torch.Tensor:
+        """``target_mix``'s weight in ``dtype`` (the projection dtype), cast by each call: an edit through
+        ``.data``, which moves neither its address nor its version, reaches the next one."""
+        return self.target_mix.weight.detach().to(dtype).contiguous()
 
     def attend(self, tokens: torch.Tensor, n_cells: int) -> tuple[torch.Tensor, torch.Tensor]:
         """``forward`` before the cells' output projection and ``target_mix``: (the cell
@@ -384,7 +379,7 @@ class CellLayer2P(nn.Module):
         cell_norm, row_norm, operand = (None, None, True) if then is None else then
         cell_next = _attend_accumulate(fa.feature_attentions[0], cell_out, cells, alpha, cell_norm, operand=operand)
         plain_mix = type(fa.target_mix) is nn.Linear and fa.target_mix.bias is None and not _hooked(fa.target_mix)
-        mix = fa.mix_weight(readout.dtype, readout.device) if readout.is_cuda and plain_mix else None
+        mix = fa.mix_weight(readout.dtype) if readout.is_cuda and plain_mix else None
         row_next = _linear_accumulate(readout, mix, rows, alpha, row_norm, lambda: fa.target_mix(readout),
                                       operand=operand) if mix is not None else \
             _accumulate(rows, fa.target_mix(readout), alpha, row_norm, operand=operand)

@@ -1,5 +1,5 @@
 """The two-phase layers' fused updates stand for module calls: where a hook watches or replaces a
-module's output, or the module is another one, the module is called."""
+module's output, or the module is another one, the module is called, with its weights as they are then."""
 
 from __future__ import annotations
 
@@ -89,3 +89,13 @@ def test_a_biased_target_mix_keeps_its_bias(cuda):
     assert torch.equal(got[0], plain[0])
     moved = got[1] - plain[1] - 0.25 * biased.bias.detach().view(2, 128)
     assert float(moved.abs().max()) <= 2.0**-11 * 16  # updates below 8, two roundings of each of the two
+
+
+def test_target_mix_is_read_as_edited(cuda):
+    layer, call = _cell(cuda)
+    _run(layer, call)
+    layer.feature_attention.target_mix.weight.data.mul_(-1.5)  # moves neither address nor version
+    fresh, _ = _cell(cuda)
+    with torch.no_grad():
+        fresh.feature_attention.target_mix.weight.mul_(-1.5)
+    assert all(torch.equal(a, b) for a, b in zip(_run(layer, call), _run(fresh, call)))
