@@ -681,8 +681,11 @@ class MultiheadAttention(nn.Module):
 
     def _project_normed(self, x: torch.Tensor, x_kv: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor] | None:
         """The q and k|v projections with their q/k norms formed in the same kernels, or None where
-        those do not take them (heads other than 64 wide, other dtypes or widths, gradients)."""
+        those do not take them (heads other than 64 wide, other dtypes or widths, gradients, norms that
+        are watched by hooks or are other modules)."""
         if not (self.qk_norm and self.head_dim == 64 and self._projects_by_linear(x)):
+            return None
+        if type(self.q_norm) is not RMSNorm or type(self.k_norm) is not RMSNorm or _hooked(self.q_norm, self.k_norm):
             return None
         if self.q_norm.weight is None or self.k_norm.weight is None:
             return None

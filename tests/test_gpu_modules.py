@@ -155,3 +155,21 @@ def _chain_cases(layer, steps, cuda, layer_arch):
             else:
                 check_relative(got, ref, 1e-3, f"{layer_arch} residual chain with the layer's sublayers")
     layer.layer_steps = own_steps
+
+
+def test_watched_query_norm_is_called(cuda):
+    # queries past the attention kernels' own norms (300 over 300 keys): a hook on the query norm runs,
+    # and its result is used -- zeros give what a gain of zeros gives; the projection that forms the
+    # norms itself takes the same module without a hook
+    mod = _module(cuda, 128, 2, qkv_combined=False, use_qassmax=True, qass_mode="log_only", qk_norm=True)
+    x = torch.randn(1, 2, 300, 128, generator=torch.Generator().manual_seed(3)).half().to(cuda)
+    seen = []
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        assert mod._project_normed(x, x) is not None
+        handle = mod.q_norm.register_forward_hook(lambda m, args, out: seen.append(1) or torch.zeros_like(out))
+        got = mod.attend(x, x)
+        handle.remove()
+    with torch.no_grad():
+        mod.q_norm.weight.zero_()
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+        assert seen and torch.equal(got, mod.attend(x, x))
