@@ -218,6 +218,8 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream_of(device: torch.device) -> int:
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index if device.index is not None else torch.cuda.current_device()
     return torch._C._cuda_getCurrentRawStream(index)  # current_stream(device).cuda_stream without the Stream object
 

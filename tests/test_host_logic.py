@@ -9,6 +9,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from nori_amd import _native as nat
 from nori_amd.kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, _split_strides, _vector_layout, scale_caches
 
 
@@ -145,3 +146,9 @@ def test_log_only_qass_logit_scale_rounds_log_n_in_the_query_dtype():
     assert mod.log_only_logit_scale(256, torch.float16) != math.log(256) / 8.0  # the fp16 rounding is kept
     assert mod.log_only_logit_scale(1, torch.float16) == 1.0 / 8.0
     assert mod.log_only_logit_scale(0, torch.float32) == 1.0 / 8.0
+
+
+def test_a_stream_is_asked_of_gpu_devices_only():
+    # a tensor on the host has no stream to launch on: refused, not given the current GPU's
+    with pytest.raises(ValueError, match="cuda"):
+        nat.stream_of(torch.device("cpu"))
