@@ -169,7 +169,9 @@ def lib() -> ctypes.CDLL:
         if found != ABI_VERSION:
             raise RuntimeError(f"{LIBRARY} has ABI version {found}, this package binds version {ABI_VERSION}; rebuild it")
         for name, (restype, argtypes) in (SIGNATURES | OPS).items():
-            fn = getattr(handle, name)
+            fn = getattr(handle, name, None)
+            if fn is None:  # the package's own entry points move without the ABI version
+                raise RuntimeError(f"{LIBRARY} has no {name}: it was built from other sources; rebuild it")
             fn.restype = restype
             fn.argtypes = argtypes
         _lib = handle

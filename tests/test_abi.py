@@ -286,3 +286,13 @@ def test_qk_prologue_only_on_the_short_context_path():
         None, nat.NORI_F16, 0, 0, 0, None, 0, None, 0, ctypes.addressof(keyed), None,
     )
     assert rc == nat.NORI_ERR_UNSUPPORTED
+
+
+def test_a_library_of_other_sources_asks_to_be_rebuilt(monkeypatch):
+    # the package's own entry points carry no version: one that is missing is named, with what to do
+    from nori_amd import _native as nat
+
+    monkeypatch.setattr(nat, "_lib", None)
+    monkeypatch.setattr(nat, "OPS", nat.OPS | {"nori_not_built_yet": (ctypes.c_int, [])})
+    with pytest.raises(RuntimeError, match="nori_not_built_yet.*rebuild"):
+        nat.lib()
