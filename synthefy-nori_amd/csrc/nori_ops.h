@@ -9,6 +9,10 @@
 extern "C" {
 #endif
 
+// Moves with every change of a signature or struct below; the package binds one version.
+#define NORI_OPS_VERSION 2
+int nori_ops_version(void);
+
 // QASS base scale of one key count (QASSMaxScaling.forward's base branch, src/synthefy_nori/model/
 // layer.py:316-456, under fp16 autocast): with l = T(log n), T the rounding to fp16,
 //     out[o] = T(l * T(1 + T(tanh(T(W2 h + b2)[o])))),  h = T(gelu(T(w1 l + b1))),

@@ -32,3 +32,5 @@ int launch_status(const char* what) {
 extern "C" int nori_abi_version(void) { return NORI_ABI_VERSION; }
 
 extern "C" const char* nori_last_error(void) { return g_error; }
+
+extern "C" int nori_ops_version(void) { return NORI_OPS_VERSION; }

@@ -129,7 +129,8 @@ class DenseApplyArgs(ctypes.Structure):
     )
 
 
-# The package's own entry points beyond the C ABI (csrc/nori_ops.h).
+# The package's own entry points beyond the C ABI (csrc/nori_ops.h), and their version.
+OPS_VERSION = 2
 OPS: dict[str, tuple[object, list]] = {
     "nori_qass_base": (ctypes.c_int, [_f32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp]),
     "nori_linear_f16_head_norm": (
@@ -168,9 +169,14 @@ def lib() -> ctypes.CDLL:
         found = handle.nori_abi_version()
         if found != ABI_VERSION:
             raise RuntimeError(f"{LIBRARY} has ABI version {found}, this package binds version {ABI_VERSION}; rebuild it")
+        # the package's own entry points move without the ABI version
+        ops = getattr(handle, "nori_ops_version", None)
+        found = 0 if ops is None else ops()
+        if found != OPS_VERSION:
+            raise RuntimeError(f"{LIBRARY} has version {found} of the package's own entry points, not {OPS_VERSION}; rebuild it")
         for name, (restype, argtypes) in (SIGNATURES | OPS).items():
             fn = getattr(handle, name, None)
-            if fn is None:  # the package's own entry points move without the ABI version
+            if fn is None:
                 raise RuntimeError(f"{LIBRARY} has no {name}: it was built from other sources; rebuild it")
             fn.restype = restype
             fn.argtypes = argtypes

@@ -289,10 +289,14 @@ def test_qk_prologue_only_on_the_short_context_path():
 
 
 def test_a_library_of_other_sources_asks_to_be_rebuilt(monkeypatch):
-    # the package's own entry points carry no version: one that is missing is named, with what to do
+    # the package's own entry points move without the ABI version: another version of them, or one
+    # that is missing, is named with what to do
     from nori_amd import _native as nat
 
     monkeypatch.setattr(nat, "_lib", None)
     monkeypatch.setattr(nat, "OPS", nat.OPS | {"nori_not_built_yet": (ctypes.c_int, [])})
     with pytest.raises(RuntimeError, match="nori_not_built_yet.*rebuild"):
+        nat.lib()
+    monkeypatch.setattr(nat, "OPS_VERSION", nat.OPS_VERSION + 1)
+    with pytest.raises(RuntimeError, match="own entry points.*rebuild"):
         nat.lib()
