@@ -385,9 +385,13 @@ __global__ void __launch_bounds__(kThreads) icl_attention_rows_kernel(const Args
     }
 }
 
-// Whether the kernel above takes a call: 16-byte loads of q, K and V, 8-byte stores.
-bool takes_rows(const Args& a, int64_t groups) {
-    return a.q_dtype == NORI_F16 && (a.flags & kQVec8) && (a.flags & kOutVec4) && a.d % 8 == 0 && a.d <= 64 &&
+// Whether the kernel above takes a call: 16-byte loads of q, K and V, 8-byte stores; and heads that fill
+// its groups of 8 lanes. The one above it gives a head d / 4 lanes (to a power of two), so at up to 32
+// elements it holds more queries a wavefront. 2 heads of 16 / 32 / 40 / 56, with q/k norms: one query over
+// 12 keys of 53,333 rows 20 / 32 / 54 / 68 us there, 38 / 39 / 41 / 52 us here; 4 queries over 6 keys of
+// 40,000 rows 25 / 46 / 87 / 90 there, 37 / 37 / 38 / 40 here.
+bool takes_rows(const Args& a, int64_t groups, int64_t qb) {
+    return (a.d > 32 || (a.d > 16 && qb > 1)) && a.q_dtype == NORI_F16 && (a.flags & kQVec8) && (a.flags & kOutVec4) && a.d % 8 == 0 && a.d <= 64 &&
            (uintptr_t)a.kv % 16 == 0 && a.kv_bg % 8 == 0 && a.kv_row % 8 == 0 && a.kv_half % 8 == 0 && groups < 0x7fffffffLL;
 }
 
@@ -440,7 +444,7 @@ int launch_short(int kv_dtype, const Args& a, const Prologue& pro, hipStream_t s
         case NORI_F16: {
             // blocks of up to 5 queries, as even as they come
             const int64_t nqb = (a.nq + 4) / 5, qb = (a.nq + nqb - 1) / nqb, groups = a.bg * a.heads * nqb;
-            if (takes_rows(a, groups)) return launch_rows(a, (uint32_t)groups, (uint32_t)nqb, (int)qb, pro, stream);
+            if (takes_rows(a, groups, qb)) return launch_rows(a, (uint32_t)groups, (uint32_t)nqb, (int)qb, pro, stream);
             return launch_group<NORI_F16>(a, pro, stream);
         }
         case NORI_BF16: return launch_group<NORI_BF16>(a, pro, stream);

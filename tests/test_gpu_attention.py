@@ -727,3 +727,11 @@ def test_grouped_queries_against_the_row_kernel(cuda, d, h, hk, nq, nk, prologue
         got = nori_amd.icl_attention(queries, kv, lse=lse, qk_prologue=pro)
         assert bool(((got.double().cpu() - exp).abs() <= tol).all())
         assert torch.isfinite(lse).all()
+
+
+@pytest.mark.parametrize("d", [16, 32, 40])
+@pytest.mark.parametrize("nq,nk", [(1, 7), (2, 7), (6, 33)])
+@pytest.mark.parametrize("prologue", [False, True])
+def test_narrow_heads_around_the_grouped_kernels_rule(cuda, d, nq, nk, prologue):
+    # heads of up to 32 keep the kernel of a query a group for one query (up to 16 for any count)
+    test_grouped_queries_against_the_row_kernel(cuda, d, 2, 2, nq, nk, prologue)
