@@ -9,7 +9,8 @@
 // write against 2K FLOP), so the kernel is built for bandwidth: each x row is read from HBM
 // once and each output row written once.
 //   * A workgroup of 8 wavefronts keeps a chunk of 128 output columns of W in LDS as f16 (zero
-//     rows past n) and walks blocks of 256 rows (128 while 256 leave CUs idle).
+//     rows past n) and walks blocks of 256 rows; small calls take blocks of 128, and chunks of 64
+//     where K is 256 (the rule stands at launch()).
 //   * Each wavefront holds its 32 (16) rows of x as v_mfma_f32_16x16x32_f16 B operands (lane
 //     n + 16*(k/8) holds row n, elements 8*(k/8)..+8 of every 32-wide step) and computes the
 //     transposed product W x^T tile by tile: each lane ends with four consecutive output
@@ -176,9 +177,10 @@ __global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(c
     _Float16* my = lds + NC * PITCH + wave * WROWS * SP;
     const int ncols = min(NC, a.n - c0);
     for (; blk < last; blk += a.teams) {
-        // the next block's rows (the last block loads its own again, unused)
+        // the next block's rows
         f16x8 xn[NR][KS];
-        load_x(blk + a.teams < last ? blk + a.teams : blk, xn);
+        const bool more = blk + a.teams < last;  // uniform over the workgroup
+        if (more) load_x(blk + a.teams, xn);
         // lane r < WROWS has row r's place in y; the store passes (8 rows each, 8 lanes a row)
         // take it from there
         const int64_t row0 = blk * BROWS + wave * WROWS;
@@ -219,6 +221,7 @@ __global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(c
                 }
             }
         }
+        if (!more) break;
 #pragma unroll
         for (int nt = 0; nt < NR; ++nt)
 #pragma unroll
@@ -234,24 +237,36 @@ int launch_tiles(LinArgs a, int cus, hipStream_t stream) {
     if (hipFuncSetAttribute((const void*)linear_f16_kernel<KS, NC, NR, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
         return fail(NORI_ERR_RUNTIME, "linear_f16: cannot reserve %zu bytes of LDS", lds);
+    a.nchunks = (a.n + NC - 1) / NC;
     a.nblocks = (a.rows + BROWS - 1) / BROWS;
     // resident workgroups (LDS-bound, 16 wavefronts per CU at most), dealt to the XCDs in whole
     // teams: one workgroup per column chunk over the same row blocks
     const int64_t slots = (int64_t)cus * std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / lds, 2)) / 8;
-    a.teams = (int)std::max<int64_t>(1, std::min<int64_t>(slots / a.nchunks, (a.nblocks + 7) / 8));
+    const int64_t per_xcd = (a.nblocks + 7) / 8, most = std::max<int64_t>(1, std::min<int64_t>(slots / a.nchunks, per_xcd));
+    const int64_t rounds = (per_xcd + most - 1) / most;
+    a.teams = (int)((per_xcd + rounds - 1) / rounds);  // no more than share the blocks evenly
     const int64_t grid = 8 * (int64_t)a.teams * a.nchunks;
     if (grid > 0x7fffffffLL) return fail(NORI_ERR_UNSUPPORTED, "linear_f16: %d columns exceed one launch", a.n);
     hipLaunchKernelGGL((linear_f16_kernel<KS, NC, NR, NORM>), dim3((unsigned)grid), dim3(kThreads), lds, stream, a);
     return launch_status("linear_f16");
 }
 
-template <int KS, int NC, bool NORM>
+// The tile of a call. Workgroups of 256 rows x 128 columns from 0.4 of them a CU: below, twice as many of
+// 128 rows are ahead (4,096 rows, K 128: N 768, 96 of them, 7.3 -> 6.3 us), above, W staged twice as often
+// costs more (8,192 x 768, 192 of them: 8.5 us against 8.9 in 128 rows; 33,000 x 128, 129: 7.9 against 8.2).
+// At K 256 a workgroup stages 64 KB of W, so while chunks of 64 leave no more than one workgroup a CU they
+// are ahead: 64 to 4,096 rows, N 256 6.9 - 8.3 -> 4.9 - 6.1 us. Teams share the blocks evenly: 65,536 x 640, K 128:
+// 27.1 -> 26.7 us, N 384 20.1 -> 19.8; and the last block of a workgroup loads no rows after it, which cost
+// calls of about a block each 5 to 10 % (20,000 x 640: 13.9 -> 12.7 us).
+template <int KS, bool NORM>
 int launch(LinArgs a, hipStream_t stream) {
-    a.nchunks = (a.n + NC - 1) / NC;
     const int cus = device_cus();
-    // 256-row blocks; 128-row ones while those leave CUs without a workgroup
-    if ((a.rows + 255) / 256 * a.nchunks < cus) return launch_tiles<KS, NC, 1, NORM>(a, cus, stream);
-    return launch_tiles<KS, NC, 2, NORM>(a, cus, stream);
+    const int64_t chunks = (a.n + 127) / 128, blocks = (a.rows + 255) / 256;
+    if (5 * blocks * chunks >= 2 * cus) return launch_tiles<KS, 128, 2, NORM>(a, cus, stream);
+    if constexpr (KS == 8) {
+        if (2 * ((a.rows + 127) / 128) * chunks <= cus) return launch_tiles<KS, 64, 1, NORM>(a, cus, stream);
+    }
+    return launch_tiles<KS, 128, 1, NORM>(a, cus, stream);
 }
 
 // ---------------------------------------------------------------- projection + residual + norm
@@ -463,8 +478,8 @@ int run_linear(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, i
     a.eps = eps;
     a.norm_cols = norm_cols;
     hipStream_t s = (hipStream_t)stream;
-    if (norm_cols > 0) return k == 128 ? launch<4, 128, true>(a, s) : launch<8, 128, true>(a, s);
-    return k == 128 ? launch<4, 128, false>(a, s) : launch<8, 128, false>(a, s);
+    if (norm_cols > 0) return k == 128 ? launch<4, true>(a, s) : launch<8, true>(a, s);
+    return k == 128 ? launch<4, false>(a, s) : launch<8, false>(a, s);
 }
 
 }  // namespace

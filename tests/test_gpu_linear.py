@@ -329,3 +329,18 @@ def test_weights_on_another_device_are_refused(cuda):
     assert projection.linear_head_norm(x, w, gain.to(cuda), 1e-6, 64) is None
     with pytest.raises(RuntimeError):
         projection.linear(x, w)
+
+
+@pytest.mark.parametrize("k", [128, 256])
+@pytest.mark.parametrize("rows,n", [(128, 4), (129, 64), (4095, 196), (6500, 516), (13057, 260), (26000, 132), (100001, 68)])
+def test_tiles_at_their_rules_edges(cuda, k, rows, n):
+    # 128- and 256-row blocks, 64- and 128-column chunks, one block a workgroup and several shared
+    # unevenly: dyadic operands, so every order of the sums gives the same fp32 value; the rows around
+    # the output stay as they are
+    g = torch.Generator().manual_seed(rows + n + k)
+    x, w = dyadic((rows, k), 1 / 8, 4.0, g, cuda), dyadic((n, k), 1 / 64, 1.0, g, cuda)
+    buf = torch.full((rows + 2, n), 7.0, dtype=torch.float16, device=cuda)
+    projection.linear(x, w, out=buf[1:-1], any_width=True)
+    want = (x.double() @ w.double().t()).half()
+    assert torch.equal(buf[1:-1], want) and torch.equal(kernel_linear(x, w), want)
+    assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
