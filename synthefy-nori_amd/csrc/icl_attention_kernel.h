@@ -803,10 +803,11 @@ icl_attention_kernel(const Args a) {
     // Anchored on the first block alone, and tested only at the end, a cache with a few wide
     // channels (2 % of them eight times the rest: logits of 6 log2 units' spread) sent most
     // workgroups through both scans: 6.46 -> 3.53 ms at d 44, 33 x 8 x 1024 queries x 65536 keys,
-    // 1.50 -> 0.92 ms at 16384 keys. Unit-normal caches, which never rescan, pay for the added
-    // tests: 3.52 -> 3.59 ms. (Slack: over ten such caches 3.60 ms on average at 2, 3.85 at 4 (one in
-    // three rescans somewhere), 4.3 at 8; four blocks apart at 2 or 4 3.62, 16 apart 4.2; a test in
-    // one step of every block 3.59-3.63.) The two scans do the same arithmetic
+    // 1.50 -> 0.92 ms at 16384 keys. Unit-normal caches, which never rescan, pay for the added tests and
+    // moves: 3.40 -> 3.50 ms there, 9 x 8 x 256 x 16384 keys 94 -> 98.5 us, 9 x 8 x 300 x 700 24.1 -> 25.8 us.
+    // (Slack: over ten wide-channel caches 3.60 ms on average at 2, 3.85 at 4 (one in three rescans
+    // somewhere), 4.3 at 8; four blocks apart at 2 or 4 3.62, 16 apart 4.2; a test in one step of every
+    // block 3.59-3.63.) The two scans do the same arithmetic
     // otherwise. (The VALU-mode kernels scan once with the test on: at DP 64 the second pass's
     // live state spills inside their loop and costs more than the test.)
     if constexpr (resident(NW)) {

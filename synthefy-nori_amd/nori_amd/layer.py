@@ -1302,9 +1302,11 @@ class EncoderBaseLayer(nn.Module):
     # small layers of the fused widths issue their launches from one native call
     # (nori_dense_apply); False keeps the sublayers' own calls
     native_apply = True
-    # Up to this many tokens. One 6m layer, native against its own calls: 2,304 tokens 116 / 349 us,
-    # 32,768 152 / 271, 65,280 197 / 268, 204,000 592 / 632. Past that the kernels outlast the host,
-    # and the own calls free each operand as they go where the native scratch holds 10 bytes an element.
+    # Up to this many tokens. One layer over 9 to 34 groups, native against its own calls: width 128 2,304
+    # tokens 105 / 283 us, 34,816 185 / 248, 65,280 244 / 259, 204,000 740 / 791, 261,800 905 / 993; width 256
+    # (4 heads, hidden 1024), whose projections the own calls give to the library GEMM, 2,304 tokens
+    # 164 / 290 us, 16,384 287 / 294, 34,816 329 / 339, 204,000 1,606 / 1,799, 261,800 1,988 / 2,273. Past that the
+    # kernels outlast the host by far and the scratch (10 bytes an element) grows past 0.7 GB.
     _NATIVE_TOKENS = 262144
 
     def _apply_native(self, x: torch.Tensor, kv_cache, feature_atten_mask) -> torch.Tensor | None:

@@ -8,7 +8,8 @@ output buffer (``out``), the transposed [table, group, row] view of a cell buffe
 copies. ``linear`` routes to it the shapes where it is the faster of the two (same-box A/B against the
 library GEMM at inner width 128: 139,264 rows x 128 -> 128 in 20 against 26 us, -> 256 in 25.5
 against 28, -> 384 in 32 against 59.5; 655,360 rows 67 against 101, 114 against 126, 157 against 261.
-At inner width 256 the library was level or faster up to 256 columns); everything else (other dtypes, widths or shapes, short operands, CPU
+At inner width 256 neither is ahead throughout: 65,536 rows 256 -> 256 in 21.4 against 18.8 us, 163,840 in
+40.9 against 43.1); everything else (other dtypes, widths or shapes, short operands, CPU
 tensors) is ``F.linear``. The two differ only in the order of the fp32 sums.
 """
 
@@ -22,7 +23,7 @@ from . import _native as nat
 
 __all__ = ["linear", "linear_head_norm", "linear_residual", "linear_residual_norm", "takes_kernel"]
 
-_WIDTHS = (128,)  # inner widths routed to the kernel (it also takes 256, where the library GEMM was faster)
+_WIDTHS = (128,)  # inner widths routed to the kernel (it also takes 256, where neither is ahead throughout)
 _MAX_N = 384      # output widths up to this
 _MIN_ROWS = 4096  # below this the library GEMM's launch is as cheap
 
