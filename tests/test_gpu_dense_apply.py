@@ -147,3 +147,10 @@ def test_parameters_on_another_device_or_of_another_shape_are_refused(cuda):
             assert spoiled._apply_native(x, cache, None) is None, spoil.__name__
             with pytest.raises((RuntimeError, ValueError)):
                 spoiled.forward_test_with_cache(x, {"seq_kv": cache})
+
+
+@pytest.mark.parametrize("shared,quantized", [(False, True), (True, False)])
+def test_native_apply_past_the_split_mlp(cuda, shared, quantized):
+    # 11,700 tokens: the SwiGLU kernel of whole workgroups and projections of several blocks a workgroup
+    test_native_apply_equals_the_layers_calls(cuda, 128, 2, 1, 1300, 9, 300, shared, quantized)
+    test_native_apply_equals_the_layers_calls(cuda, 256, 4, 1, 1300, 9, 300, shared, quantized)

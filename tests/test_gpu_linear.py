@@ -232,9 +232,9 @@ def test_residual_norm_declines_what_it_does_not_take(cuda):
 
 
 def test_two_phase_steps_take_the_fused_pass(cuda, monkeypatch):
-    """A cell layer and a row layer under fp16 autocast: every attention update whose next norm
-    is an fp16 operand goes through the fused kernel, and the result matches the separate
-    projection + residual + norm passes to within the fp16 roundings of the updates (at these
+    """A cell layer and a row layer under fp16 autocast: every update goes through its fused kernel
+    (with the next norm, or without one at a layer's end), and the result matches the separate
+    projection or MLP, residual and norm passes to within the fp16 roundings of the updates (at these
     row counts the separate projection is the library GEMM, which sums in another order)."""
     from nori_amd import two_phase
 
@@ -247,23 +247,30 @@ def test_two_phase_steps_take_the_fused_pass(cuda, monkeypatch):
     targets = torch.randn(3, 96, 2, 128, generator=g, device=cuda)
     memory = torch.randn(3, 96, 4, 256, generator=g, device=cuda).to(torch.float16)
     calls = []
-    fused = projection.linear_residual_norm
+    fused = {name: getattr(two_phase, name) for name in
+             ("linear_residual_norm", "linear_residual", "swiglu_mlp_residual_norm", "swiglu_mlp_residual")}
 
-    def spy(a, *args, **kw):
-        y = fused(a, *args, **kw)
-        calls.append((int(a.shape[-1]), y is not None))
-        return y
+    def spy(name):
+        def call(a, *args, **kw):
+            y = fused[name](a, *args, **kw)
+            calls.append((name, int(a.shape[-1]), y is not None and y is not False))
+            return y
+        return call
 
     def run(take):
-        monkeypatch.setattr(two_phase, "linear_residual_norm", spy if take else (lambda *a, **k: None))
+        for name in fused:  # the fused updates with and without a next norm, or none of them
+            declines = (lambda *a, **k: None) if name.endswith("norm") else (lambda *a, **k: False)
+            monkeypatch.setattr(two_phase, name, spy(name) if take else declines)
         with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
             c, t = layer(cells, targets, 64)
             r = row_layer(t.reshape(3, 96, 256), 64, memory)
         return c, t, r
 
     c1, t1, r1 = run(True)
-    assert calls and all(took for _, took in calls)
-    assert sorted(set(k for k, _ in calls)) == [128, 256]
+    assert calls and all(took for _, _, took in calls)
+    assert sorted(set((name, k) for name, k, _ in calls)) == [
+        ("linear_residual", 128), ("linear_residual", 256), ("linear_residual_norm", 128), ("linear_residual_norm", 256),
+        ("swiglu_mlp_residual", 256), ("swiglu_mlp_residual_norm", 128), ("swiglu_mlp_residual_norm", 256)]
     c0, t0, r0 = run(False)
     for got, ref in ((c1, c0), (t1, t0), (r1, r0)):
         scale = ref.abs().amax()

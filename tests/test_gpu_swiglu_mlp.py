@@ -233,3 +233,11 @@ def test_residual_without_a_norm_equals_the_separate_passes(width, hidden, rows)
     want = residual_add(stream, swiglu_mlp(x, gate_up, down, hp), 0.2)
     assert swiglu_mlp_residual(x, gate_up, down, hp, stream, 0.2)
     assert torch.equal(stream, want) and torch.equal(buf[rows], guard)
+
+
+# At up to 32 rows per CU (8,192 on 256) width 128 runs the kernel whose wavefronts split the hidden units;
+# past that, whole workgroups of 128 rows, the last of them ragged.
+@pytest.mark.parametrize("rows", [8192, 8193, 16385])
+def test_residual_epilogues_around_the_split_rule(rows):
+    test_residual_norm_epilogue_equals_the_separate_kernels(128, 128, 256, rows)
+    test_residual_without_a_norm_equals_the_separate_passes(128, 256, rows)
