@@ -124,6 +124,8 @@ class QASSMaxScaling(nn.Module):
             return False
         if first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None or _hooked(self.base_mlp):
             return False
+        if [type(m) for m in self.base_mlp] != [nn.Linear, nn.GELU, nn.Linear] or self.base_mlp[1].approximate != "none":
+            return False
         params = self._base_weights()
         if torch.is_autocast_enabled("cuda"):  # which casts these dtypes, to its own
             if torch.get_autocast_dtype("cuda") != torch.float16 \

@@ -187,3 +187,21 @@ def test_base_scale_follows_the_dtype_its_linears_compute_in():
     m.base_mlp[-1].float()
     with torch.inference_mode(), pytest.raises(RuntimeError):
         m(q, 300)
+
+
+def test_base_scale_of_other_modules_calls_them():
+    # a layer of another class, or another activation, in the base MLP: the module's own call
+    class Shifted(torch.nn.Linear):
+        def forward(self, x):
+            return super().forward(x) + 1.0
+
+    q = torch.randn(40, 3, 2, 64, generator=torch.Generator().manual_seed(8)).half().to(DEV)
+    for at, other in ((0, Shifted(1, 64)), (1, torch.nn.GELU(approximate="tanh")), (1, torch.nn.Tanh()), (2, Shifted(64, 128))):
+        m = _module(2, 64, seed=9)
+        m.base_mlp[at] = other
+        m = m.to(DEV)
+        with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+            got = m(q, 300)
+            log_n = torch.full((), math.log(300.0), device=DEV, dtype=torch.float16)
+            scale = log_n.view(1, 1, 1, 1) * (1.0 + torch.tanh(m.base_mlp(log_n.view(1, 1)).view(1, 1, 2, 64)))
+            assert torch.equal(got, layer_mod.qass_gate(q, *m._gate_weights(), scale))
