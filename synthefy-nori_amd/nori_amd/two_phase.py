@@ -107,7 +107,7 @@ def _attend_accumulate(attn: MultiheadAttention, atten: torch.Tensor, stream: to
     ``dest``, as ``_linear_accumulate``): ``atten`` the attention output [..., H, D] with ``stream``'s
     leading shape, any row strides."""
     a = atten.reshape(*atten.shape[:-2], -1)
-    w_o = attn._linear_weights(atten.device)[2] if atten.is_cuda else None
+    w_o = attn._linear_weights(atten.device)[2] if atten.is_cuda and type(attn) is MultiheadAttention else None
     if w_o is None:
         return _accumulate(_moved(stream, dest), attn.project_out(atten), alpha, then, operand=operand)
     return _linear_accumulate(a, w_o, stream, alpha, then, lambda: attn.project_out(atten), operand=operand, dest=dest)

@@ -8,7 +8,7 @@ import copy
 import pytest
 import torch
 
-from nori_amd.layer import SwiGLUMLP
+from nori_amd.layer import MultiheadAttention, SwiGLUMLP
 from nori_amd.two_phase import CellLayer2P, RowLayer2P
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +99,17 @@ def test_target_mix_is_read_as_edited(cuda):
     with torch.no_grad():
         fresh.feature_attention.target_mix.weight.mul_(-1.5)
     assert all(torch.equal(a, b) for a, b in zip(_run(layer, call), _run(fresh, call)))
+
+
+def test_another_attention_class_projects_its_own_output(cuda):
+    class Silent(MultiheadAttention):
+        def project_out(self, atten_out):
+            return torch.zeros_like(super().project_out(atten_out))
+
+    for make, path in ((_cell, "feature_attention.feature_attentions.0"), (_row, "feature_attentions.0")):
+        layer, call = make(cuda)
+        zeroed = copy.deepcopy(layer)
+        with torch.no_grad():
+            zeroed.get_submodule(path).out_proj_weight.zero_()
+        layer.get_submodule(path).__class__ = Silent
+        assert all(torch.equal(a, b) for a, b in zip(_run(layer, call), _run(zeroed, call)))
