@@ -35,6 +35,8 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
     if (B <= 0 || R <= 0 || G <= 0 || h <= 0 || e <= 0 || e % h || p->nk <= 1)
         return fail(NORI_ERR_INVALID, "dense_apply: bad shape (%lld x %lld x %lld, %d heads of %d, %lld keys)", (long long)B,
                     (long long)R, (long long)G, h, e, (long long)p->nk);
+    if (p->qkv_dtype != NORI_F16 && p->qkv_dtype != NORI_F32)
+        return fail(NORI_ERR_UNSUPPORTED, "dense_apply: %s q|k|v weights", dtype_name(p->qkv_dtype));
     if (e != 128 && e != 256) return fail(NORI_ERR_UNSUPPORTED, "dense_apply: width %d is not 128 or 256", e);
     const int d = e / h;
     const int64_t need = nori_dense_apply_scratch_bytes(B, R, G, e, h, p->nk);
@@ -51,7 +53,7 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
     const int64_t ws_bytes = p->scratch_bytes - (at - reinterpret_cast<char*>(p->scratch));
     const float scale = p->logit_scale;
     int st;
-#define NORI_STEP(call) if ((st = (call)) != NORI_OK) return st
+#define NORI_STEP(call) do { if ((st = (call)) != NORI_OK) return st; } while (0)
     // sequence attention, in [table, group, row] order
     NORI_STEP(nori_rms_norm_rows(p->x, n, e, G, R, R * G * e, e, G * (int64_t)e, p->eps_seq, a0, NORI_F16, stream));
     NORI_STEP(nori_linear_f16(a0, 1, 1, n, e, 0, 0, e, p->w_q, e, e, a1, 0, 0, e, stream));
@@ -68,7 +70,11 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
     NORI_STEP(nori_swiglu_mlp_residual_rms_norm(a0, NORI_F16, n, e, e, p->gate_up, p->down, p->hidden, p->alpha, p->out, e,
                                                 e, p->eps_feat, a1, n, 0, e, stream));
     // feature attention over each row's groups
-    NORI_STEP(nori_linear_f16(a1, 1, 1, n, e, 0, 0, e, p->w_qkv, e, 3 * e, qkv, 0, 0, 3 * e, stream));
+    if (p->qkv_dtype == NORI_F32)
+        NORI_STEP(nori_linear_f16_w32(a1, 1, 1, n, e, 0, 0, e, reinterpret_cast<const float*>(p->w_qkv), e, 3 * e, qkv, 0, 0,
+                                      3 * e, stream));
+    else
+        NORI_STEP(nori_linear_f16(a1, 1, 1, n, e, 0, 0, e, p->w_qkv, e, 3 * e, qkv, 0, 0, 3 * e, stream));
     const uint16_t* q3 = reinterpret_cast<const uint16_t*>(qkv);
     NORI_STEP(nori_icl_attention(q3, NORI_F16, B * R, G, h, d, 3 * G * e, 3 * e, d, q3 + e, NORI_F16, nullptr, G, h,
                                  3 * G * e, 3 * e, e, 0, 0, 0, scale, a0, NORI_F16, G * e, e, d, nullptr, 0, ws, ws_bytes,

@@ -64,7 +64,7 @@ constexpr int kThreads = kWaves * 64;
 
 struct LinArgs {
     const _Float16* x; int64_t rows, n_mid, n_inner, x_outer, x_mid, x_row;
-    const _Float16* w; int64_t w_row;
+    const void* w; int64_t w_row;  // fp16, or fp32 (W32 kernels)
     int n;
     _Float16* y; int64_t y_outer, y_mid, y_row;
     int nchunks, teams;  // column chunks; workgroups per XCD and chunk
@@ -122,8 +122,11 @@ __device__ __forceinline__ uint4 head_norm8(uint4 v, const float (&w)[8], float 
 
 // NR 16-row tiles per wavefront. A workgroup keeps its column chunk of W in LDS and walks row
 // blocks, loading the next block's x rows before it computes the current one's; the workgroups
-// of a chunk's row blocks and those of the other chunks over the same rows share an XCD.
-template <int KS, int NC, int NR, bool NORM>
+// of a chunk's row blocks and those of the other chunks over the same rows share an XCD. W32: the
+// weights are fp32 and rounded to fp16 as they are staged, the values of a cast; a caller whose
+// parameter is fp32 then launches no cast on each call and keeps none (a layer's cast and the gap around
+// it are 4-5 us, a third of a short layer's projection and more).
+template <int KS, int NC, int NR, bool NORM, bool W32>
 __global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(const LinArgs a) {
     constexpr int PITCH = 32 * KS + 8;  // f16 per staged W row: +16 bytes spreads the 16-row reads over the banks
     constexpr int GC = 64;              // output columns staged per wavefront between stores
@@ -158,7 +161,17 @@ __global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(c
     for (int e = tid; e < NC * KS * 4; e += kThreads) {
         const int r = e / (KS * 4), q = e % (KS * 4);
         uint4 v = {0u, 0u, 0u, 0u};
-        if (c0 + r < a.n) v = *reinterpret_cast<const uint4*>(a.w + (int64_t)(c0 + r) * a.w_row + 8 * q);
+        if (c0 + r < a.n) {
+            const int64_t at = (int64_t)(c0 + r) * a.w_row + 8 * q;
+            if constexpr (W32) {
+                const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(a.w) + at);
+                const f32x4 lo = p[0], hi = p[1];
+                v = uint4{pack_f16_rn(lo[0], lo[1]), pack_f16_rn(lo[2], lo[3]), pack_f16_rn(hi[0], hi[1]),
+                          pack_f16_rn(hi[2], hi[3])};
+            } else {
+                v = *reinterpret_cast<const uint4*>(reinterpret_cast<const _Float16*>(a.w) + at);
+            }
+        }
         *reinterpret_cast<uint4*>(wt + r * PITCH + 8 * q) = v;
     }
     float gain[8];
@@ -229,12 +242,12 @@ __global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(c
     }
 }
 
-template <int KS, int NC, int NR, bool NORM>
+template <int KS, int NC, int NR, bool NORM, bool W32>
 int launch_tiles(LinArgs a, int cus, hipStream_t stream) {
     constexpr int BROWS = kWaves * NR * 16;
     constexpr size_t lds = ((size_t)NC * (32 * KS + 8) + (size_t)BROWS * 72) * sizeof(_Float16);
     static_assert(lds <= 160 * 1024, "a chunk of W and the staged rows fit one workgroup's LDS");
-    if (hipFuncSetAttribute((const void*)linear_f16_kernel<KS, NC, NR, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)linear_f16_kernel<KS, NC, NR, NORM, W32>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)
         return fail(NORI_ERR_RUNTIME, "linear_f16: cannot reserve %zu bytes of LDS", lds);
     a.nchunks = (a.n + NC - 1) / NC;
@@ -247,7 +260,7 @@ int launch_tiles(LinArgs a, int cus, hipStream_t stream) {
     a.teams = (int)((per_xcd + rounds - 1) / rounds);  // no more than share the blocks evenly
     const int64_t grid = 8 * (int64_t)a.teams * a.nchunks;
     if (grid > 0x7fffffffLL) return fail(NORI_ERR_UNSUPPORTED, "linear_f16: %d columns exceed one launch", a.n);
-    hipLaunchKernelGGL((linear_f16_kernel<KS, NC, NR, NORM>), dim3((unsigned)grid), dim3(kThreads), lds, stream, a);
+    hipLaunchKernelGGL((linear_f16_kernel<KS, NC, NR, NORM, W32>), dim3((unsigned)grid), dim3(kThreads), lds, stream, a);
     return launch_status("linear_f16");
 }
 
@@ -258,15 +271,15 @@ int launch_tiles(LinArgs a, int cus, hipStream_t stream) {
 // are ahead: 64 to 4,096 rows, N 256 6.9 - 8.3 -> 4.9 - 6.1 us. Teams share the blocks evenly: 65,536 x 640, K 128:
 // 27.1 -> 26.7 us, N 384 20.1 -> 19.8; and the last block of a workgroup loads no rows after it, which cost
 // calls of about a block each 5 to 10 % (20,000 x 640: 13.9 -> 12.7 us).
-template <int KS, bool NORM>
+template <int KS, bool NORM, bool W32>
 int launch(LinArgs a, hipStream_t stream) {
     const int cus = device_cus();
     const int64_t chunks = (a.n + 127) / 128, blocks = (a.rows + 255) / 256;
-    if (5 * blocks * chunks >= 2 * cus) return launch_tiles<KS, 128, 2, NORM>(a, cus, stream);
+    if (5 * blocks * chunks >= 2 * cus) return launch_tiles<KS, 128, 2, NORM, W32>(a, cus, stream);
     if constexpr (KS == 8) {
-        if (2 * ((a.rows + 127) / 128) * chunks <= cus) return launch_tiles<KS, 64, 1, NORM>(a, cus, stream);
+        if (2 * ((a.rows + 127) / 128) * chunks <= cus) return launch_tiles<KS, 64, 1, NORM, W32>(a, cus, stream);
     }
-    return launch_tiles<KS, 128, 1, NORM>(a, cus, stream);
+    return launch_tiles<KS, 128, 1, NORM, W32>(a, cus, stream);
 }
 
 // ---------------------------------------------------------------- projection + residual + norm
@@ -440,7 +453,7 @@ namespace {
 int run_linear(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k, int64_t x_outer_stride,
                int64_t x_mid_stride, int64_t x_row_stride, const void* weight, int64_t w_row_stride, int32_t n, void* y,
                int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, const void* gain, int gain_dtype,
-               float eps, int32_t norm_cols, void* stream) {
+               float eps, int32_t norm_cols, void* stream, bool w32 = false) {
     clear_error();
     if (n_outer < 0 || n_mid < 0 || n_inner < 0 || k <= 0 || n <= 0)
         return fail(NORI_ERR_INVALID, "linear_f16: bad shape n_outer=%lld n_mid=%lld n_inner=%lld k=%d n=%d",
@@ -454,7 +467,7 @@ int run_linear(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, i
     if (!x || !weight || !y) return fail(NORI_ERR_INVALID, "linear_f16: null pointer");
     // 16-byte x and W row chunks, 8-byte output pieces
     if ((uintptr_t)x % 16 || x_row_stride % 8 || x_mid_stride % 8 || x_outer_stride % 8 || (uintptr_t)weight % 16 ||
-        w_row_stride % 8 || w_row_stride < k || (uintptr_t)y % 8 || y_row_stride % 4 || y_mid_stride % 4 ||
+        w_row_stride % (w32 ? 4 : 8) || w_row_stride < k || (uintptr_t)y % 8 || y_row_stride % 4 || y_mid_stride % 4 ||
         y_outer_stride % 4)
         return fail(NORI_ERR_UNSUPPORTED,
                     "linear_f16: x and weight rows must be 16-byte aligned, output rows 8-byte aligned");
@@ -466,7 +479,7 @@ int run_linear(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, i
     a.x_outer = x_outer_stride;
     a.x_mid = x_mid_stride;
     a.x_row = x_row_stride;
-    a.w = reinterpret_cast<const _Float16*>(weight);
+    a.w = weight;
     a.w_row = w_row_stride;
     a.n = n;
     a.y = reinterpret_cast<_Float16*>(y);
@@ -478,8 +491,9 @@ int run_linear(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, i
     a.eps = eps;
     a.norm_cols = norm_cols;
     hipStream_t s = (hipStream_t)stream;
-    if (norm_cols > 0) return k == 128 ? launch<4, true>(a, s) : launch<8, true>(a, s);
-    return k == 128 ? launch<4, false>(a, s) : launch<8, false>(a, s);
+    if (norm_cols > 0) return k == 128 ? launch<4, true, false>(a, s) : launch<8, true, false>(a, s);
+    if (w32) return k == 128 ? launch<4, false, true>(a, s) : launch<8, false, true>(a, s);
+    return k == 128 ? launch<4, false, false>(a, s) : launch<8, false, false>(a, s);
 }
 
 }  // namespace
@@ -490,6 +504,14 @@ extern "C" int nori_linear_f16(const void* x, int64_t n_outer, int64_t n_mid, in
                                int64_t y_row_stride, void* stream) {
     return run_linear(x, n_outer, n_mid, n_inner, k, x_outer_stride, x_mid_stride, x_row_stride, weight, w_row_stride, n,
                       y, y_outer_stride, y_mid_stride, y_row_stride, nullptr, NORI_F32, 0.f, 0, stream);
+}
+
+extern "C" int nori_linear_f16_w32(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
+                                   int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride,
+                                   const float* weight, int64_t w_row_stride, int32_t n, void* y, int64_t y_outer_stride,
+                                   int64_t y_mid_stride, int64_t y_row_stride, void* stream) {
+    return run_linear(x, n_outer, n_mid, n_inner, k, x_outer_stride, x_mid_stride, x_row_stride, weight, w_row_stride, n,
+                      y, y_outer_stride, y_mid_stride, y_row_stride, nullptr, NORI_F32, 0.f, 0, stream, true);
 }
 
 extern "C" int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,

@@ -10,7 +10,7 @@ extern "C" {
 #endif
 
 // Moves with every change of a signature or struct below; the package binds one version.
-#define NORI_OPS_VERSION 2
+#define NORI_OPS_VERSION 3
 int nori_ops_version(void);
 
 // QASS base scale of one key count (QASSMaxScaling.forward's base branch, src/synthefy_nori/model/
@@ -27,6 +27,12 @@ int nori_qass_base(float log_n, const void* w1, const void* b1, const void* w2, 
 // of 4, 2^31 rows or more and unaligned operands return NORI_ERR_UNSUPPORTED.
 int nori_rms_norm_rows(const float* x, int64_t rows, int32_t cols, int64_t d1, int64_t d2, int64_t s0, int64_t s1,
                        int64_t s2, float eps, void* y, int y_dtype, void* stream);
+
+// nori_linear_f16 of fp32 weights, each rounded to fp16 as it is staged: bit for bit nori_linear_f16 of
+// their fp16 cast. weight 16-byte aligned, its row stride a multiple of 4.
+int nori_linear_f16_w32(const void* x, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k, int64_t x_outer_stride,
+                        int64_t x_mid_stride, int64_t x_row_stride, const float* weight, int64_t w_row_stride, int32_t n,
+                        void* y, int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, void* stream);
 
 // nori_linear_f16 followed by the per-head RMSNorm of its first norm_cols columns, taken as heads
 // of 64 (a multiple of 64): each head row v becomes T(T(v * rsqrt(mean(v^2) + eps)) * gain) with T
@@ -65,7 +71,7 @@ typedef struct {
     float* out;
     const void *w_q, *w_out, *w_qkv, *w_feat_out;
     const void *base_w1, *base_b1, *base_w2, *base_b2, *gate_w1, *gate_b1, *gate_w2, *gate_b2;
-    int32_t base_dtype, qass_hidden;
+    int32_t qkv_dtype, base_dtype, qass_hidden;
     const void *gate_up, *down;
     int32_t hidden;
     float eps_seq, eps_mlp, eps_feat, alpha, logit_scale, log_n;

@@ -121,7 +121,7 @@ class DenseApplyArgs(ctypes.Structure):
         [(n, _i64) for n in ("tables", "rows", "groups")] + [("embed", _i32), ("heads", _i32)]
         + [(n, _vp) for n in ("x", "out", "w_q", "w_out", "w_qkv", "w_feat_out", "base_w1", "base_b1", "base_w2", "base_b2",
                               "gate_w1", "gate_b1", "gate_w2", "gate_b2")]
-        + [("base_dtype", _i32), ("qass_hidden", _i32), ("gate_up", _vp), ("down", _vp), ("hidden", _i32)]
+        + [("qkv_dtype", _i32), ("base_dtype", _i32), ("qass_hidden", _i32), ("gate_up", _vp), ("down", _vp), ("hidden", _i32)]
         + [(n, _f32) for n in ("eps_seq", "eps_mlp", "eps_feat", "alpha", "logit_scale", "log_n")]
         + [("kv", _vp), ("kv_dtype", _i32), ("kv_scales", _vp), ("nk", _i64), ("kv_heads", _i32)]
         + [(n, _i64) for n in ("kv_bg", "kv_row", "kv_half", "sc_bg", "sc_row", "sc_half")]
@@ -130,9 +130,12 @@ class DenseApplyArgs(ctypes.Structure):
 
 
 # The package's own entry points beyond the C ABI (csrc/nori_ops.h), and their version.
-OPS_VERSION = 2
+OPS_VERSION = 3
 OPS: dict[str, tuple[object, list]] = {
     "nori_qass_base": (ctypes.c_int, [_f32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp]),
+    "nori_linear_f16_w32": (
+        ctypes.c_int, [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _i32, _vp, _i64, _i64, _i64, _vp],
+    ),
     "nori_linear_f16_head_norm": (
         ctypes.c_int,
         [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _i32, _vp, _i64, _i64, _i64, _vp, _i32, _f32, _i32, _vp],

@@ -33,6 +33,7 @@ from typing import Optional
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _module_base
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .attention import attend_dense, compute_attention_blockwise, icl_attention, takes_prologue
@@ -40,7 +41,7 @@ from . import _native as nat
 from . import kv_project
 from .kv_cache_scaling import BlockwiseSeqKV, ScalableSeqKV, scale_caches
 from .projection import linear as proj_linear
-from .projection import linear_head_norm, linear_residual, linear_residual_norm
+from .projection import linear_head_norm, linear_param, linear_residual, linear_residual_norm, param_weight
 from .norm import (FUSED_MLP_WIDTHS, QASS_GATE_HIDDEN, RMSNorm, group_major_operand, operand_dtype, projection_operand,
                    qass_base, qass_base_weights, qass_gate, residual_add, residual_add_norm, rms_norm_, silu_mul, swiglu_mlp,
                    swiglu_mlp_residual_norm)
@@ -119,12 +120,14 @@ class QASSMaxScaling(nn.Module):
     def _fused_base_applies(self, q: torch.Tensor) -> bool:
         """The base scale as one HIP launch: where its linears compute in fp16 and no gradient is
         asked for, the 64-wide hidden layer."""
-        first, last = self.base_mlp[0], self.base_mlp[-1]
-        if not (self.fused and q.is_cuda and q.dtype == torch.float16 and first.weight.is_cuda):
+        layers = tuple(self.base_mlp._modules.values())
+        if not (self.fused and q.is_cuda and q.dtype == torch.float16):
             return False
-        if first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None or _hooked(self.base_mlp):
+        if tuple(map(type, layers)) != (nn.Linear, nn.GELU, nn.Linear) or layers[1].approximate != "none":
             return False
-        if [type(m) for m in self.base_mlp] != [nn.Linear, nn.GELU, nn.Linear] or self.base_mlp[1].approximate != "none":
+        first, last = layers[0], layers[2]
+        if not first.weight.is_cuda or first.out_features != QASS_GATE_HIDDEN or first.bias is None or last.bias is None \
+                or _hooked(self.base_mlp):
             return False
         params = self._base_weights()
         if torch.is_autocast_enabled("cuda"):  # which casts these dtypes, to its own
@@ -164,7 +167,7 @@ class QASSMaxScaling(nn.Module):
 
     def _base_weights(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
         """The base MLP's own parameters (w1, b1, w2, b2): the kernel rounds them itself."""
-        first, last = self.base_mlp[0], self.base_mlp[-1]
+        first, _, last = self.base_mlp._modules.values()
         return first.weight, first.bias, last.weight, last.bias
 
     def _gate_weights(self) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -467,13 +470,8 @@ class MultiheadAttention(nn.Module):
 
     def _live_weight(self, first: int, last: int) -> torch.Tensor:
         """Projections ``first`` to ``last - 1`` of (q, k, v) as one F.linear weight
-        [(last - first) * H * D, E], in the dtype autocast casts it to. Cast by each call, on its own
-        stream, from the parameter as it is then: a kept cast misses an edit through ``.data``,
-        which moves neither address nor version, and is not ordered with calls on other streams."""
-        w = self.qkv_proj_weight[first:last].reshape(-1, self.embed_dim)
-        if torch.is_autocast_enabled("cuda") and w.dtype in (torch.float32, torch.float16, torch.bfloat16):
-            w = w.to(torch.get_autocast_dtype("cuda"))
-        return w
+        [(last - first) * H * D, E]: the parameter itself, for ``linear_param``."""
+        return self.qkv_proj_weight[first:last].reshape(-1, self.embed_dim)
 
     def _projects_by_linear(self, x: torch.Tensor) -> bool:
         """Whether a projection of x on the GPU takes the F.linear form for models without q/k norms
@@ -622,7 +620,7 @@ class MultiheadAttention(nn.Module):
         if self.qkv_combined:
             x = x.reshape(-1, *x.shape[-2:])
             if self._projects_by_linear(x):
-                qkv = proj_linear(x, self._live_weight(0, 3))
+                qkv = linear_param(x, self._live_weight(0, 3))
                 qkv = qkv.view(*x.shape[:-1], 3, self.num_heads, self.head_dim)
             else:
                 qkv = torch.einsum("... s, j h d s -> ... j h d", x, self.qkv_proj_weight)
@@ -663,20 +661,21 @@ class MultiheadAttention(nn.Module):
                 return self.attend_projected(normed[0].view(BS, F, self.num_heads, self.head_dim),
                                              normed[1].view(BS, n_kv, 2, self.num_heads, self.head_dim), attn_mask,
                                              normed=True)
-        if use_linear:
-            if kept:
-                w_q, w_kv, _ = self._linear_weights(x.device)
-            else:
-                w = self._live_weight(0, 1 if copy_first_head_kv else 3)
-                w_q, w_kv = w[: self.num_heads * self.head_dim], w[self.num_heads * self.head_dim:]
+        if kept:
+            w_q, w_kv, _ = self._linear_weights(x.device)
             q = proj_linear(x, w_q).view(BS, F, self.num_heads, self.head_dim)
+        elif use_linear:
+            w = param_weight(x, self._live_weight(0, 1 if copy_first_head_kv else 3))
+            w_q, w_kv = w.split((self.embed_dim, w.shape[0] - self.embed_dim))
+            q = linear_param(x, w_q).view(BS, F, self.num_heads, self.head_dim)
         else:
             q = torch.einsum("... s, h d s -> ... h d", x.reshape(BS, F, -1), self.qkv_proj_weight[0])
         kv_w = self.qkv_proj_weight[1:]
         if copy_first_head_kv:
             kv = torch.einsum("... s, j h d s -> ... j h d", x_kv.reshape(BS, n_kv, -1), kv_w[:, :1])
         elif use_linear:
-            kv = proj_linear(x_kv, w_kv).view(BS, n_kv, 2, self.num_heads, self.head_dim)
+            kv = proj_linear(x_kv, w_kv) if kept else linear_param(x_kv, w_kv)
+            kv = kv.view(BS, n_kv, 2, self.num_heads, self.head_dim)
         else:
             kv = torch.einsum("... s, j h d s -> ... j h d", x_kv.reshape(BS, n_kv, -1), kv_w)
         return self.attend_projected(q, kv, attn_mask)
@@ -782,11 +781,17 @@ def _report_sdpa_once() -> None:
 
 def _hooked(*modules: nn.Module) -> bool:
     """Whether a call of any of the modules, or of one inside them, would run a forward hook."""
-    from torch.nn.modules import module as base
-
-    if base._global_forward_hooks or base._global_forward_pre_hooks:
+    if _module_base._global_forward_hooks or _module_base._global_forward_pre_hooks:
         return True
-    return any(m._forward_hooks or m._forward_pre_hooks for top in modules for m in top.modules())
+    left = list(modules)  # (walked by hand: Module.modules() takes several times as long)
+    while left:
+        m = left.pop()
+        if m is None:
+            continue
+        if m._forward_hooks or m._forward_pre_hooks:
+            return True
+        left.extend(m._modules.values())
+    return False
 
 
 class EncoderBaseLayer(nn.Module):
@@ -975,7 +980,7 @@ class EncoderBaseLayer(nn.Module):
             return None
         del operand
         w_out = feat._linear_weights(x.device)[2]
-        qkv = proj_linear(tokens.view(b * r, g, e), feat._live_weight(0, 3)).view(b * r, g, 3, feat.num_heads, feat.head_dim)
+        qkv = linear_param(tokens.view(b * r, g, e), feat._live_weight(0, 3)).view(b * r, g, 3, feat.num_heads, feat.head_dim)
         del tokens
         out = icl_attention(feat._apply_extra_attn_scale(qkv[:, :, 0], g), qkv[:, :, 1:]).view(x.shape)
         if not linear_residual(out, w_out, stream, alpha):
@@ -1328,8 +1333,10 @@ class EncoderBaseLayer(nn.Module):
             return None
         if int(kv_cache.batch) != b or int(kv_cache.groups) != g:
             return None
-        seq = self.sequence_attentions[1 if self.seq_attn_isolated else 0]
-        feat, mlp, norms = self.feature_attentions[0], self.mlp[0], self.layer_norms
+        subs = self._modules  # (module attributes and list items otherwise cost a microsecond each)
+        seq = subs["sequence_attentions"]._modules["1" if self.seq_attn_isolated else "0"]
+        feat, mlp = subs["feature_attentions"]._modules["0"], subs["mlp"]._modules["0"]
+        norms = tuple(subs["layer_norms"]._modules.values())
         qass = seq.qassmax
         if type(seq) is not MultiheadAttention or type(feat) is not MultiheadAttention or type(mlp) is not SwiGLUMLP \
                 or type(qass) is not QASSMaxScaling or qass.qass_mode != "full" or len(norms) != 3:
@@ -1364,7 +1371,9 @@ class EncoderBaseLayer(nn.Module):
             return None
         w_q, _, w_out = seq._linear_weights(x.device)
         w_feat_out, w_qkv = feat._linear_weights(x.device)[2], feat._live_weight(0, 3)
-        if w_qkv.dtype != torch.float16 or not w_qkv.is_contiguous():
+        if w_qkv.dtype == torch.bfloat16:
+            w_qkv = w_qkv.to(torch.float16)
+        if w_qkv.dtype not in (torch.float32, torch.float16) or not w_qkv.is_contiguous():
             return None
         base, gate = qass_base_weights(*qass._base_weights()), qass._gate_weights()
         gate_up, _, down, hidden = mlp._stacked_weights(x, multiple=32)
@@ -1373,9 +1382,11 @@ class EncoderBaseLayer(nn.Module):
         shaped = ((w_q, (e, e)), (w_out, (e, e)), (w_qkv, (3 * e, e)), (w_feat_out, (e, e)), (gate_up, (2 * hidden, e)),
                   (down, (e, hidden)), *zip(base, ((hid, 1), (hid,), (e, hid), (e,))),
                   *zip(gate, ((hid, d), (hid,), (d, hid), (d,))))
-        if any(t.device != x.device or tuple(t.shape) != shape for t, shape in shaped):
-            return None
-        if scales is not None and scales.device != x.device:
+        gpu = x.get_device()
+        for t, shape in shaped:
+            if t.get_device() != gpu or t.shape != shape:
+                return None
+        if scales is not None and scales.get_device() != gpu:
             return None
         lib = nat.lib()
         scratch = torch.empty(lib.nori_dense_apply_scratch_bytes(b, r, g, e, heads, n_keys), dtype=torch.uint8, device=x.device)
@@ -1384,7 +1395,7 @@ class EncoderBaseLayer(nn.Module):
         args = nat.DenseApplyArgs(
             b, r, g, e, heads, x.data_ptr(), out.data_ptr(), w_q.data_ptr(), w_out.data_ptr(), w_qkv.data_ptr(),
             w_feat_out.data_ptr(), *(t.data_ptr() for t in base), *(t.data_ptr() for t in gate),
-            nat.dtype_code(base[0].dtype), QASS_GATE_HIDDEN,
+            nat.dtype_code(w_qkv.dtype), nat.dtype_code(base[0].dtype), QASS_GATE_HIDDEN,
             gate_up.data_ptr(), down.data_ptr(), hidden, *(float(m.eps) for m in norms), self._alpha_value(q16),
             1.0 / math.sqrt(float(d)), math.log(float(n_keys)), payload.data_ptr(), nat.dtype_code(payload.dtype),
             None if payload.dtype != torch.int8 else scales.data_ptr(), n_keys, kv_heads, *payload.stride()[:3], *sc,

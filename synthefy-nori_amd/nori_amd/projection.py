@@ -21,7 +21,8 @@ import torch
 
 from . import _native as nat
 
-__all__ = ["linear", "linear_head_norm", "linear_residual", "linear_residual_norm", "takes_kernel"]
+__all__ = ["linear", "linear_head_norm", "linear_param", "linear_residual", "linear_residual_norm", "param_weight",
+           "takes_kernel"]
 
 _WIDTHS = (128,)  # inner widths routed to the kernel (it also takes 256, where neither is ahead throughout)
 _MAX_N = 384      # output widths up to this
@@ -83,10 +84,12 @@ def _common_grid(*tensors: torch.Tensor) -> tuple | None:
     return (grid,) + tuple(tuple([0] * pad + st[::-1]) for st in strides)
 
 
-def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = False, min_rows: int = _MIN_ROWS) -> bool:
+def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = False, min_rows: int = _MIN_ROWS,
+                 weight_dtype: torch.dtype = torch.float16) -> bool:
     """Whether ``linear(x, weight)`` runs on the HIP kernel (``any_width``: whether the kernel
-    can take the operands at all, whatever the routing rule says)."""
-    if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == torch.float16 and weight.dim() == 2
+    can take the operands at all, whatever the routing rule says; ``weight_dtype`` float32: the one
+    that rounds its weights)."""
+    if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == weight_dtype and weight.dim() == 2
             and weight.device == x.device):  # (F.linear refuses a weight on another device)
         return False
     k = int(x.shape[-1])
@@ -97,7 +100,8 @@ def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = Fal
         return False
     if x.stride(-1) != 1:
         return False
-    if weight.stride(-1) != 1 or weight.stride(0) % 8 or weight.data_ptr() % 16 or x.data_ptr() % 16:
+    if weight.stride(-1) != 1 or weight.stride(0) * weight.element_size() % 16 or weight.data_ptr() % 16 \
+            or x.data_ptr() % 16:
         return False
     if x.numel() // k < min_rows:
         return False
@@ -133,6 +137,41 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor | None = Non
             ctypes.c_void_p(out.data_ptr()), yo, ym, yr, nat.stream_of(x.device),
         ),
         "linear_f16",
+    )
+    return out
+
+
+def param_weight(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``weight``, a parameter or rows of one, as ``linear_param`` takes it for operands like x: itself
+    where the kernel rounds fp32 weights as it stages them (``nori_linear_f16_w32``), else the cast
+    autocast makes, formed by this call. Nothing is kept, so an edit through ``.data``, which moves
+    neither address nor version, reaches the next call, and each call is ordered on its own stream."""
+    if not torch.is_autocast_enabled("cuda") or weight.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        return weight
+    dtype = torch.get_autocast_dtype("cuda")
+    if dtype == torch.float16 and takes_kernel(x, weight, weight_dtype=torch.float32):
+        return weight
+    return weight.to(dtype)
+
+
+def linear_param(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``linear(x, weight)`` as autocast computes it, of a parameter as it is on this call
+    (``param_weight``)."""
+    weight = param_weight(x, weight)
+    if weight.dtype != torch.float32 or x.dtype != torch.float16:
+        return linear(x, weight)
+    n = int(weight.shape[0])
+    out = torch.empty(tuple(x.shape[:-1]) + (n,), dtype=torch.float16, device=x.device)
+    common = _common_grid(x, out)
+    if not torch.is_autocast_enabled("cuda") or common is None:
+        return linear(x, weight)
+    (no, nm, ni), sx, sy = common
+    nat.check(
+        nat.lib().nori_linear_f16_w32(
+            x.data_ptr(), no, nm, ni, int(x.shape[-1]), *sx, weight.data_ptr(), int(weight.stride(0)), n, out.data_ptr(),
+            *sy, nat.stream_of(x.device),
+        ),
+        "linear_f16_w32",
     )
     return out
 

@@ -351,3 +351,24 @@ def test_tiles_at_their_rules_edges(cuda, k, rows, n):
     want = (x.double() @ w.double().t()).half()
     assert torch.equal(buf[1:-1], want) and torch.equal(kernel_linear(x, w), want)
     assert bool((buf[0] == 7.0).all()) and bool((buf[-1] == 7.0).all())
+
+
+@pytest.mark.parametrize("k", [128, 256])
+@pytest.mark.parametrize("rows,n", [(1, 4), (129, 260), (6500, 384), (40000, 132)])
+def test_fp32_weights_are_rounded_as_a_cast_rounds_them(cuda, k, rows, n):
+    # nori_linear_f16_w32: bit for bit the kernel on the fp16 cast, weights from the fp16 subnormals up
+    # and off the fp16 grid, rows of a wider weight
+    g = torch.Generator(device=cuda).manual_seed(rows + n + k)
+    x = torch.randn(rows, k, generator=g, device=cuda).half()
+    wide = torch.randn(n, k + 4, generator=g, device=cuda) * torch.exp2(torch.randint(-24, 2, (n, k + 4), generator=g, device=cuda))
+    for w in (wide[:, :k].contiguous(), wide[:, :k]):
+        y = torch.empty(rows, n, dtype=torch.float16, device=cuda)
+        nat.check(nat.lib().nori_linear_f16_w32(x.data_ptr(), 1, 1, rows, k, 0, 0, k, w.data_ptr(), w.stride(0), n,
+                                                y.data_ptr(), 0, 0, n, nat.stream_of(x.device)), "linear_f16_w32")
+        cast = w.half().contiguous()
+        assert torch.equal(y, kernel_linear(x, cast))
+        with torch.inference_mode(), torch.autocast("cuda", dtype=torch.float16):
+            assert torch.equal(projection.linear_param(x, w), projection.linear(x, cast))
+            # strides and bytes the kernel does not take: the cast
+            odd = torch.zeros(n * k + 1, device=cuda)[1:].view(n, k).copy_(w)
+            assert torch.equal(projection.linear_param(x, odd), projection.linear(x, cast))
