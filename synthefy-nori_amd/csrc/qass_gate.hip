@@ -233,35 +233,41 @@ qass_gate_kernel(const uint16_t* q, int64_t rows, int heads, int d, int64_t qs, 
     }
 }
 
-// The base scale: one output per thread. Every workgroup forms the 64 hidden units anew (one erf a
+// The base scale: 64 outputs a workgroup. Every workgroup forms the 64 hidden units anew (a GELU a
 // lane) rather than pass them through memory, and takes its 64 rows of w2 through LDS: element loads,
-// so that weights of any alignment are taken (a parameter may be a view into a flat buffer), each
-// 64 consecutive elements of the wavefront. Weights are rounded to fp16 here, as autocast casts them, so
-// the caller passes the parameters themselves: no cast to keep or to launch. As torch ops this vector of a few hundred values
-// took eleven launches a layer (fill, two GEMMs with their bias copies, GELU, tanh, add, multiply,
-// weight casts), 37 us of device time and three times that on the host; as one kernel about 3 us.
+// so that weights of any alignment are taken (a parameter may be a view into a flat buffer), 16 a thread
+// in flight at once (the index clamped: under a condition each waits for the last, 19-28 us). Weights are
+// rounded to fp16 here, as autocast casts them, so the caller passes the parameters themselves: no cast to
+// keep or to launch. As torch ops this vector of a few hundred values took eleven launches a layer (fill,
+// two GEMMs with their bias copies, GELU, tanh, add, multiply, weight casts), 37 us of device time and
+// three times that on the host; as one kernel about 3 us.
+constexpr int kBaseThreads = 256;
+
 template <int WT>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(kBaseThreads)
 qass_base_kernel(float log_n, const void* w1, const void* b1, const void* w2, const void* b2, int n_out, uint16_t* out) {
     __shared__ float hid[kHid];
     __shared__ float wt[64][kHid + 1];
+    constexpr int PER = 64 * kHid / kBaseThreads;
     const int tid = threadIdx.x, o0 = blockIdx.x * 64, o = o0 + tid;
-    auto cast = [](const void* p, int64_t i) { return r16(load_elem<WT>(p, i)); };
     const int64_t first = (int64_t)o0 * kHid;
     const int left = min(64, n_out - o0) * kHid;  // elements of this workgroup's rows
-    float w[kHid];
+    const int hu = tid % kHid;
+    const float u = load_elem<WT>(w1, hu), c = load_elem<WT>(b1, hu), bias = load_elem<WT>(b2, min(o0 + hu, n_out - 1));
+    float w[PER];
 #pragma unroll
-    for (int i = 0; i < kHid; ++i) w[i] = kHid * i + tid < left ? cast(w2, first + kHid * i + tid) : 0.0f;
+    for (int i = 0; i < PER; ++i) w[i] = load_elem<WT>(w2, first + min(kBaseThreads * i + tid, left - 1));
+    __builtin_amdgcn_sched_barrier(0);  // every load issued before the first is used
     const float l = r16(log_n);
-    hid[tid] = r16(gelu(r16(cast(w1, tid) * l + cast(b1, tid))));
+    if (tid < kHid) hid[tid] = r16(gelu(r16(r16(u) * l + r16(c))));
 #pragma unroll
-    for (int i = 0; i < kHid; ++i) wt[i][tid] = w[i];
+    for (int i = 0; i < PER; ++i) wt[(kBaseThreads * i + tid) / kHid][(kBaseThreads * i + tid) % kHid] = r16(w[i]);
     __syncthreads();
-    if (o >= n_out) return;
+    if (tid >= 64 || o >= n_out) return;
     float acc = 0.0f;
 #pragma unroll
     for (int j = 0; j < kHid; ++j) acc = fmaf(wt[tid][j], hid[j], acc);
-    const float delta = r16(acc + cast(b2, o));
+    const float delta = r16(acc + r16(bias));
     out[o] = f32_to_f16(l * r16(1.0f + r16(tanh_f32(delta))));
 }
 
@@ -322,7 +328,7 @@ extern "C" int nori_qass_base(float log_n, const void* w1, const void* b1, const
         return fail(NORI_ERR_UNSUPPORTED, "qass_base: unsupported weight dtype %s", dtype_name(w_dtype));
     if (n_out <= 0) return fail(NORI_ERR_INVALID, "qass_base: %d outputs", n_out);
     if (!w1 || !b1 || !w2 || !b2 || !out) return fail(NORI_ERR_INVALID, "qass_base: null pointer");
-    const dim3 grid((unsigned)((n_out + 63) / 64)), block(64);
+    const dim3 grid((unsigned)((n_out + 63) / 64)), block(kBaseThreads);
     hipStream_t stream = (hipStream_t)stream_v;
     auto o = reinterpret_cast<uint16_t*>(out);
     if (w_dtype == NORI_F32)

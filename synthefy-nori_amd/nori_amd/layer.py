@@ -686,16 +686,18 @@ class MultiheadAttention(nn.Module):
         are watched by hooks or are other modules)."""
         if not (self.qk_norm and self.head_dim == 64 and self._projects_by_linear(x)):
             return None
-        if type(self.q_norm) is not RMSNorm or type(self.k_norm) is not RMSNorm or _hooked(self.q_norm, self.k_norm):
+        q_norm, k_norm = self.q_norm, self.k_norm
+        if type(q_norm) is not RMSNorm or type(k_norm) is not RMSNorm or _hooked(q_norm, k_norm):
             return None
-        if self.q_norm.weight is None or self.k_norm.weight is None:
+        q_gain, k_gain = q_norm.weight, k_norm.weight
+        if q_gain is None or k_gain is None:
             return None
         w_q, w_kv, _ = self._linear_weights(x.device)
         width = self.num_heads * self.head_dim
-        q = linear_head_norm(x, w_q, self.q_norm.weight, self.q_norm.eps, width)
+        q = linear_head_norm(x, w_q, q_gain, q_norm.eps, width)
         if q is None:
             return None
-        kv = linear_head_norm(x_kv, w_kv, self.k_norm.weight, self.k_norm.eps, width)
+        kv = linear_head_norm(x_kv, w_kv, k_gain, k_norm.eps, width)
         return None if kv is None else (q, kv)
 
     def attend_projected(self, q: torch.Tensor, kv: torch.Tensor, attn_mask: torch.Tensor | None = None, *,

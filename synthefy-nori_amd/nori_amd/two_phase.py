@@ -249,7 +249,7 @@ class DecoupledFeatureAttention(nn.Module):
     def mix_weight(self, dtype: torch.dtype) -> torch.Tensor:
         """``target_mix``'s weight in ``dtype`` (the projection dtype), cast by each call: an edit through
         ``.data``, which moves neither its address nor its version, reaches the next one."""
-        return self.target_mix.weight.detach().to(dtype).contiguous()
+        return self.target_mix.weight.to(dtype)
 
     def attend(self, tokens: torch.Tensor, n_cells: int) -> tuple[torch.Tensor, torch.Tensor]:
         """``forward`` before the cells' output projection and ``target_mix``: (the cell
@@ -378,7 +378,8 @@ class CellLayer2P(nn.Module):
         del tokens
         cell_norm, row_norm, operand = (None, None, True) if then is None else then
         cell_next = _attend_accumulate(fa.feature_attentions[0], cell_out, cells, alpha, cell_norm, operand=operand)
-        plain_mix = type(fa.target_mix) is nn.Linear and fa.target_mix.bias is None and not _hooked(fa.target_mix)
+        mixer = fa.target_mix
+        plain_mix = type(mixer) is nn.Linear and mixer.bias is None and not _hooked(mixer)
         mix = fa.mix_weight(readout.dtype) if readout.is_cuda and plain_mix else None
         row_next = _linear_accumulate(readout, mix, rows, alpha, row_norm, lambda: fa.target_mix(readout),
                                       operand=operand) if mix is not None else \
