@@ -19,9 +19,11 @@
 // double-buffered ring, the next chunk's loads in flight while the current chunk computes; one
 // barrier per chunk.
 //
-// What bounds it: an LDS read of a weight operand serves one 32-cycle MFMA of one wavefront, so the
-// LDS pipe and the matrix pipe of a CU are equally loaded (width 128: HBM as well, 8 to 20 bytes
-// an element of x). Chunks of 32 on 32x32x16 MFMAs took 32 registers for G^T and U^T, which left one
+// What bounds it: no one pipe. An LDS read of a weight operand serves one 32-cycle MFMA of one wavefront,
+// and the gate and the epilogue are VALU work. Counters, as shares of the kernel's cycles: width 128 (655,360
+// rows) MFMA 36 %, VALU issue 52 %, LDS issue 30 %, bank conflicts 14 %, with the residual epilogue 24, 50, 24 and
+// 9 % at 3 TB/s; width 256 with it (163,840 rows, hidden 704) 36, 35, 24 and 13 %; width 352, one wavefront per
+// SIMD, 19, 13, 11 and 7 %: latency. Chunks of 32 on 32x32x16 MFMAs took 32 registers for G^T and U^T, which left one
 // wavefront per SIMD at width 256 (one workgroup of 108 KB), each operand read just before its
 // MFMA: 163,840 rows of 256 (hidden 704) 315 us plain and 380 us with the residual epilogue, against
 // 210 us (845 TFLOP/s) and 246 us; 655,360 rows of 128 (256) 262 and 362 against 220 and 291 us
