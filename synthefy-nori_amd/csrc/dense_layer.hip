@@ -65,7 +65,7 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
                                  p->kv_heads, p->kv_bg, p->kv_row, p->kv_half, p->sc_bg, p->sc_row, p->sc_half, scale, a1,
                                  NORI_F16, R * e, e, d, nullptr, 0, ws, ws_bytes, stream));
     // x + alpha u into the new stream, then the MLP with its residual, each with the next norm
-    NORI_STEP(nori_linear_f16_residual(a1, B, R, G, e, R * G * e, e, R * (int64_t)e, p->w_out, e, p->alpha, p->x, R * G * e,
+    NORI_STEP(nori_linear_f16_residual(a1, B, R, G, e, R * G * e, e, R * (int64_t)e, p->w_out, e, NORI_F16, p->alpha, p->x, R * G * e,
                                        G * (int64_t)e, e, p->out, p->eps_mlp, a0, R * G * e, G * (int64_t)e, e, stream));
     NORI_STEP(nori_swiglu_mlp_residual_rms_norm(a0, NORI_F16, n, e, e, p->gate_up, p->down, p->hidden, p->alpha, p->out, e,
                                                 e, p->eps_feat, a1, n, 0, e, stream));
@@ -79,7 +79,7 @@ extern "C" int nori_dense_apply(const nori_dense_apply_args* p, void* stream) {
     NORI_STEP(nori_icl_attention(q3, NORI_F16, B * R, G, h, d, 3 * G * e, 3 * e, d, q3 + e, NORI_F16, nullptr, G, h,
                                  3 * G * e, 3 * e, e, 0, 0, 0, scale, a0, NORI_F16, G * e, e, d, nullptr, 0, ws, ws_bytes,
                                  stream));
-    NORI_STEP(nori_linear_f16_residual(a0, 1, 1, n, e, 0, 0, e, p->w_feat_out, e, p->alpha, p->out, 0, 0, e, p->out, 0.f,
+    NORI_STEP(nori_linear_f16_residual(a0, 1, 1, n, e, 0, 0, e, p->w_feat_out, e, NORI_F16, p->alpha, p->out, 0, 0, e, p->out, 0.f,
                                        nullptr, 0, 0, 0, stream));
 #undef NORI_STEP
     return NORI_OK;

@@ -92,6 +92,18 @@ __device__ __forceinline__ uint32_t pack_f16_rn(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, f16x2{(_Float16)lo, (_Float16)hi});
 }
 
+// 8 consecutive weights from element at, as fp16: fp16 as they lie, or fp32 rounded (the values of a cast)
+template <bool W32>
+__device__ __forceinline__ uint4 weight8(const void* w, int64_t at) {
+    if constexpr (W32) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(w) + at);
+        const f32x4 lo = p[0], hi = p[1];
+        return uint4{pack_f16_rn(lo[0], lo[1]), pack_f16_rn(lo[2], lo[3]), pack_f16_rn(hi[0], hi[1]),
+                     pack_f16_rn(hi[2], hi[3])};
+    }
+    return *reinterpret_cast<const uint4*>(reinterpret_cast<const _Float16*>(w) + at);
+}
+
 // sum over the 8 lanes of a store row (DPP: lane ^ 1, lane ^ 2, the other quad of 8)
 __device__ __forceinline__ float sum8(float v) {
     v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, false));
@@ -161,17 +173,7 @@ __global__ void __launch_bounds__(kThreads, KS == 4 ? 4 : 2) linear_f16_kernel(c
     for (int e = tid; e < NC * KS * 4; e += kThreads) {
         const int r = e / (KS * 4), q = e % (KS * 4);
         uint4 v = {0u, 0u, 0u, 0u};
-        if (c0 + r < a.n) {
-            const int64_t at = (int64_t)(c0 + r) * a.w_row + 8 * q;
-            if constexpr (W32) {
-                const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(a.w) + at);
-                const f32x4 lo = p[0], hi = p[1];
-                v = uint4{pack_f16_rn(lo[0], lo[1]), pack_f16_rn(lo[2], lo[3]), pack_f16_rn(hi[0], hi[1]),
-                          pack_f16_rn(hi[2], hi[3])};
-            } else {
-                v = *reinterpret_cast<const uint4*>(reinterpret_cast<const _Float16*>(a.w) + at);
-            }
-        }
+        if (c0 + r < a.n) v = weight8<W32>(a.w, (int64_t)(c0 + r) * a.w_row + 8 * q);
         *reinterpret_cast<uint4*>(wt + r * PITCH + 8 * q) = v;
     }
     float gain[8];
@@ -286,7 +288,7 @@ int launch(LinArgs a, hipStream_t stream) {
 
 struct ResArgs {
     const _Float16* a; int64_t rows, n_mid, n_inner, a_outer, a_mid, a_row;
-    const _Float16* w; int64_t w_row;
+    const void* w; int64_t w_row;  // fp16, or fp32 (W32 kernels, rounded as they are staged)
     const float* x; int64_t x_outer, x_mid, x_row;
     float* xo;    // the updated stream, at x's strides (may be x)
     _Float16* y;  // null: no norm
@@ -303,7 +305,7 @@ struct ResArgs {
 // consecutive elements each), so stream rows move 256 contiguous bytes per row and
 // instruction and output rows 128. Lane l handles tile rows 4 p + l / 16 (p = 0..3) at
 // columns 64 q + 4 (l % 16) for every chunk q: its chunk index in the row is 16 q + l % 16.
-template <int KS, int WAVES>
+template <int KS, int WAVES, bool W32>
 __global__ void __launch_bounds__(WAVES * 64, KS == 4 ? 4 : 2) linear_residual_norm_kernel(const ResArgs a) {
     constexpr int K = 32 * KS, PITCH = K + 8;
     constexpr int kBlockRows = WAVES * 16;
@@ -315,8 +317,7 @@ __global__ void __launch_bounds__(WAVES * 64, KS == 4 ? 4 : 2) linear_residual_n
 
     for (int e = tid; e < K * (K / 8); e += WAVES * 64) {
         const int r = e / (K / 8), q = e % (K / 8);
-        *reinterpret_cast<uint4*>(wt + r * PITCH + 8 * q) =
-            *reinterpret_cast<const uint4*>(a.w + (int64_t)r * a.w_row + 8 * q);
+        *reinterpret_cast<uint4*>(wt + r * PITCH + 8 * q) = weight8<W32>(a.w, (int64_t)r * a.w_row + 8 * q);
     }
     const _Float16* wa = wt + (lane & 15) * PITCH + 8 * g;
     _Float16* ut = wt + K * PITCH + wave * 16 * UP;
@@ -428,20 +429,20 @@ __global__ void __launch_bounds__(WAVES * 64, KS == 4 ? 4 : 2) linear_residual_n
     }
 }
 
-template <int KS, int WAVES>
+template <int KS, int WAVES, bool W32>
 int launch_residual(ResArgs a, hipStream_t stream) {
     constexpr int K = 32 * KS;
     constexpr size_t lds = ((size_t)K * (K + 8) + (size_t)WAVES * 16 * 72) * sizeof(_Float16);
     constexpr int kBlockRows = WAVES * 16;
     static_assert(lds <= 160 * 1024, "W must fit one workgroup's LDS");
-    if (hipFuncSetAttribute((const void*)linear_residual_norm_kernel<KS, WAVES>,
+    if (hipFuncSetAttribute((const void*)linear_residual_norm_kernel<KS, WAVES, W32>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return fail(NORI_ERR_RUNTIME, "linear_f16_residual_rms_norm: cannot reserve %zu bytes of LDS", lds);
     a.nblocks = (a.rows + kBlockRows - 1) / kBlockRows;
     // resident workgroups per CU: LDS-bound, and at most 16 wavefronts per CU
     const int per_cu = std::max(1, (int)std::min<size_t>(160 * 1024 / lds, 16 / WAVES));
     const int64_t grid = std::min<int64_t>(a.nblocks, (int64_t)device_cus() * per_cu);
-    hipLaunchKernelGGL((linear_residual_norm_kernel<KS, WAVES>), dim3((unsigned)grid), dim3(WAVES * 64), lds,
+    hipLaunchKernelGGL((linear_residual_norm_kernel<KS, WAVES, W32>), dim3((unsigned)grid), dim3(WAVES * 64), lds,
                        stream, a);
     return launch_status("linear_f16_residual_rms_norm");
 }
@@ -535,7 +536,7 @@ extern "C" int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t
 namespace {
 
 int run_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k, int64_t a_outer_stride,
-                 int64_t a_mid_stride, int64_t a_row_stride, const void* weight, int64_t w_row_stride, float alpha,
+                 int64_t a_mid_stride, int64_t a_row_stride, const void* weight, int64_t w_row_stride, bool w32, float alpha,
                  const float* x, int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, float* x_out,
                  float eps, void* y, int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, void* stream) {
     clear_error();
@@ -551,7 +552,7 @@ int run_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner,
     if (!a || !weight || !x || !x_out) return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: null pointer");
     // 16-byte operand and weight chunks, 16-byte pieces of x, 8-byte pieces of y
     if ((uintptr_t)a % 16 || a_row_stride % 8 || a_mid_stride % 8 || a_outer_stride % 8 || (uintptr_t)weight % 16 ||
-        w_row_stride % 8 || w_row_stride < k || (uintptr_t)x % 16 || (uintptr_t)x_out % 16 || x_row_stride % 4 || x_mid_stride % 4 ||
+        w_row_stride % (w32 ? 4 : 8) || w_row_stride < k || (uintptr_t)x % 16 || (uintptr_t)x_out % 16 || x_row_stride % 4 || x_mid_stride % 4 ||
         x_outer_stride % 4 || (uintptr_t)y % 8 || y_row_stride % 4 || y_mid_stride % 4 || y_outer_stride % 4)
         return fail(NORI_ERR_UNSUPPORTED, "linear_f16_residual_rms_norm: operand and weight rows must be 16-byte "
                     "aligned, stream rows 16-byte aligned, output rows 8-byte aligned");
@@ -563,7 +564,7 @@ int run_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner,
     r.a_outer = a_outer_stride;
     r.a_mid = a_mid_stride;
     r.a_row = a_row_stride;
-    r.w = reinterpret_cast<const _Float16*>(weight);
+    r.w = weight;
     r.w_row = w_row_stride;
     r.x = x;
     r.xo = x_out;
@@ -577,7 +578,8 @@ int run_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner,
     r.alpha = alpha;
     r.eps = eps;
     hipStream_t s = (hipStream_t)stream;
-    return k == 128 ? launch_residual<4, 8>(r, s) : launch_residual<8, 8>(r, s);
+    if (w32) return k == 128 ? launch_residual<4, 8, true>(r, s) : launch_residual<8, 8, true>(r, s);
+    return k == 128 ? launch_residual<4, 8, false>(r, s) : launch_residual<8, 8, false>(r, s);
 }
 
 }  // namespace
@@ -593,17 +595,21 @@ extern "C" int nori_linear_f16_residual_rms_norm(const void* a, int64_t n_outer,
         return fail(NORI_ERR_INVALID, "linear_f16_residual_rms_norm: null pointer");
     }
     return run_residual(a, n_outer, n_mid, n_inner, k, a_outer_stride, a_mid_stride, a_row_stride, weight, w_row_stride,
-                        alpha, x, x_outer_stride, x_mid_stride, x_row_stride, x, eps, y, y_outer_stride, y_mid_stride,
+                        false, alpha, x, x_outer_stride, x_mid_stride, x_row_stride, x, eps, y, y_outer_stride, y_mid_stride,
                         y_row_stride, stream);
 }
 
 extern "C" int nori_linear_f16_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
                                         int64_t a_outer_stride, int64_t a_mid_stride, int64_t a_row_stride,
-                                        const void* weight, int64_t w_row_stride, float alpha, const float* x,
+                                        const void* weight, int64_t w_row_stride, int w_dtype, float alpha, const float* x,
                                         int64_t x_outer_stride, int64_t x_mid_stride, int64_t x_row_stride, float* x_out,
                                         float eps, void* y, int64_t y_outer_stride, int64_t y_mid_stride,
                                         int64_t y_row_stride, void* stream) {
+    if (w_dtype != NORI_F16 && w_dtype != NORI_F32) {
+        clear_error();
+        return fail(NORI_ERR_UNSUPPORTED, "linear_f16_residual: %s weights", dtype_name(w_dtype));
+    }
     return run_residual(a, n_outer, n_mid, n_inner, k, a_outer_stride, a_mid_stride, a_row_stride, weight, w_row_stride,
-                        alpha, x, x_outer_stride, x_mid_stride, x_row_stride, x_out, eps, y, y_outer_stride, y_mid_stride,
+                        w_dtype == NORI_F32, alpha, x, x_outer_stride, x_mid_stride, x_row_stride, x_out, eps, y, y_outer_stride, y_mid_stride,
                         y_row_stride, stream);
 }

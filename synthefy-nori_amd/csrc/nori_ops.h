@@ -10,7 +10,7 @@ extern "C" {
 #endif
 
 // Moves with every change of a signature or struct below; the package binds one version.
-#define NORI_OPS_VERSION 3
+#define NORI_OPS_VERSION 4
 int nori_ops_version(void);
 
 // QASS base scale of one key count (QASSMaxScaling.forward's base branch, src/synthefy_nori/model/
@@ -45,10 +45,10 @@ int nori_linear_f16_head_norm(const void* x, int64_t n_outer, int64_t n_mid, int
                               void* stream);
 
 // nori_linear_f16_residual_rms_norm with the updated stream written to x_out, at x's strides (x_out may
-// be x), and with y NULL without the norm.
+// be x), with y NULL without the norm, and of fp16 or fp32 weights (w_dtype; fp32 as nori_linear_f16_w32).
 int nori_linear_f16_residual(const void* a, int64_t n_outer, int64_t n_mid, int64_t n_inner, int32_t k,
                              int64_t a_outer_stride, int64_t a_mid_stride, int64_t a_row_stride, const void* weight,
-                             int64_t w_row_stride, float alpha, const float* x, int64_t x_outer_stride,
+                             int64_t w_row_stride, int w_dtype, float alpha, const float* x, int64_t x_outer_stride,
                              int64_t x_mid_stride, int64_t x_row_stride, float* x_out, float eps, void* y,
                              int64_t y_outer_stride, int64_t y_mid_stride, int64_t y_row_stride, void* stream);
 

@@ -130,7 +130,7 @@ class DenseApplyArgs(ctypes.Structure):
 
 
 # The package's own entry points beyond the C ABI (csrc/nori_ops.h), and their version.
-OPS_VERSION = 3
+OPS_VERSION = 4
 OPS: dict[str, tuple[object, list]] = {
     "nori_qass_base": (ctypes.c_int, [_f32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp]),
     "nori_linear_f16_w32": (
@@ -142,7 +142,7 @@ OPS: dict[str, tuple[object, list]] = {
     ),
     "nori_linear_f16_residual": (
         ctypes.c_int,
-        [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _f32, _vp, _i64, _i64, _i64, _vp, _f32, _vp, _i64, _i64,
+        [_vp, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _vp, _i64, _i32, _f32, _vp, _i64, _i64, _i64, _vp, _f32, _vp, _i64, _i64,
          _i64, _vp],
     ),
     "nori_swiglu_mlp_residual": (ctypes.c_int, [_vp, _i64, _i32, _i64, _vp, _vp, _i32, _f32, _vp, _i64, _vp]),

@@ -90,7 +90,7 @@ def takes_kernel(x: torch.Tensor, weight: torch.Tensor, *, any_width: bool = Fal
     can take the operands at all, whatever the routing rule says; ``weight_dtype`` float32: the one
     that rounds its weights)."""
     if not (x.is_cuda and x.dtype == torch.float16 and weight.dtype == weight_dtype and weight.dim() == 2
-            and weight.device == x.device):  # (F.linear refuses a weight on another device)
+            and weight.get_device() == x.get_device()):  # (F.linear refuses a weight on another device)
         return False
     k = int(x.shape[-1])
     widths = (128, 256) if any_width else _WIDTHS
@@ -208,7 +208,7 @@ def linear_residual_norm(a: torch.Tensor, weight: torch.Tensor, stream: torch.Te
     """``stream += alpha * F.linear(a, weight)`` in place, then the RMSNorm (no weight, ``eps``)
     of the updated stream rows in fp16, in one kernel (``nori_linear_f16_residual_rms_norm``):
     bit for bit ``linear`` followed by the fused residual + norm pass. ``a`` [..., K] fp16,
-    ``weight`` [K, K] fp16 (K 128 or 256), ``stream`` [..., K] fp32 with ``a``'s leading shape
+    ``weight`` [K, K] fp16, or fp32 rounded to fp16 as it is read (K 128 or 256), ``stream`` [..., K] fp32 with ``a``'s leading shape
     (any row strides: e.g. the [table, row, group] cells beside an attention output in
     [table, group, row] order), ``out`` the same shape in fp16 (new and laid out like
     ``stream`` when None). ``dest`` (``stream``'s shape and strides) takes the sum in ``stream``'s
@@ -231,7 +231,7 @@ def linear_residual(a: torch.Tensor, weight: torch.Tensor, stream: torch.Tensor,
 
 def _linear_residual(a, weight, stream, alpha, eps, out, dest) -> bool:
     k = int(a.shape[-1])
-    if not (a.is_cuda and a.dtype == torch.float16 and weight.dtype == torch.float16 and stream.dtype == torch.float32
+    if not (a.is_cuda and a.dtype == torch.float16 and weight.dtype in (torch.float16, torch.float32) and stream.dtype == torch.float32
             and k in (128, 256) and tuple(weight.shape) == (k, k) and tuple(stream.shape) == tuple(a.shape)
             and stream.device == a.device and weight.device == a.device):
         return False
@@ -247,14 +247,16 @@ def _linear_residual(a, weight, stream, alpha, eps, out, dest) -> bool:
         return False
     (no, nm, ni), sa, sx = common[:3]
     sy = (0, 0, 0) if out is None else common[3]
-    if (a.data_ptr() % 16 or any(st % 8 for st in sa) or weight.data_ptr() % 16 or weight.stride(0) % 8
-            or stream.data_ptr() % 16 or dest.data_ptr() % 16 or any(st % 4 for st in sx)
+    if (a.data_ptr() % 16 or any(st % 8 for st in sa) or weight.data_ptr() % 16
+            or weight.stride(0) * weight.element_size() % 16 or stream.data_ptr() % 16 or dest.data_ptr() % 16 or any(st % 4 for st in sx)
             or (out is not None and (out.data_ptr() % 8 or any(st % 4 for st in sy)))):
         return False
-    head = (a.data_ptr(), no, nm, ni, k, *sa, weight.data_ptr(), int(weight.stride(0)), float(alpha), stream.data_ptr(), *sx)
+    head = (a.data_ptr(), no, nm, ni, k, *sa, weight.data_ptr(), int(weight.stride(0)))
+    update = (float(alpha), stream.data_ptr(), *sx)
     tail = (float(eps), nat.ptr(out), *sy, nat.stream_of(a.device))
-    if out is not None and dest is stream:
-        nat.check(nat.lib().nori_linear_f16_residual_rms_norm(*head, *tail), "linear_f16_residual_rms_norm")
+    if out is not None and dest is stream and weight.dtype == torch.float16:
+        nat.check(nat.lib().nori_linear_f16_residual_rms_norm(*head, *update, *tail), "linear_f16_residual_rms_norm")
     else:
-        nat.check(nat.lib().nori_linear_f16_residual(*head, dest.data_ptr(), *tail), "linear_f16_residual")
+        nat.check(nat.lib().nori_linear_f16_residual(*head, nat.dtype_code(weight.dtype), *update, dest.data_ptr(), *tail),
+                  "linear_f16_residual")
     return True

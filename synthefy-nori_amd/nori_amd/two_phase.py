@@ -80,11 +80,11 @@ def _linear_accumulate(a: torch.Tensor, weight: torch.Tensor, stream: torch.Tens
                        dest: torch.Tensor | None = None) -> torch.Tensor | None:
     """``_accumulate(stream, project(), alpha, then, ...)`` where ``project()`` is ``F.linear(a,
     weight)`` under fp16 autocast: ``a`` [..., K] with ``stream``'s leading shape (any row
-    strides), ``weight`` [K, K] in the projection dtype. The projection, the residual update and
+    strides), ``weight`` [K, K] fp16, or fp32 to be rounded to it. The projection, the residual update and
     the next norm, when it is formed in the fp16 operand dtype, run as one kernel
     (``linear_residual_norm``, ``linear_residual``: u never reaches memory) wherever it takes the
     operands. ``dest`` (laid out like ``stream``) takes the sum, and ``stream`` is left as it is."""
-    if a.is_cuda and operand_dtype(stream) == torch.float16 and weight.dtype == torch.float16:
+    if a.is_cuda and operand_dtype(stream) == torch.float16 and weight.dtype in (torch.float16, torch.float32):
         if then is None:
             if linear_residual(a, weight, stream, alpha, dest):
                 return None
@@ -247,9 +247,11 @@ class DecoupledFeatureAttention(nn.Module):
         return cells_out, self.target_mix(readout).view(b, r, self.target_tokens, width)
 
     def mix_weight(self, dtype: torch.dtype) -> torch.Tensor:
-        """``target_mix``'s weight in ``dtype`` (the projection dtype), cast by each call: an edit through
-        ``.data``, which moves neither its address nor its version, reaches the next one."""
-        return self.target_mix.weight.to(dtype)
+        """``target_mix``'s weight for a projection in ``dtype``, as it is on this call (an edit through
+        ``.data``, which moves neither its address nor its version, reaches the next one): the fp32
+        parameter, which the update's kernel rounds itself, or a cast of another dtype."""
+        w = self.target_mix.weight
+        return w if w.dtype == torch.float32 else w.to(dtype)
 
     def attend(self, tokens: torch.Tensor, n_cells: int) -> tuple[torch.Tensor, torch.Tensor]:
         """``forward`` before the cells' output projection and ``target_mix``: (the cell

@@ -372,3 +372,18 @@ def test_fp32_weights_are_rounded_as_a_cast_rounds_them(cuda, k, rows, n):
             # strides and bytes the kernel does not take: the cast
             odd = torch.zeros(n * k + 1, device=cuda)[1:].view(n, k).copy_(w)
             assert torch.equal(projection.linear_param(x, odd), projection.linear(x, cast))
+
+
+@pytest.mark.parametrize("k", [128, 256])
+@pytest.mark.parametrize("rows", [1, 129, 5001])
+def test_residual_of_fp32_weights(cuda, k, rows):
+    # the residual kernels round fp32 weights as a cast does: bit for bit, with and without the norm
+    g = torch.Generator(device=cuda).manual_seed(rows + k)
+    a = torch.randn(rows, k, generator=g, device=cuda).half()
+    w = torch.randn(k, k + 4, generator=g, device=cuda)[:, :k] / k ** 0.5
+    x = torch.randn(rows, k, generator=g, device=cuda)
+    want, got, bare = x.clone(), x.clone(), x.clone()
+    y_ref = projection.linear_residual_norm(a, w.half().contiguous(), want, ALPHA, 1e-5)
+    y = projection.linear_residual_norm(a, w, got, ALPHA, 1e-5)
+    assert torch.equal(y, y_ref) and torch.equal(got, want)
+    assert projection.linear_residual(a, w, bare, ALPHA) and torch.equal(bare, want)
