@@ -269,18 +269,23 @@ int launch_tiles(LinArgs a, int cus, hipStream_t stream) {
 // The tile of a call. Workgroups of 256 rows x 128 columns from 0.4 of them a CU: below, twice as many of
 // 128 rows are ahead (4,096 rows, K 128: N 768, 96 of them, 7.3 -> 6.3 us), above, W staged twice as often
 // costs more (8,192 x 768, 192 of them: 8.5 us against 8.9 in 128 rows; 33,000 x 128, 129: 7.9 against 8.2).
-// At K 256 a workgroup stages 64 KB of W, so while chunks of 64 leave no more than one workgroup a CU they
-// are ahead: 64 to 4,096 rows, N 256 6.9 - 8.3 -> 4.9 - 6.1 us. Teams share the blocks evenly: 65,536 x 640, K 128:
-// 27.1 -> 26.7 us, N 384 20.1 -> 19.8; and the last block of a workgroup loads no rows after it, which cost
-// calls of about a block each 5 to 10 % (20,000 x 640: 13.9 -> 12.7 us).
+// At K 256 a workgroup stages 64 KB of W, so chunks of 64 are ahead while an XCD's share of the blocks (it
+// takes whole ones) leaves no more than one such workgroup a CU: 64 to 4,096 rows, N 256 6.9 - 8.3 -> 4.9 - 6.1
+// us; 6,600 to 8,192 rows, N 512 11.4 -> 9.1; past it (2,304 rows, N 1536) they take 15.6 us against 11.5.
+// Teams share the blocks evenly: 65,536 x 640, K 128: 27.1 -> 26.7 us, N 384 20.1 -> 19.8; and the last block of
+// a workgroup loads no rows after it, which cost calls of about a block each 5 to 10 % (20,000 x 640:
+// 13.9 -> 12.7 us).
 template <int KS, bool NORM, bool W32>
 int launch(LinArgs a, hipStream_t stream) {
     const int cus = device_cus();
     const int64_t chunks = (a.n + 127) / 128, blocks = (a.rows + 255) / 256;
-    if (5 * blocks * chunks >= 2 * cus) return launch_tiles<KS, 128, 2, NORM, W32>(a, cus, stream);
+    const bool tall = 5 * blocks * chunks >= 2 * cus;
     if constexpr (KS == 8) {
-        if (2 * ((a.rows + 127) / 128) * chunks <= cus) return launch_tiles<KS, 64, 1, NORM, W32>(a, cus, stream);
+        auto fits = [&](int64_t nblocks) { return (nblocks + 7) / 8 * 8 * 2 * chunks <= cus; };
+        if (tall && fits(blocks)) return launch_tiles<KS, 64, 2, NORM, W32>(a, cus, stream);
+        if (!tall && fits((a.rows + 127) / 128)) return launch_tiles<KS, 64, 1, NORM, W32>(a, cus, stream);
     }
+    if (tall) return launch_tiles<KS, 128, 2, NORM, W32>(a, cus, stream);
     return launch_tiles<KS, 128, 1, NORM, W32>(a, cus, stream);
 }
 

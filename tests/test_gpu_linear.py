@@ -339,7 +339,8 @@ def test_weights_on_another_device_are_refused(cuda):
 
 
 @pytest.mark.parametrize("k", [128, 256])
-@pytest.mark.parametrize("rows,n", [(128, 4), (129, 64), (4095, 196), (6500, 516), (13057, 260), (26000, 132), (100001, 68)])
+@pytest.mark.parametrize("rows,n", [(128, 4), (129, 64), (4095, 196), (6500, 516), (13057, 260), (26000, 132), (100001, 68),
+                                    (8000, 512), (2304, 1540)])
 def test_tiles_at_their_rules_edges(cuda, k, rows, n):
     # 128- and 256-row blocks, 64- and 128-column chunks, one block a workgroup and several shared
     # unevenly: dyadic operands, so every order of the sums gives the same fp32 value; the rows around
